@@ -14,6 +14,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "coffee_hip.h"
@@ -243,7 +244,16 @@ constexpr bool has_o32() {
   return sizeof(T) == 4 && TX == 128 && TY == 8;
 }
 
-template <typename T, bool F, bool L, bool D, bool S, int TX, int TY>
+// Calls f with the star boundary's template argument: 0 none, 1 the pulsar
+// (problem 1), 2 the perturbed dipole (problem 2).
+template <typename F>
+void with_star(int star, F&& f) {
+  if (star == 1) f(std::integral_constant<int, 1>{});
+  else if (star == 2) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, 0>{});
+}
+
+template <typename T, bool F, bool L, bool D, int S, int TX, int TY>
 void launch_stage(bool tiled, int tblocks, dim3 grid, dim3 block, hipStream_t s, const FlatK<T>& k,
                   const FlatIO<T>& io, T as, T bs, T ts, const TileMap& tm) {
   if (tiled)
@@ -253,19 +263,18 @@ void launch_stage(bool tiled, int tblocks, dim3 grid, dim3 block, hipStream_t s,
 }
 
 template <typename T, bool F, bool L, int TX, int TY>
-void launch_stage_fl(bool dg, bool star, bool tiled, int tblocks, dim3 grid, dim3 block,
+void launch_stage_fl(bool dg, int star, bool tiled, int tblocks, dim3 grid, dim3 block,
                      hipStream_t s, const FlatK<T>& k, const FlatIO<T>& io, T as, T bs, T ts,
                      const TileMap& tm) {
-  if (dg) {
-    if (star) launch_stage<T, F, L, true, true, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
-    else launch_stage<T, F, L, true, false, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
-  } else {
-    if (star) launch_stage<T, F, L, false, true, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
-    else launch_stage<T, F, L, false, false, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
-  }
+  auto with = [&](auto st) {
+    constexpr int S = decltype(st)::value;
+    if (dg) launch_stage<T, F, L, true, S, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
+    else launch_stage<T, F, L, false, S, TX, TY>(tiled, tblocks, grid, block, s, k, io, as, bs, ts, tm);
+  };
+  with_star(star, with);
 }
 
-template <typename T, int TX, int TY, bool S>
+template <typename T, int TX, int TY, int S>
 void launch_ko_tiled(bool o32, int tblocks, hipStream_t s, const FlatK<T>& k, const FlatIO<T>& io,
                      T t1, const TileMap& tm) {
   if constexpr (has_o32<T, TX, TY>()) {
@@ -292,7 +301,7 @@ void p_buffers(int st, T* a, T* b, T* cb, FlatIO<T>& io) {
 
 template <typename T, int TX, int TY>
 int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7], T* const B[7],
-                  T* const Cp, double time, hipStream_t s, bool star) {
+                  T* const Cp, double time, hipStream_t s, int star) {
   static const double As[5] = {0, -0.4178904745, -1.192151694643, -1.697784692471,
                                -1.514183444257};
   static const double Bs[5] = {0.1496590219993, 0.3792103129999, 0.8229550293869,
@@ -327,6 +336,7 @@ int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7],
     p_buffers<T>(st, A[6], B[6], Cp, io);
     const T as = (T)As[st], bs = (T)Bs[st];
     const T ts = t0 + (T)cs[st] * dt;
+    if (star) io.star = star_phase(k, k.omega * ts);
     const char* name = st == 0 ? "ez_stage_first" : (st == 4 ? "ez_stage_last" : "ez_stage");
     rc = timed(c, name, s, [&] {
       if (st == 0)
@@ -345,19 +355,16 @@ int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7],
   }
   io.in[6] = io.out[6] = nullptr;
   const T t1 = t0 + dt;
+  if (star) io.star = star_phase(k, k.omega * t1);
   return timed(c, "ez_ko", s, [&] {
-    if (dg) {
+    with_star(star, [&](auto st) {
+      constexpr int S = decltype(st)::value;
       // diagnostics mode: the one-thread-per-cell KO kernel with the energy
       // accounting (bitwise the same field results as the tiled one)
-      if (star) ez_ko_kernel<T, true, true><<<grid, block, 0, s>>>(k, io, t1);
-      else ez_ko_kernel<T, false, true><<<grid, block, 0, s>>>(k, io, t1);
-    } else if (tiled) {
-      if (star) launch_ko_tiled<T, TX, TY, true>(o32, tblocks, s, k, io, t1, tm);
-      else launch_ko_tiled<T, TX, TY, false>(o32, tblocks, s, k, io, t1, tm);
-    } else {
-      if (star) ez_ko_kernel<T, true><<<grid, block, 0, s>>>(k, io, t1);
-      else ez_ko_kernel<T, false><<<grid, block, 0, s>>>(k, io, t1);
-    }
+      if (dg) ez_ko_kernel<T, S, true><<<grid, block, 0, s>>>(k, io, t1);
+      else if (tiled) launch_ko_tiled<T, TX, TY, S>(o32, tblocks, s, k, io, t1, tm);
+      else ez_ko_kernel<T, S><<<grid, block, 0, s>>>(k, io, t1);
+    });
   });
 }
 
@@ -429,7 +436,7 @@ int ez_step_impl(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t
       }
   }
 
-  const bool star = k.problem == 1 || k.problem == 2;
+  const int star = k.problem == 1 || k.problem == 2 ? k.problem : 0;
   int tx = 64, ty = 8;
   tile_shape<T>(c->variant, tx, ty);
   constexpr bool f32 = sizeof(T) == 4;

@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 namespace coffee {
 
 template <typename T>
@@ -51,8 +53,24 @@ struct FlatK {
   T tp_start1, tp_end1, rpert11, rpert21, dw1, nT1, ph11, ph21, dph1;
 };
 
+// Star multipole rotated to the time of a stage: the dipole vector, the
+// quadrupole tensor and its offset (pulsar_impl.hpp:57-119 rotate them by
+// phase = omega t at every cell and component).  They are the same for the
+// whole grid, so the host fills them once per launch: evaluated per cell,
+// with one kernel for both problems, the inlined boundary took 160-172
+// registers (21 spilled per lane in the 128 x 8 tile); with the rotation
+// hoisted and the two problems' kernels apart the pulsar kernels need 112-127
+// and spill none (FP32 pulsar box 160 x 128 x 120: 864 -> 717 us per step).
+template <typename T>
+struct StarPhase {
+  T p[3];
+  T q11, q12, q13, q22, q23, q33;
+  T ox, oy;
+};
+
 template <typename T>
 struct FlatIO {
+  StarPhase<T> star;
   const T* __restrict__ in[7];
   T* __restrict__ out[7];
   T* __restrict__ dU[7];
@@ -132,42 +150,52 @@ __device__ __forceinline__ T shape_fn(T r, T r0, T del) {
   return T(0.5) * (T(1) - tanh((r - r0) / del));
 }
 
+// Rotation of the multipole by `phase` (host code; sine and cosine rounded
+// once from FP64, the products in T as the reference's Scalar builds).
 template <typename T>
-__device__ T dipole2_d(T x, T y, T z, T p1, T p2, T p3, T phase, int n) {
-  // pulsar_impl.hpp:57-80
-  const T tiny = TinyOf<T>::v;
-  T c = cos(phase), s = sin(phase);
-  T p1t = p1 * c - p2 * s, p2t = p1 * s + p2 * c, p3t = p3;
-  T r2 = x * x + y * y + z * z;
-  T den = sqrt(cube(r2)) + tiny;
-  T pr = p1t * x + p2t * y + p3t * z;
-  T comp = n == 0 ? x : (n == 1 ? y : z);
-  T pt = n == 0 ? p1t : (n == 1 ? p2t : p3t);
-  return (T(3) * comp * pr / (r2 + tiny) - pt) / den;
+inline StarPhase<T> star_phase(const FlatK<T>& k, T phase) {
+  const T c = (T)::cos((double)phase), s = (T)::sin((double)phase);
+  StarPhase<T> m;
+  m.p[0] = k.p1 * c - k.p2 * s;
+  m.p[1] = k.p1 * s + k.p2 * c;
+  m.p[2] = k.p3;
+  m.q11 = k.q11 * c * c - T(2) * k.q12 * c * s + k.q22 * s * s;
+  m.q12 = k.q12 * (T)::cos((double)(T(2) * phase)) + (k.q11 - k.q22) * c * s;
+  m.q22 = k.q22 * c * c + k.q11 * s * s + T(2) * k.q12 * c * s;
+  m.q13 = k.q13 * c - k.q23 * s;
+  m.q23 = k.q23 * c + k.q13 * s;
+  m.q33 = -k.q11 - k.q22;
+  m.ox = k.qox * c - k.qoy * s;
+  m.oy = k.qox * s + k.qoy * c;
+  return m;
 }
 
+// b = dipole of the star at (x, y, z) (pulsar_impl.hpp:57-80).
 template <typename T>
-__device__ T quadrupole_d(const FlatK<T>& k, T x, T y, T z, T phase, int n) {
-  // pulsar_impl.hpp:82-119
+__device__ __forceinline__ void dipole2_d(const StarPhase<T>& m, T x, T y, T z, T b[3]) {
   const T tiny = TinyOf<T>::v;
-  T c = cos(phase), s = sin(phase);
-  T q11t = k.q11 * c * c - T(2) * k.q12 * c * s + k.q22 * s * s;
-  T q12t = k.q12 * cos(T(2) * phase) + (k.q11 - k.q22) * c * s;
-  T q22t = k.q22 * c * c + k.q11 * s * s + T(2) * k.q12 * c * s;
-  T q13t = k.q13 * c - k.q23 * s;
-  T q23t = k.q23 * c + k.q13 * s;
-  T q33t = -k.q11 - k.q22;
-  T ox = k.qox * c - k.qoy * s, oy = k.qox * s + k.qoy * c;
-  T x1 = x - ox, y1 = y - oy, z1 = z - k.qoz;
-  T r2 = x1 * x1 + y1 * y1 + z1 * z1;
-  T r7 = cube(r2) * sqrt(r2);
-  T xqx = q11t * x1 * x1 + T(2) * q12t * x1 * y1 + q22t * y1 * y1 +
-          T(2) * (q13t * x1 + q23t * y1) * z1 + q33t * z1 * z1;
-  T a0 = n == 0 ? q11t : (n == 1 ? q12t : q13t);
-  T a1 = n == 0 ? q12t : (n == 1 ? q22t : q23t);
-  T a2 = n == 0 ? q13t : (n == 1 ? q23t : q33t);
-  T comp = n == 0 ? x1 : (n == 1 ? y1 : z1);
-  return (T(-2) * (a0 * x1 + a1 * y1 + a2 * z1) * r2 + T(5) * comp * xqx) / (r7 + tiny);
+  const T r2 = x * x + y * y + z * z;
+  const T den = sqrt(cube(r2)) + tiny;
+  const T pr = m.p[0] * x + m.p[1] * y + m.p[2] * z;
+  const T pos[3] = {x, y, z};
+#pragma unroll
+  for (int n = 0; n < 3; n++) b[n] = (T(3) * pos[n] * pr / (r2 + tiny) - m.p[n]) / den;
+}
+
+// b += quadrupole of the star at (x, y, z) (pulsar_impl.hpp:82-119).
+template <typename T>
+__device__ __forceinline__ void add_quadrupole_d(const StarPhase<T>& m, T qoz, T x, T y, T z,
+                                                 T b[3]) {
+  const T tiny = TinyOf<T>::v;
+  const T x1 = x - m.ox, y1 = y - m.oy, z1 = z - qoz;
+  const T r2 = x1 * x1 + y1 * y1 + z1 * z1;
+  const T r7 = cube(r2) * sqrt(r2);
+  const T xqx = m.q11 * x1 * x1 + T(2) * m.q12 * x1 * y1 + m.q22 * y1 * y1 +
+                T(2) * (m.q13 * x1 + m.q23 * y1) * z1 + m.q33 * z1 * z1;
+  const T den = r7 + tiny;
+  b[0] += (T(-2) * (m.q11 * x1 + m.q12 * y1 + m.q13 * z1) * r2 + T(5) * x1 * xqx) / den;
+  b[1] += (T(-2) * (m.q12 * x1 + m.q22 * y1 + m.q23 * z1) * r2 + T(5) * y1 * xqx) / den;
+  b[2] += (T(-2) * (m.q13 * x1 + m.q23 * y1 + m.q33 * z1) * r2 + T(5) * z1 * xqx) / den;
 }
 
 template <typename T>
@@ -220,11 +248,11 @@ __device__ void twistv_d(const FlatK<T>& k, T t, T x, T y, T z, T ri, T v[3]) {
   v[2] = -dw * R1 * sinth * s0;
 }
 
-// boundary_pulsar (problem 1, field_solver_EZ.cpp:711-839) and
-// boundary_alfven (problem 2, .cpp:841-1005) on one cell's values.
-template <typename T>
-__device__ void star_boundary(const FlatK<T>& k, T x, T y, T z, T t, T& ex, T& ey, T& ez, T& bx,
-                              T& by, T& bz) {
+// boundary_pulsar (STAR = 1, problem 1, field_solver_EZ.cpp:711-839) and
+// boundary_alfven (STAR = 2, problem 2, .cpp:841-1005) on one cell's values.
+template <typename T, int STAR>
+__device__ __forceinline__ void star_boundary(const FlatK<T>& k, const StarPhase<T>& m, T x, T y, T z,
+                                              T t, T& ex, T& ey, T& ez, T& bx, T& by, T& bz) {
   const T tiny = TinyOf<T>::v;
   T rl = T(1.5) * k.radius, ri = T(0.5) * k.radius;
   T r2 = x * x + y * y + z * z;
@@ -234,14 +262,12 @@ __device__ void star_boundary(const FlatK<T>& k, T x, T y, T z, T t, T& ex, T& e
   T scaleEpar = T(0.5) * k.delta[0], scaleEperp = T(0.25) * k.delta[0];
   T scaleB = scaleEpar;
   T d1 = T(4) * k.delta[0];
-  T phase = k.omega * t;
-  T vx = 0, vy = 0, vz = 0, bxn, byn, bzn;
-  if (k.problem == 1) {
+  T vx = 0, vy = 0, vz = 0, bn[3];
+  dipole2_d(m, x, y, z, bn);
+  if (STAR == 1) {
     vx = -k.omega * y;
     vy = k.omega * x;
-    bxn = k.b0 * (dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 0) + quadrupole_d(k, x, y, z, phase, 0));
-    byn = k.b0 * (dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 1) + quadrupole_d(k, x, y, z, phase, 1));
-    bzn = k.b0 * (dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 2) + quadrupole_d(k, x, y, z, phase, 2));
+    add_quadrupole_d(m, k.qoz, x, y, z, bn);
   } else {
     T th = acos(z / r);
     if (k.pert_type == 0 || k.pert_type == 1) {
@@ -266,10 +292,8 @@ __device__ void star_boundary(const FlatK<T>& k, T x, T y, T z, T t, T& ex, T& e
       vy = v[1];
       vz = v[2];
     }
-    bxn = k.b0 * dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 0);
-    byn = k.b0 * dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 1);
-    bzn = k.b0 * dipole2_d(x, y, z, k.p1, k.p2, k.p3, phase, 2);
   }
+  const T bxn = k.b0 * bn[0], byn = k.b0 * bn[1], bzn = k.b0 * bn[2];
   T s = shape_fn(r, k.radius - d1, scaleB);
   T bn_r = bxn * x + byn * y + bzn * z;
   T B_r = bx * x + by * y + bz * z;
@@ -377,7 +401,7 @@ __device__ __forceinline__ bool in_layer(const FlatK<T>& k, T x, T y, T z) {
 // read) and the absorbing-layer cells of U are saved to Un; LAST: dU is not
 // written back (the next step starts with As = 0) and the absorbing layer is
 // applied.
-template <typename T, bool FIRST, bool LAST, bool DIAG, bool STAR>
+template <typename T, bool FIRST, bool LAST, bool DIAG, int STAR>
 __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& io, const int i,
                                            const int j, const int kk, const int c,
                                            const T (&d)[7][3], T (&u)[7], const T (&dprev)[7],
@@ -472,7 +496,7 @@ __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& i
   else project_cell(u[0], u[1], u[2], u[3], u[4], u[5]);
   if (STAR) {
     const T x = node_pos(k, 0, i), y = node_pos(k, 1, j), z = node_pos(k, 2, kk);
-    star_boundary(k, x, y, z, tstage, u[0], u[1], u[2], u[3], u[4], u[5]);
+    star_boundary<T, STAR>(k, io.star, x, y, z, tstage, u[0], u[1], u[2], u[3], u[4], u[5]);
   }
   if (LAST && k.pml_any) {
     // damping_boundary (damping_boundary.cpp:5-83): E toward En, B toward Bbg
@@ -506,7 +530,7 @@ __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& i
 // f + (KOeps/64) sum_axes delta^6 f, u[6] = P (untouched on the CPU path).
 // DIAG: e_before = |E|^2 + |B|^2 before the KO update; dU_KO = the change
 // (field_solver_EZ.cpp:447-453), then the projection's accounting.
-template <typename T, bool STAR, bool DIAG = false, bool O32 = false>
+template <typename T, int STAR, bool DIAG = false, bool O32 = false>
 __device__ __forceinline__ void ko_cell_finish(const FlatK<T>& k, const FlatIO<T>& io, int i,
                                                int j, int kk, int c, T (&u)[7], T t,
                                                T e_before = T(0)) {
@@ -521,7 +545,7 @@ __device__ __forceinline__ void ko_cell_finish(const FlatK<T>& k, const FlatIO<T
   }
   if (STAR) {
     const T x = node_pos(k, 0, i), y = node_pos(k, 1, j), z = node_pos(k, 2, kk);
-    star_boundary(k, x, y, z, t, u[0], u[1], u[2], u[3], u[4], u[5]);
+    star_boundary<T, STAR>(k, io.star, x, y, z, t, u[0], u[1], u[2], u[3], u[4], u[5]);
   }
 #pragma unroll
   for (int q = 0; q < 6; q++) stf<T, O32>(io.out[q], c, u[q]);
@@ -531,7 +555,7 @@ __device__ __forceinline__ void ko_cell_finish(const FlatK<T>& k, const FlatIO<T
 // Simple stage kernel: one thread per cell, stencil neighbours read straight
 // from global memory (periodic axes wrap into the interior).  Used for grids
 // the tiled kernel does not take and as the second implementation in tests.
-template <typename T, bool FIRST, bool LAST, bool DIAG, bool STAR>
+template <typename T, bool FIRST, bool LAST, bool DIAG, int STAR>
 __global__ void __launch_bounds__(256)
     ez_stage_kernel(const FlatK<T> k, const FlatIO<T> io, const T As, const T Bs, const T tstage) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + k.guard[0];
@@ -565,7 +589,7 @@ __global__ void __launch_bounds__(256)
 
 // Simple Kreiss_Oliger kernel (one thread per cell); DIAG adds the energy
 // accounting (diagnostics mode always runs this kernel).
-template <typename T, bool STAR, bool DIAG = false>
+template <typename T, int STAR, bool DIAG = false>
 __global__ void __launch_bounds__(256) ez_ko_kernel(const FlatK<T> k, const FlatIO<T> io, const T t) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + k.guard[0];
   const int j = blockIdx.y * blockDim.y + threadIdx.y + k.guard[1];

@@ -54,7 +54,7 @@ __device__ __forceinline__ int amap(int v, int n, int g, int per) {
 
 // Whether a tiled kernel keeps the x-y halo of R+LA planes in registers
 // (fetched with the centre columns) or of one plane.
-template <typename T, bool STAR, int HPT, int NT>
+template <typename T, int STAR, int HPT, int NT>
 constexpr bool deep_halo() {
   return !STAR && HPT == 1 && sizeof(T) * NT <= 4096;
 }
@@ -62,7 +62,7 @@ constexpr bool deep_halo() {
 // Planes of look-ahead of the centre columns (LA) of the stage kernels: two
 // where the registers allow (FP32 kernels with the deep halo, but not the
 // last stage, whose absorbing-layer operands take the room), else one.
-template <typename T, bool STAR, bool LAST, int HPT, int NT>
+template <typename T, int STAR, bool LAST, int HPT, int NT>
 constexpr int centre_lookahead() {
   return deep_halo<T, STAR, HPT, NT>() && sizeof(T) == 4 && !LAST ? 2 : 1;
 }
@@ -83,7 +83,7 @@ __device__ __forceinline__ void halo_xy(int h, int& hx, int& hy) {
   }
 }
 
-template <typename T, int TX, int TY, bool FIRST, bool LAST, bool DIAG, bool STAR>
+template <typename T, int TX, int TY, bool FIRST, bool LAST, bool DIAG, int STAR>
 __global__ void __launch_bounds__(TX * TY)
     ez_stage_tiled(const FlatK<T> k, const FlatIO<T> io, const T As, const T Bs, const T ts,
                    const TileMap tm) {
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(TX * TY)
   }
 }
 
-template <typename T, int TX, int TY, bool STAR, bool O32>
+template <typename T, int TX, int TY, int STAR, bool O32>
 __global__ void __launch_bounds__(TX * TY)
     ez_ko_tiled(const FlatK<T> k, const FlatIO<T> io, const T tko, const TileMap tm) {
   constexpr int R = 3, LX = TX + 2 * R, LY = TY + 2 * R, NF = 6, NT = TX * TY;
