@@ -82,35 +82,15 @@ GrK<float>& grk<float>(GrState* S) { return S->kf; }
 template <>
 GrK<double>& grk<double>(GrState* S) { return S->kd; }
 
-// Guard cells with the flat solver's kernels: periodic ones in place in one
-// pass (wrap, dst == src), frozen ones copied slab by slab (src -> dst).
+// Periodic guards of one buffer in place, with the flat solver's kernel.
 template <typename T>
-int gr_guards(coffee_ctx* c, hipStream_t s, T* const dst[7], T* const src[7], bool wrap) {
+int gr_wrap_guards(coffee_ctx* c, hipStream_t s, T* const a[7]) {
   const FlatK<T>& k = flat_k<T>(c);
-  Ptr7<T> d, r;
-  for (int q = 0; q < 7; q++) {
-    d.p[q] = dst[q];
-    r.p[q] = src[q];
-  }
-  if (wrap) {
-    if (!k.per[0] && !k.per[1] && !k.per[2]) return COFFEE_OK;
-    const long total = (long)k.dims[0] * k.dims[1] * k.dims[2] - (long)k.n[0] * k.n[1] * k.n[2];
-    const int blocks = (int)std::min<long>((total + 255) / 256, 8192);
-    return timed(c, "guard_fill", s, [&] { guard_wrap_kernel<T><<<blocks, 256, 0, s>>>(k, d, 7); });
-  }
-  for (int ax = 0; ax < 3; ax++) {
-    if (wrap != (bool)k.per[ax]) continue;
-    long ext = 2L * k.guard[ax];
-    for (int a = 0; a < 3; a++)
-      if (a != ax) ext *= k.dims[a];
-    int blocks = (int)std::min<long>((ext + 255) / 256, 4096);
-    int rc = timed(c, wrap ? "guard_fill" : "guard_copy", s, [&] {
-      if (wrap) guard_slab_kernel<T, true><<<blocks, 256, 0, s>>>(k, ax, d, r, 7);
-      else guard_slab_kernel<T, false><<<blocks, 256, 0, s>>>(k, ax, d, r, 7);
-    });
-    if (rc) return rc;
-  }
-  return COFFEE_OK;
+  if (!k.per[0] && !k.per[1] && !k.per[2]) return COFFEE_OK;
+  Ptr7<T> d;
+  for (int q = 0; q < 7; q++) d.p[q] = a[q];
+  const int blocks = (int)std::min<long>((guard_count(k) + 255) / 256, 8192);
+  return timed(c, "guard_fill", s, [&] { guard_wrap_kernel<T><<<blocks, 256, 0, s>>>(k, d, 7); });
 }
 
 template <typename T, bool F, bool L>
@@ -173,7 +153,7 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   }
   A[6] = (T*)f->P;
   for (int q = 0; q < 7; q++) B[q] = (T*)c->scratch[q];
-  int rc = gr_guards<T>(c, s, B, A, false);
+  int rc = copy_frozen_guards<T>(c, s, B, A, nullptr);
   if (rc) return rc;
 
   GrIO<T> io{};
@@ -264,7 +244,7 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
       });
     }
     if (rc) return rc;
-    rc = gr_guards<T>(c, s, out, out, true);
+    rc = gr_wrap_guards<T>(c, s, out);
     if (rc) return rc;
   }
   for (int q = 0; q < 7; q++) {
@@ -276,7 +256,7 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
     else gr_ko_kernel<T><<<grid, block, 0, s>>>(k, io);
   });
   if (rc) return rc;
-  return gr_guards<T>(c, s, A, A, true);
+  return gr_wrap_guards<T>(c, s, A);
 }
 
 template <typename T>

@@ -65,6 +65,7 @@ void fill_k(const coffee_grid& g, const coffee_params& p, FlatK<T>& k) {
   k.problem = p.problem;
   k.pert_type = p.pert_type;
   k.mask_lanes = p.mask_lanes > 0 ? p.mask_lanes : 1;
+  k.images = 0;
   k.pml_any = (p.pml[0] > 0 || p.pml[1] > 0 || p.pml[2] > 0) ? 1 : 0;
   k.sigpml = (T)p.sigpml;
   k.radius = (T)p.radius;
@@ -158,60 +159,55 @@ __global__ void __launch_bounds__(256)
   for (; i < e; i += 256) __builtin_nontemporal_store(__builtin_nontemporal_load(&src[i]), &dst[i]);
 }
 
+// Periodic guard fill of the caller's arrays in place.
 template <typename T>
-int guard_slabs(coffee_ctx* c, hipStream_t s, T* const dst[7], T* const src[7], bool wrap,
-                int nfields = 7) {
-  FlatK<T>& k = kparams<T>(c);
-  Ptr7<T> d, r;
-  for (int q = 0; q < 7; q++) {
-    d.p[q] = dst[q];
-    r.p[q] = src[q];
-  }
-  if (wrap) {
-    // in place (dst == src): every periodic guard cell in one launch
-    if (!k.per[0] && !k.per[1] && !k.per[2]) return COFFEE_OK;
-    const long total = (long)k.dims[0] * k.dims[1] * k.dims[2] - (long)k.n[0] * k.n[1] * k.n[2];
-    const int blocks = (int)std::min<long>((total + 255) / 256, 8192);
-    return timed(c, "guard_fill", s, [&] {
-      guard_wrap_kernel<T><<<blocks, 256, 0, s>>>(k, d, nfields);
-    });
-  }
-  for (int ax = 0; ax < 3; ax++) {
-    if (k.guard[ax] == 0) continue;
-    if (wrap != (bool)k.per[ax]) continue;
-    long ext = 2L * k.guard[ax];
-    for (int a = 0; a < 3; a++)
-      if (a != ax) ext *= k.dims[a];
-    int blocks = (int)std::min<long>((ext + 255) / 256, 4096);
-    int rc;
-    if (wrap)
-      rc = timed(c, "guard_fill", s, [&] {
-        guard_slab_kernel<T, true><<<blocks, 256, 0, s>>>(k, ax, d, r, nfields);
-      });
-    else
-      rc = timed(c, "guard_copy", s, [&] {
-        guard_slab_kernel<T, false><<<blocks, 256, 0, s>>>(k, ax, d, r, nfields);
-      });
-    if (rc) return rc;
-  }
-  return COFFEE_OK;
+int wrap_guards(coffee_ctx* c, hipStream_t s, T* const a[7], int nfields = 7) {
+  const FlatK<T>& k = kparams<T>(c);
+  if (!k.per[0] && !k.per[1] && !k.per[2]) return COFFEE_OK;
+  Ptr7<T> d;
+  for (int q = 0; q < 7; q++) d.p[q] = a[q];
+  const int blocks = (int)std::min<long>((guard_count(k) + 255) / 256, 8192);
+  return timed(c, "guard_fill", s, [&] {
+    guard_wrap_kernel<T><<<blocks, 256, 0, s>>>(k, d, nfields);
+  });
 }
 
-// Planes per workgroup: one workgroup per CU (256 CUs) marching the whole
-// z extent measured best at 512^3 (fewest warm-up planes, no chunk seams);
-// grids with fewer tiles per plane split z so every CU still gets work.
-int auto_zchunk(int tiles_per_plane, int nz) {
-  int nzc = (256 + tiles_per_plane - 1) / tiles_per_plane;
-  int zc = (nz + nzc - 1) / nzc;
-  return zc < 8 ? 8 : zc;
+// Cost of a stage of the tiled kernels with a TX x TY tile and z split into
+// nzc chunks, in planes marched one after the other on a CU: a tile workgroup
+// of 512 or 1024 threads has a CU (256 of them) to itself, so the tiles run in
+// rounds, and a chunk of zc planes lasts zc plus about 10 (its launch, the
+// queue's first 2R + 1 planes and their latency).  Near a star some workgroups take
+// about twice as long per plane; the last of them sets the end.  `weight` is
+// the time of one plane of this tile.
+double chunk_cost(int tiles, int nz, int nzc, bool star, double weight) {
+  const int zc = (nz + nzc - 1) / nzc;
+  const int blocks = tiles * ((nz + zc - 1) / zc);
+  const int rounds = (blocks + 255) / 256;
+  return (rounds * (zc + 10.0) + (star ? zc : 0)) * weight;
 }
 
-// Tile (columns x rows) of the tiled kernels: variant 0 picks the measured
-// best for the Scalar type on MI355X at 512^3 (FP32 128 x 8 = 1024 threads,
-// 3.5 % faster per step than 64 x 16; FP64 64 x 8 = 512 threads, equal to
-// 128 x 4); 2/3/4 force 64 x 4/8/16 (16 only in FP32), 5 and 6 wider rows
-// (FP32 128 x 8, 256 x 4; FP64 128 x 4 for both: a 256 x 2 FP64 tile does not
-// fit in LDS), 7 = 128 x 4; variant 1 is the thread-per-cell schedule.
+// The z chunk of the lowest cost (at least 2 planes), and that cost.
+int auto_zchunk(int tiles, int nz, bool star, double weight, double* cost) {
+  int best = 1;
+  double least = 0;
+  for (int nzc = 1; nzc <= std::max(1, nz / 2) && nzc <= 256; nzc++) {
+    const double v = chunk_cost(tiles, nz, nzc, star, weight);
+    if (nzc == 1 || v < least) {
+      least = v;
+      best = nzc;
+    }
+  }
+  if (cost) *cost = least;
+  return (nz + best - 1) / best;
+}
+
+// Tile (columns x rows) of the tiled kernels: variant 0 without a z chunk is
+// planned by auto_schedule; with one it is the tile that measured best at
+// 512^3 (FP32 128 x 8 = 1024 threads, 3.5 % faster per step than 64 x 16; FP64
+// 64 x 8 = 512 threads, equal to 128 x 4); 2/3/4 force 64 x 4/8/16 (16 only in
+// FP32), 5 and 6 wider rows (FP32 128 x 8, 256 x 4; FP64 128 x 4 for both: a
+// 256 x 2 FP64 tile does not fit in LDS), 7 = 128 x 4; variant 1 is the
+// thread-per-cell schedule.
 template <typename T>
 void tile_shape(int variant, int& tx, int& ty) {
   const bool f32 = sizeof(T) == 4;
@@ -233,6 +229,40 @@ void tile_shape(int variant, int& tx, int& ty) {
     tx = 128;
     ty = 4;
   }
+}
+
+// Kernel schedule of a grid when the caller sets none, by size only (all
+// schedules give bitwise the same results):
+// - thread-per-cell kernels where a step is launches and latency: their one
+//   round of loads ends sooner than the planes a tile marches.  The line is
+//   where the two cross (us per step): FP32 64^3 68 against 69, 80^3 139
+//   against 117; FP64 48^3 91 against 94, 64^3 123 against 100; with a star,
+//   whose cells slow few workgroups, FP32 64^3 69 against 86, 80^3 149 against
+//   148, FP64 80^3 325 against 334, 96^3 465 against 476.
+// - above it the tile and z chunk of the lowest chunk_cost.  A plane of a 128 x
+//   8 tile takes 1.6 times as long as one of a 64 x 8 tile (21.2 against 12.1
+//   us at 128^3, less 10 % since it fetches half as many x halos per cell,
+//   which shows once the fields come from HBM: 384^3 8.2 against 9.1 ms).
+//   Against one workgroup per CU for whole columns wherever the tiles gave that
+//   (the earlier rule): 128^3 281 -> 256 us, 192^3 1896 -> 1195, 384^3 11.4 ->
+//   8.2 ms, FP64 200^3 4.19 -> 2.80 ms, 384^3 23.5 -> 16.2 ms.
+struct FlatSchedule {
+  bool tiled;
+  int tx, ty, zc;
+};
+
+template <typename T>
+FlatSchedule auto_schedule(const FlatK<T>& k, bool star) {
+  constexpr bool f32 = sizeof(T) == 4;
+  const double n = (double)k.n[0] * k.n[1] * k.n[2];
+  const double small = f32 ? 300e3 : (star ? 550e3 : 130e3);
+  if (n <= small) return {false, 64, 8, 1};
+  auto tiles = [&](int tx, int ty) { return ((k.n[0] + tx - 1) / tx) * ((k.n[1] + ty - 1) / ty); };
+  double c64 = 0, c128 = 0;
+  FlatSchedule s{true, 64, 8, auto_zchunk(tiles(64, 8), k.n[2], star, 1.0, &c64)};
+  if (!f32) return s;
+  const int z128 = auto_zchunk(tiles(128, 8), k.n[2], star, 1.6, &c128);
+  return c128 < c64 ? FlatSchedule{true, 128, 8, z128} : s;
 }
 
 // The FP32 default tile (tile_shape variant 0) also has a Kreiss-Oliger
@@ -300,8 +330,8 @@ void p_buffers(int st, T* a, T* b, T* cb, FlatIO<T>& io) {
 }
 
 template <typename T, int TX, int TY>
-int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7], T* const B[7],
-                  T* const Cp, double time, hipStream_t s, int star) {
+int ez_launch_all(coffee_ctx* c, FlatK<T> k, FlatIO<T> io, T* const A[7], T* const B[7],
+                  T* const Cp, double time, hipStream_t s, int star, const bool tiled, int zc) {
   static const double As[5] = {0, -0.4178904745, -1.192151694643, -1.697784692471,
                                -1.514183444257};
   static const double Bs[5] = {0.1496590219993, 0.3792103129999, 0.8229550293869,
@@ -313,11 +343,11 @@ int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7],
   TileMap tm;
   tm.ntx = (k.n[0] + TX - 1) / TX;
   tm.nty = (k.n[1] + TY - 1) / TY;
-  tm.zc = c->zchunk > 0 ? c->zchunk : auto_zchunk(tm.ntx * tm.nty, k.n[2]);
+  tm.zc = zc > 0 ? zc : auto_zchunk(tm.ntx * tm.nty, k.n[2], star != 0, 1.0, nullptr);
   if (tm.zc > k.n[2]) tm.zc = k.n[2];
   tm.nzc = (k.n[2] + tm.zc - 1) / tm.zc;
   const int tblocks = tm.ntx * tm.nty * tm.nzc;
-  const bool tiled = c->variant != 1;
+  k.images = !tiled && k.per[0] && k.per[1] && k.per[2];
   const bool dg = c->diagnostics != 0;
   // every field array (dims0 x dims1 x dims2 scalars) addressable by a
   // 32-bit byte offset (Kreiss-Oliger kernel)
@@ -356,7 +386,7 @@ int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7],
   io.in[6] = io.out[6] = nullptr;
   const T t1 = t0 + dt;
   if (star) io.star = star_phase(k, k.omega * t1);
-  return timed(c, "ez_ko", s, [&] {
+  rc = timed(c, "ez_ko", s, [&] {
     with_star(star, [&](auto st) {
       constexpr int S = decltype(st)::value;
       // diagnostics mode: the one-thread-per-cell KO kernel with the energy
@@ -366,6 +396,9 @@ int ez_launch_all(coffee_ctx* c, const FlatK<T>& k, FlatIO<T> io, T* const A[7],
       else ez_ko_kernel<T, S><<<grid, block, 0, s>>>(k, io, t1);
     });
   });
+  // single-GPU exchange: periodic guards of the caller's arrays
+  if (rc || k.images) return rc;
+  return wrap_guards<T>(c, s, A);
 }
 
 template <typename T>
@@ -398,14 +431,8 @@ int ez_step_impl(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t
   if (!Cp) return fail(c, COFFEE_ERR_STATE, "flat step needs the third P buffer");
 
   // Frozen (non-periodic) guards must be present in the partner buffers.
-  rc = guard_slabs<T>(c, s, B, A, false);
+  rc = copy_frozen_guards<T>(c, s, B, A, Cp);
   if (rc) return rc;
-  {
-    T* const cd[7] = {Cp, Cp, Cp, Cp, Cp, Cp, Cp};
-    T* const cs[7] = {A[6], A[6], A[6], A[6], A[6], A[6], A[6]};
-    rc = guard_slabs<T>(c, s, cd, cs, false, 1);
-    if (rc) return rc;
-  }
 
   FlatIO<T> io{};
   for (int q = 0; q < 3; q++) {
@@ -437,18 +464,23 @@ int ez_step_impl(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t
   }
 
   const int star = k.problem == 1 || k.problem == 2 ? k.problem : 0;
-  int tx = 64, ty = 8;
+  int tx = 64, ty = 8, zc = c->zchunk;
+  bool tiled = c->variant != 1;
   tile_shape<T>(c->variant, tx, ty);
+  if (c->variant == 0 && zc == 0) {
+    const FlatSchedule fs = auto_schedule<T>(k, star != 0);
+    tiled = fs.tiled;
+    tx = fs.tx;
+    ty = fs.ty;
+    zc = fs.zc;
+  }
   constexpr bool f32 = sizeof(T) == 4;
-  if (tx == 128 && ty == 4) rc = ez_launch_all<T, 128, 4>(c, k, io, A, B, Cp, time, s, star);
-  else if (tx == 128) rc = ez_launch_all<T, 128, f32 ? 8 : 4>(c, k, io, A, B, Cp, time, s, star);
-  else if (tx == 256) rc = ez_launch_all<T, f32 ? 256 : 128, 4>(c, k, io, A, B, Cp, time, s, star);
-  else if (ty == 4) rc = ez_launch_all<T, 64, 4>(c, k, io, A, B, Cp, time, s, star);
-  else if (ty == 16) rc = ez_launch_all<T, 64, 16>(c, k, io, A, B, Cp, time, s, star);
-  else rc = ez_launch_all<T, 64, 8>(c, k, io, A, B, Cp, time, s, star);
-  if (rc) return rc;
-  // single-GPU exchange: periodic guards of the caller's arrays
-  return guard_slabs<T>(c, s, A, A, true);
+  if (tx == 128 && ty == 4) return ez_launch_all<T, 128, 4>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
+  if (tx == 128) return ez_launch_all<T, 128, f32 ? 8 : 4>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
+  if (tx == 256) return ez_launch_all<T, f32 ? 256 : 128, 4>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
+  if (ty == 4) return ez_launch_all<T, 64, 4>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
+  if (ty == 16) return ez_launch_all<T, 64, 16>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
+  return ez_launch_all<T, 64, 8>(c, k, io, A, B, Cp, time, s, star, tiled, zc);
 }
 
 template <typename T>
@@ -664,13 +696,13 @@ int coffee_fill_guards(coffee_ctx* c, const coffee_fields* f, void* stream) {
     if (rc) return rc;
     float* A[7];
     state_ptrs<float>(f, A);
-    return guard_slabs<float>(c, s, A, A, true);
+    return wrap_guards<float>(c, s, A);
   }
   int rc = check_fields<double>(c, f, false);
   if (rc) return rc;
   double* A[7];
   state_ptrs<double>(f, A);
-  return guard_slabs<double>(c, s, A, A, true);
+  return wrap_guards<double>(c, s, A);
 }
 
 int coffee_total_energy(coffee_ctx* c, void* const comp[3], double* out, void* stream) {
@@ -762,12 +794,12 @@ int coffee_fill_guards_arrays(const coffee_grid* grid, const int periodic[3], vo
       float* A[7] = {};
       for (int q = 0; q < m; q++) A[q] = (float*)arrays[base + q];
       for (int q = m; q < 7; q++) A[q] = A[0];
-      rc = guard_slabs<float>(&tmp, s, A, A, true, m);
+      rc = wrap_guards<float>(&tmp, s, A, m);
     } else {
       double* A[7] = {};
       for (int q = 0; q < m; q++) A[q] = (double*)arrays[base + q];
       for (int q = m; q < 7; q++) A[q] = A[0];
-      rc = guard_slabs<double>(&tmp, s, A, A, true, m);
+      rc = wrap_guards<double>(&tmp, s, A, m);
     }
     if (rc) return fail(nullptr, rc, tmp.err);
   }

@@ -122,6 +122,23 @@ inline FlatK<float>& flat_k<float>(coffee_ctx* c) { return c->kf; }
 template <>
 inline FlatK<double>& flat_k<double>(coffee_ctx* c) { return c->kd; }
 
+// Frozen (non-periodic) guard cells of a step's partner buffers: dst takes
+// src's (7 fields), dst2 src[6]'s when given.
+template <typename T>
+int copy_frozen_guards(coffee_ctx* c, hipStream_t s, T* const dst[7], T* const src[7], T* dst2) {
+  const FlatK<T>& k = flat_k<T>(c);
+  if (k.per[0] && k.per[1] && k.per[2]) return COFFEE_OK;
+  Ptr7<T> d, r;
+  for (int q = 0; q < 7; q++) {
+    d.p[q] = dst[q];
+    r.p[q] = src[q];
+  }
+  const int blocks = (int)std::min<long>((guard_count(k) + 255) / 256, 8192);
+  return timed(c, "guard_copy", s, [&] {
+    guard_copy_kernel<T><<<blocks, 256, 0, s>>>(k, d, r, dst2);
+  });
+}
+
 // Entry points of the other translation units, dispatched from the ABI.
 int gr_create(coffee_ctx* c);
 int gr_step(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t s);

@@ -43,6 +43,7 @@ struct FlatK {
   T c12[3];    // inv_delta / 12
   T dt, ch2, tau, KOfac, damp_over_dt;
   int divB_clean, use_edotb, problem, pert_type, mask_lanes;
+  int images;  // the thread-per-cell kernels also store the periodic guard images
   int pml_any;
   T xl[3], xh[3];      // absorbing-layer bounds
   T pmlscale[3];       // pmllen * delta
@@ -390,6 +391,37 @@ __device__ __forceinline__ T pml_sigma(T x, T xl, T xh, T scale, T sig0) {
   return T(0);
 }
 
+// Periodic images of interior cell (i, j, kk) in the guard cells: the cells
+// one period away along each axis subset that lie inside the array, which is
+// what send_guard_cells leaves there when every axis is periodic
+// (sim_env.cpp:365-438).  Only cells within a guard width of a face have any.
+// Stored by the thread-per-cell kernel that writes a field's final values (E,
+// B in Kreiss-Oliger, P in the last stage), so a small grid's step, which
+// lasts as long as its launches, needs no fill launch (5 of 37 us at 32^3 FP32).  The tiled
+// kernels leave the guards to guard_wrap_kernel: with these stores they ran
+// 0.7 ms slower at 512^3 FP32 against the 0.14 ms of that launch.  So does a
+// box with a frozen axis: its corner guards take frozen cells, which no
+// interior thread holds.
+template <typename T, bool O32, int NF>
+__device__ __forceinline__ void store_images(const FlatK<T>& k, T* const (&out)[NF], int i, int j,
+                                             int kk, const T (&v)[NF]) {
+  const int l0 = i >= k.n[0] ? -1 : 0, h0 = i < 2 * k.guard[0] ? 1 : 0;
+  const int l1 = j >= k.n[1] ? -1 : 0, h1 = j < 2 * k.guard[1] ? 1 : 0;
+  const int l2 = kk >= k.n[2] ? -1 : 0, h2 = kk < 2 * k.guard[2] ? 1 : 0;
+  if (!(l0 | h0 | l1 | h1 | l2 | h2)) return;
+#pragma unroll 1
+  for (int c = l2; c <= h2; c++)
+#pragma unroll 1
+    for (int b = l1; b <= h1; b++)
+#pragma unroll 1
+      for (int a = l0; a <= h0; a++) {
+        if (!(a | b | c)) continue;
+        const int o = (i + a * k.n[0]) + ((j + b * k.n[1]) + (kk + c * k.n[2]) * k.dims[1]) * k.dims[0];
+#pragma unroll
+        for (int q = 0; q < NF; q++) stf<T, O32>(out[q], o, v[q]);
+      }
+}
+
 template <typename T>
 __device__ __forceinline__ bool in_layer(const FlatK<T>& k, T x, T y, T z) {
   return x > k.xh[0] || x < k.xl[0] || y > k.xh[1] || y < k.xl[1] || z > k.xh[2] || z < k.xl[2];
@@ -401,7 +433,7 @@ __device__ __forceinline__ bool in_layer(const FlatK<T>& k, T x, T y, T z) {
 // read) and the absorbing-layer cells of U are saved to Un; LAST: dU is not
 // written back (the next step starts with As = 0) and the absorbing layer is
 // applied.
-template <typename T, bool FIRST, bool LAST, bool DIAG, int STAR>
+template <typename T, bool FIRST, bool LAST, bool DIAG, int STAR, bool IMG = false>
 __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& io, const int i,
                                            const int j, const int kk, const int c,
                                            const T (&d)[7][3], T (&u)[7], const T (&dprev)[7],
@@ -523,6 +555,11 @@ __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& i
 #pragma unroll
   for (int q = 0; q < 6; q++) io.out[q][c] = u[q];
   if (io.out[6]) io.out[6][c] = u[6];
+  if (IMG && LAST && k.images && io.out[6]) {
+    T* const p[1] = {io.out[6]};
+    const T v[1] = {u[6]};
+    store_images<T, false, 1>(k, p, i, j, kk, v);
+  }
 }
 
 // Per-cell end of the Kreiss-Oliger pass (field_solver_EZ.cpp:390-457 with
@@ -530,7 +567,7 @@ __device__ __forceinline__ void stage_cell(const FlatK<T>& k, const FlatIO<T>& i
 // f + (KOeps/64) sum_axes delta^6 f, u[6] = P (untouched on the CPU path).
 // DIAG: e_before = |E|^2 + |B|^2 before the KO update; dU_KO = the change
 // (field_solver_EZ.cpp:447-453), then the projection's accounting.
-template <typename T, int STAR, bool DIAG = false, bool O32 = false>
+template <typename T, int STAR, bool DIAG = false, bool O32 = false, bool IMG = false>
 __device__ __forceinline__ void ko_cell_finish(const FlatK<T>& k, const FlatIO<T>& io, int i,
                                                int j, int kk, int c, T (&u)[7], T t,
                                                T e_before = T(0)) {
@@ -550,11 +587,16 @@ __device__ __forceinline__ void ko_cell_finish(const FlatK<T>& k, const FlatIO<T
 #pragma unroll
   for (int q = 0; q < 6; q++) stf<T, O32>(io.out[q], c, u[q]);
   if (io.out[6]) stf<T, O32>(io.out[6], c, u[6]);
+  if (IMG && k.images) {
+    T* const p[6] = {io.out[0], io.out[1], io.out[2], io.out[3], io.out[4], io.out[5]};
+    const T v[6] = {u[0], u[1], u[2], u[3], u[4], u[5]};
+    store_images<T, O32, 6>(k, p, i, j, kk, v);
+  }
 }
 
 // Simple stage kernel: one thread per cell, stencil neighbours read straight
-// from global memory (periodic axes wrap into the interior).  Used for grids
-// the tiled kernel does not take and as the second implementation in tests.
+// from global memory (periodic axes wrap into the interior).  Used for small
+// grids (auto_schedule) and as the second implementation in tests.
 template <typename T, bool FIRST, bool LAST, bool DIAG, int STAR>
 __global__ void __launch_bounds__(256)
     ez_stage_kernel(const FlatK<T> k, const FlatIO<T> io, const T As, const T Bs, const T tstage) {
@@ -584,7 +626,7 @@ __global__ void __launch_bounds__(256)
   T dp[7];
 #pragma unroll
   for (int q = 0; q < 7; q++) dp[q] = FIRST ? T(0) : io.dU[q][c];
-  stage_cell<T, FIRST, LAST, DIAG, STAR>(k, io, i, j, kk, c, d, u, dp, As, Bs, tstage);
+  stage_cell<T, FIRST, LAST, DIAG, STAR, true>(k, io, i, j, kk, c, d, u, dp, As, Bs, tstage);
 }
 
 // Simple Kreiss_Oliger kernel (one thread per cell); DIAG adds the energy
@@ -619,41 +661,75 @@ __global__ void __launch_bounds__(256) ez_ko_kernel(const FlatK<T> k, const Flat
     for (int q = 0; q < 6; q++) v[q] = io.in[q][c];
     e_before = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) + (v[3] * v[3] + v[4] * v[4] + v[5] * v[5]);
   }
-  ko_cell_finish<T, STAR, DIAG>(k, io, i, j, kk, c, u, t, e_before);
+  ko_cell_finish<T, STAR, DIAG, false, true>(k, io, i, j, kk, c, u, t, e_before);
 }
 
-// Guard slabs of one axis: periodic -> copy from the interior one period
-// away (send_array_{x,y,z} on a single periodic rank, sim_env.cpp:365-438);
-// COPY mode -> copy the same cell from src to dst (frozen guards of the
-// ping-pong buffer).
 template <typename T>
 struct Ptr7 {
   T* p[7];
 };
 
-template <typename T, bool WRAP>
+// Guard cell t (0 <= t < guard_count) of a grid, without overlap: the z slabs
+// (whole x-y planes), then the y slabs of interior planes, then the x slabs
+// of interior rows.
+template <typename T>
+__device__ __forceinline__ void guard_cell(const FlatK<T>& k, long t, int& i, int& j, int& kk) {
+  const long d0 = k.dims[0], d1 = k.dims[1];
+  const int g0 = k.guard[0], g1 = k.guard[1], g2 = k.guard[2];
+  const long nzs = 2L * g2 * d0 * d1;
+  const long nys = 2L * g1 * d0 * k.n[2];
+  if (t < nzs) {
+    i = (int)(t % d0);
+    const long r = t / d0;
+    j = (int)(r % d1);
+    const int m = (int)(r / d1);
+    kk = m < g2 ? m : k.dims[2] - 2 * g2 + m;
+  } else if (t < nzs + nys) {
+    const long u = t - nzs;
+    i = (int)(u % d0);
+    const long r = u / d0;
+    const int m = (int)(r % (2 * g1));
+    kk = g2 + (int)(r / (2 * g1));
+    j = m < g1 ? m : k.dims[1] - 2 * g1 + m;
+  } else {
+    const long u = t - nzs - nys;
+    const int m = (int)(u % (2 * g0));
+    const long r = u / (2 * g0);
+    j = g1 + (int)(r % k.n[1]);
+    kk = g2 + (int)(r / k.n[1]);
+    i = m < g0 ? m : k.dims[0] - 2 * g0 + m;
+  }
+}
+
+template <typename T>
+__host__ __device__ inline long guard_count(const FlatK<T>& k) {
+  return (long)k.dims[0] * k.dims[1] * k.dims[2] - (long)k.n[0] * k.n[1] * k.n[2];
+}
+
+// Frozen guards of the step's partner buffers: every guard cell that lies in
+// the guard slab of a non-periodic axis is copied from src to dst (7 fields),
+// and src[6] also to dst2 (the third P buffer) when given.  One launch over
+// the guard cells: the six slab launches it replaces took 39 us of a 160 x 128
+// x 120 FP32 step, each bound by its launch.
+template <typename T>
 __global__ void __launch_bounds__(256)
-    guard_slab_kernel(const FlatK<T> k, int ax, const Ptr7<T> dst, const Ptr7<T> src, int nfields) {
-  const int g = k.guard[ax];
-  // slab extent: 2g along ax, full dims along the other axes
-  int ext[3] = {k.dims[0], k.dims[1], k.dims[2]};
-  ext[ax] = 2 * g;
-  const long total = (long)ext[0] * ext[1] * ext[2];
+    guard_copy_kernel(const FlatK<T> k, const Ptr7<T> dst, const Ptr7<T> src, T* dst2) {
+  const long total = guard_count(k);
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total;
        t += (long)gridDim.x * blockDim.x) {
-    int c0 = (int)(t % ext[0]);
-    long r = t / ext[0];
-    int c1 = (int)(r % ext[1]);
-    int c2 = (int)(r / ext[1]);
-    int cc[3] = {c0, c1, c2};
-    int m = cc[ax];
-    if (m >= g) m = k.dims[ax] - 2 * g + m;  // upper slab
-    cc[ax] = m;
-    int s[3] = {cc[0], cc[1], cc[2]};
-    if (WRAP) s[ax] = m < g ? m + k.n[ax] : m - k.n[ax];
-    const int di = cc[0] + (cc[1] + cc[2] * k.dims[1]) * k.dims[0];
-    const int si = s[0] + (s[1] + s[2] * k.dims[1]) * k.dims[0];
-    for (int q = 0; q < nfields; q++) dst.p[q][di] = src.p[q][si];
+    int i, j, kk;
+    guard_cell(k, t, i, j, kk);
+    const bool frozen = (!k.per[0] && (i < k.guard[0] || i >= k.guard[0] + k.n[0])) ||
+                        (!k.per[1] && (j < k.guard[1] || j >= k.guard[1] + k.n[1])) ||
+                        (!k.per[2] && (kk < k.guard[2] || kk >= k.guard[2] + k.n[2]));
+    if (!frozen) continue;
+    const long c = i + (j + (long)kk * k.dims[1]) * k.dims[0];
+    T v[7];
+#pragma unroll
+    for (int q = 0; q < 7; q++) v[q] = src.p[q][c];
+#pragma unroll
+    for (int q = 0; q < 7; q++) dst.p[q][c] = v[q];
+    if (dst2) dst2[c] = v[6];
   }
 }
 
@@ -663,42 +739,16 @@ __global__ void __launch_bounds__(256)
 // x, then y, then z slab sequence (sim_env.cpp:365-438: a corner is copied
 // along x, the copy along y, that along z, ending at the fully wrapped
 // interior cell; along a frozen axis the copies keep the frozen guard row).
-// Guard cells are enumerated without overlap: the z slabs (whole x-y
-// planes), then the y slabs of interior planes, then the x slabs of interior
-// rows.
 template <typename T>
 __global__ void __launch_bounds__(256)
     guard_wrap_kernel(const FlatK<T> k, const Ptr7<T> a, int nfields) {
   const long d0 = k.dims[0], d1 = k.dims[1];
   const int g0 = k.guard[0], g1 = k.guard[1], g2 = k.guard[2];
-  const long nzs = 2L * g2 * d0 * d1;
-  const long nys = 2L * g1 * d0 * k.n[2];
-  const long nxs = 2L * g0 * k.n[1] * k.n[2];
-  const long total = nzs + nys + nxs;
+  const long total = guard_count(k);
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total;
        t += (long)gridDim.x * blockDim.x) {
     int i, j, kk;
-    if (t < nzs) {
-      i = (int)(t % d0);
-      const long r = t / d0;
-      j = (int)(r % d1);
-      const int m = (int)(r / d1);
-      kk = m < g2 ? m : k.dims[2] - 2 * g2 + m;
-    } else if (t < nzs + nys) {
-      const long u = t - nzs;
-      i = (int)(u % d0);
-      const long r = u / d0;
-      const int m = (int)(r % (2 * g1));
-      kk = g2 + (int)(r / (2 * g1));
-      j = m < g1 ? m : k.dims[1] - 2 * g1 + m;
-    } else {
-      const long u = t - nzs - nys;
-      const int m = (int)(u % (2 * g0));
-      const long r = u / (2 * g0);
-      j = g1 + (int)(r % k.n[1]);
-      kk = g2 + (int)(r / k.n[1]);
-      i = m < g0 ? m : k.dims[0] - 2 * g0 + m;
-    }
+    guard_cell(k, t, i, j, kk);
     int si = i, sj = j, sk = kk;
     if (k.per[0]) si = i < g0 ? i + k.n[0] : (i >= g0 + k.n[0] ? i - k.n[0] : i);
     if (k.per[1]) sj = j < g1 ? j + k.n[1] : (j >= g1 + k.n[1] ? j - k.n[1] : j);

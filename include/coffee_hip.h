@@ -199,8 +199,10 @@ int coffee_set_diagnostics(coffee_ctx *ctx, int enable);
 
 /* Kernel schedule of the solver (no reference counterpart: the reference
  * has one thread-per-cell launch geometry, field_solver_EZ.cu:10-12).
- * variant 0 = LDS-tiled z-marching kernels with the default tile for the
- * Scalar type (FP32 128 x 8, FP64 64 x 8), 1 = one thread per cell, 2/3/4 =
+ * variant 0 = chosen from the grid's size (flat solver: one thread per cell
+ * on small grids, else LDS-tiled z-marching kernels with the tile and z chunk
+ * of the lowest estimated time; with a zchunk, the default tile, FP32 128 x 8,
+ * FP64 64 x 8), 1 = one thread per cell, 2/3/4 =
  * tiled 64 wide with 4/8/16 rows per tile (16 in FP32, 8 in FP64), 5/6 = tiled
  * 128/256 wide (FP32 128 x 8 and 256 x 4; FP64 128 x 4 for both), 7 = 128 x 4;
  * variant 0 in FP32 runs Kreiss-Oliger with 32-bit field offsets when every
