@@ -126,6 +126,28 @@ constexpr int gr_tile_rows() {
   return sizeof(T) == 4 ? 8 : 4;
 }
 
+// Grids whose default schedule is the point sweep + stage sweep: 11 launches
+// of one round of loads each end before 6 launches that march planes.  The two
+// cross between 32^3 (55 against 73 us per step in FP32, 77 against 90 in
+// FP64) and 64^3 (113 against 87, 185 against 153).
+bool gr_small(const coffee_grid& g) {
+  double n = 1;
+  for (int a = 0; a < 3; a++) n *= g.dims[a] - 2 * g.guard[a];
+  return n <= 100e3;
+}
+
+int gr_alloc_w(coffee_ctx* c) {
+  GrState* S = gr_state(c);
+  const size_t bytes = (size_t)c->grid.dims[0] * c->grid.dims[1] * c->grid.dims[2] * c->scalar;
+  for (int q = 0; q < 12; q++)
+    if (!S->W[q]) {
+      hipError_t e = hipMalloc(&S->W[q], bytes);
+      if (e != hipSuccess)
+        return fail(c, COFFEE_ERR_HIP, std::string("hipMalloc GR scratch: ") + hipGetErrorString(e));
+    }
+  return COFFEE_OK;
+}
+
 template <typename T>
 int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   GrState* S = gr_state(c);
@@ -174,7 +196,8 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   const int pblocks = std::min((total + 255) / 256, 8192);
   dim3 block(64, 4, 1);
   dim3 grid((k.n[0] + 63) / 64, (k.n[1] + 3) / 4, k.n[2]);
-  // variant 1: point sweep + stage sweep; others: tiled stage kernel, which
+  // variant 1, and variant 0 on small grids: point sweep + stage sweep;
+  // others: tiled stage kernel, which
   // computes every point's metric on the fly, except variant 2, which reads
   // the halo points' metric in stages 2-5 from a table filled once (at 384^3
   // FP32 with the FP32 solver's Newton-refined metric: middle stage 2.06 ms
@@ -183,18 +206,14 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   // the tiled stage kernel addresses the fields by 32-bit byte offsets:
   // arrays of 4 GiB or more take the point schedule
   const bool fits32 = (size_t)k.dims[0] * k.dims[1] * k.dims[2] * sizeof(T) < (1ull << 32);
-  const bool tiled = c->variant != 1 && fits32;
+  const bool small = c->variant == 0 && c->zchunk == 0 && gr_small(c->grid);
+  const bool tiled = c->variant != 1 && !small && fits32;
   const bool mt = tiled && c->variant == 2;
   if (!tiled || mt) {
     // the point sweep's E, H, sqrt(g) D, sqrt(g) B and the table live in
-    // scratch arrays allocated on first use
-    const size_t bytes = (size_t)k.dims[0] * k.dims[1] * k.dims[2] * sizeof(T);
-    for (int q = 0; q < 12; q++)
-      if (!S->W[q]) {
-        hipError_t e = hipMalloc(&S->W[q], bytes);
-        if (e != hipSuccess)
-          return fail(c, COFFEE_ERR_HIP, std::string("hipMalloc GR scratch: ") + hipGetErrorString(e));
-      }
+    // scratch arrays allocated on first use (small grids: with the context)
+    rc = gr_alloc_w(c);
+    if (rc) return rc;
     for (int q = 0; q < 12; q++) io.W[q] = (T*)S->W[q];
   }
   if (!tiled) S->mtab_valid = false;  // the point sweep overwrites W
@@ -209,14 +228,15 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   TileMap tm;
   tm.ntx = (k.n[0] + 63) / 64;
   tm.nty = (k.n[1] + TY - 1) / TY;
-  {
-    // two workgroups per CU (256 CUs), whole columns when the plane has enough tiles
-    const int tiles = tm.ntx * tm.nty;
-    const int nzc = std::max(1, (512 + tiles - 1) / tiles);
-    tm.zc = c->zchunk > 0 ? c->zchunk : std::max(4, (k.n[2] + nzc - 1) / nzc);
-    if (tm.zc > k.n[2]) tm.zc = k.n[2];
-    tm.nzc = (k.n[2] + tm.zc - 1) / tm.zc;
-  }
+  // whole rounds of one workgroup per CU (the registers, and in FP64 the LDS,
+  // allow no second one): 384^3 FP32 12.0 -> 10.0 ms, 192^3 1617 -> 1358 us,
+  // FP64 128^3 986 -> 841 us against the earlier two workgroups per CU for
+  // whole columns.  The start-up of a chunk measured about 8 planes in FP32, 4
+  // in FP64 (its planes take twice as long).
+  tm.zc = c->zchunk > 0 ? c->zchunk
+                        : auto_zchunk(tm.ntx * tm.nty, k.n[2], sizeof(T) == 4 ? 8.0 : 4.0, false);
+  if (tm.zc > k.n[2]) tm.zc = k.n[2];
+  tm.nzc = (k.n[2] + tm.zc - 1) / tm.zc;
   const int tblocks = tm.ntx * tm.nty * tm.nzc;
   for (int st = 0; st < 5; st++) {
     T* const* in = (st % 2 == 0) ? A : B;
@@ -314,7 +334,9 @@ int gr_create(coffee_ctx* c) {
   fill_gr<double>(c->grid, c->params, S->kd);
   if (!(c->params.a > -1.0 && c->params.a < 1.0))
     return fail(c, COFFEE_ERR_INVALID, "spin a must satisfy |a| < 1");
-  return COFFEE_OK;
+  // the default schedule of a small grid needs its scratch in the first step,
+  // which a caller may be capturing
+  return gr_small(c->grid) ? gr_alloc_w(c) : COFFEE_OK;
 }
 
 int gr_step(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t s) {

@@ -172,34 +172,7 @@ int wrap_guards(coffee_ctx* c, hipStream_t s, T* const a[7], int nfields = 7) {
   });
 }
 
-// Cost of a stage of the tiled kernels with a TX x TY tile and z split into
-// nzc chunks, in planes marched one after the other on a CU: a tile workgroup
-// of 512 or 1024 threads has a CU (256 of them) to itself, so the tiles run in
-// rounds, and a chunk of zc planes lasts zc plus about 10 (its launch, the
-// queue's first 2R + 1 planes and their latency).  Near a star some workgroups take
-// about twice as long per plane; the last of them sets the end.  `weight` is
-// the time of one plane of this tile.
-double chunk_cost(int tiles, int nz, int nzc, bool star, double weight) {
-  const int zc = (nz + nzc - 1) / nzc;
-  const int blocks = tiles * ((nz + zc - 1) / zc);
-  const int rounds = (blocks + 255) / 256;
-  return (rounds * (zc + 10.0) + (star ? zc : 0)) * weight;
-}
-
-// The z chunk of the lowest cost (at least 2 planes), and that cost.
-int auto_zchunk(int tiles, int nz, bool star, double weight, double* cost) {
-  int best = 1;
-  double least = 0;
-  for (int nzc = 1; nzc <= std::max(1, nz / 2) && nzc <= 256; nzc++) {
-    const double v = chunk_cost(tiles, nz, nzc, star, weight);
-    if (nzc == 1 || v < least) {
-      least = v;
-      best = nzc;
-    }
-  }
-  if (cost) *cost = least;
-  return (nz + best - 1) / best;
-}
+constexpr double kFlatStart = 10;  // start-up of a z chunk, in planes (chunk_cost)
 
 // Tile (columns x rows) of the tiled kernels: variant 0 without a z chunk is
 // planned by auto_schedule; with one it is the tile that measured best at
@@ -259,10 +232,10 @@ FlatSchedule auto_schedule(const FlatK<T>& k, bool star) {
   if (n <= small) return {false, 64, 8, 1};
   auto tiles = [&](int tx, int ty) { return ((k.n[0] + tx - 1) / tx) * ((k.n[1] + ty - 1) / ty); };
   double c64 = 0, c128 = 0;
-  FlatSchedule s{true, 64, 8, auto_zchunk(tiles(64, 8), k.n[2], star, 1.0, &c64)};
+  FlatSchedule s{true, 64, 8, auto_zchunk(tiles(64, 8), k.n[2], kFlatStart, star, &c64)};
   if (!f32) return s;
-  const int z128 = auto_zchunk(tiles(128, 8), k.n[2], star, 1.6, &c128);
-  return c128 < c64 ? FlatSchedule{true, 128, 8, z128} : s;
+  const int z128 = auto_zchunk(tiles(128, 8), k.n[2], kFlatStart, star, &c128);
+  return 1.6 * c128 < c64 ? FlatSchedule{true, 128, 8, z128} : s;
 }
 
 // The FP32 default tile (tile_shape variant 0) also has a Kreiss-Oliger
@@ -343,7 +316,7 @@ int ez_launch_all(coffee_ctx* c, FlatK<T> k, FlatIO<T> io, T* const A[7], T* con
   TileMap tm;
   tm.ntx = (k.n[0] + TX - 1) / TX;
   tm.nty = (k.n[1] + TY - 1) / TY;
-  tm.zc = zc > 0 ? zc : auto_zchunk(tm.ntx * tm.nty, k.n[2], star != 0, 1.0, nullptr);
+  tm.zc = zc > 0 ? zc : auto_zchunk(tm.ntx * tm.nty, k.n[2], kFlatStart, star != 0);
   if (tm.zc > k.n[2]) tm.zc = k.n[2];
   tm.nzc = (k.n[2] + tm.zc - 1) / tm.zc;
   const int tblocks = tm.ntx * tm.nty * tm.nzc;

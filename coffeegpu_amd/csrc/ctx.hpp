@@ -122,6 +122,34 @@ inline FlatK<float>& flat_k<float>(coffee_ctx* c) { return c->kf; }
 template <>
 inline FlatK<double>& flat_k<double>(coffee_ctx* c) { return c->kd; }
 
+// Cost of a z-marching tiled launch over `tiles` tile columns with z split into
+// nzc chunks, in planes marched one after the other on a CU: a workgroup has a
+// CU (256 of them) to itself, so the tiles run in rounds, and a chunk of zc
+// planes lasts zc + start (its launch, the planes that fill the queues and
+// their latency).  With `uneven`, some workgroups take about twice as long per
+// plane (cells near a star); the last of them sets the end.
+inline double chunk_cost(int tiles, int nz, int nzc, double start, bool uneven) {
+  const int zc = (nz + nzc - 1) / nzc;
+  const int blocks = tiles * ((nz + zc - 1) / zc);
+  const int rounds = (blocks + 255) / 256;
+  return rounds * (zc + start) + (uneven ? zc : 0);
+}
+
+// The z chunk of the lowest cost (at least 2 planes), and that cost.
+inline int auto_zchunk(int tiles, int nz, double start, bool uneven, double* cost = nullptr) {
+  int best = 1;
+  double least = 0;
+  for (int nzc = 1; nzc <= std::max(1, nz / 2) && nzc <= 256; nzc++) {
+    const double v = chunk_cost(tiles, nz, nzc, start, uneven);
+    if (nzc == 1 || v < least) {
+      least = v;
+      best = nzc;
+    }
+  }
+  if (cost) *cost = least;
+  return (nz + best - 1) / best;
+}
+
 // Frozen (non-periodic) guard cells of a step's partner buffers: dst takes
 // src's (7 fields), dst2 src[6]'s when given.
 template <typename T>

@@ -48,8 +48,9 @@ class FieldSolverGREZ(FieldSolverEZ):
         self._diag = False
 
     def set_schedule(self, variant: int = 0, zchunk: int = 0):
-        """0 = LDS-tiled stage kernel computing E, H on the fly, the halo
-        points' metric of stages 2-5 read from a table filled once (default);
-        1 = point sweep (E, H arrays) + stage sweep; 2 = tiled with every
-        metric point computed on the fly.  All give bitwise the same results."""
+        """0 = LDS-tiled stage kernel computing E, H and the metric on the fly,
+        on small grids the schedule of variant 1 (default); 1 = point sweep
+        (E, H arrays) + stage sweep; 2 = tiled with the halo points' metric of
+        stages 2-5 read from a table filled once.  All give bitwise the same
+        results."""
         _lib.check(self._lib.coffee_set_schedule(self._ctx, int(variant), int(zchunk)), self._ctx)
