@@ -63,26 +63,27 @@ int with_tile(int tile, F&& f) {
 
 // The first-stage / middle / last-stage kernels and the KO kernel of a tile.
 template <typename T, typename Tag, bool F, bool L, bool D>
-void launch_stage(int blocks, hipStream_t s, SphRun<T>* runs, const SphItem* items, int n,
-                  int src, T as, T bs, T cs) {
+void launch_stage(int blocks, hipStream_t s, const SphRun<T>* runs, const SphClock* clocks,
+                  const SphItem* items, int n, int src, T as, T bs, T cs) {
   constexpr int TX = Tag::tx, TY = Tag::ty;
   if constexpr (Tag::kind == 2)
-    sph_stage_march_kernel<T, TX, TY, F, L, D><<<blocks, TX, 0, s>>>(runs, items, n, src, as, bs, cs);
+    sph_stage_march_kernel<T, TX, TY, F, L, D><<<blocks, TX, 0, s>>>(runs, clocks, items, n, src, as, bs, cs);
   else if constexpr (Tag::kind == 1)
-    sph_stage_lds_kernel<T, TX, TY, F, L, D><<<blocks, TX * TY, 0, s>>>(runs, items, n, src, as, bs, cs);
+    sph_stage_lds_kernel<T, TX, TY, F, L, D><<<blocks, TX * TY, 0, s>>>(runs, clocks, items, n, src, as, bs, cs);
   else
-    sph_stage_kernel<T, TX, TY, F, L, D><<<blocks, TX * TY, 0, s>>>(runs, items, n, src, as, bs, cs);
+    sph_stage_kernel<T, TX, TY, F, L, D><<<blocks, TX * TY, 0, s>>>(runs, clocks, items, n, src, as, bs, cs);
 }
 
 template <typename T, typename Tag>
-void launch_ko(int blocks, hipStream_t s, SphRun<T>* runs, const SphItem* items, int n, int src) {
+void launch_ko(int blocks, hipStream_t s, const SphRun<T>* runs, const SphClock* clocks,
+               const SphItem* items, int n, int src, int nruns, SphClock* next) {
   constexpr int TX = Tag::tx, TY = Tag::ty;
   if constexpr (Tag::kind == 2)
-    sph_ko_march_kernel<T, TX, TY><<<blocks, TX, 0, s>>>(runs, items, n, src);
+    sph_ko_march_kernel<T, TX, TY><<<blocks, TX, 0, s>>>(runs, clocks, items, n, src, nruns, next);
   else if constexpr (Tag::kind == 1)
-    sph_ko_lds_kernel<T, TX, TY><<<blocks, TX * TY, 0, s>>>(runs, items, n, src);
+    sph_ko_lds_kernel<T, TX, TY><<<blocks, TX * TY, 0, s>>>(runs, clocks, items, n, src, nruns, next);
   else
-    sph_ko_kernel<T, TX, TY><<<blocks, TX * TY, 0, s>>>(runs, items, n, src);
+    sph_ko_kernel<T, TX, TY><<<blocks, TX * TY, 0, s>>>(runs, clocks, items, n, src, nruns, next);
 }
 
 // Workgroups of the middle-stage kernel of a tile resident per CU.
@@ -103,6 +104,7 @@ int stage_occupancy() {
 }
 
 struct SphStateBase : SolverState {
+  virtual int prepare(coffee_ctx* c, hipStream_t s) = 0;
   virtual int step(coffee_ctx* c, hipStream_t s) = 0;
 };
 
@@ -110,33 +112,40 @@ template <typename T>
 struct SphState : SphStateBase {
   std::vector<SphRun<T>> h_runs;
   SphRun<T>* d_runs = nullptr;
+  std::vector<SphClock> h_clocks;  // as set up
+  SphClock* d_clocks = nullptr;    // two of each run, see SphClock
+  int parity = 0;                  // which of the two the next step reads
   SphItem* d_items = nullptr;
   int nitems = 0;
   int tile = 0;
   int grid_blocks = 0;
   int max_n0 = 0;
+  int max_guards = 0;           // most guard and axis cells of a run
   std::vector<void*> owned;
   bool use_graph = false;
-  hipGraphExec_t graph_exec = nullptr;
-  hipGraph_t graph = nullptr;
-  int graph_tile = -1;
+  hipGraphExec_t graph_exec[2] = {};  // one step from either parity
+  hipGraph_t graph[2] = {};
 
   ~SphState() override {
     drop_graph();
     for (void* p : owned) (void)hipFree(p);
     if (d_runs) (void)hipFree(d_runs);
+    if (d_clocks) (void)hipFree(d_clocks);
     if (d_items) (void)hipFree(d_items);
   }
 
   // A captured graph holds the work-list pointer and the launch geometry of
   // the tile it was captured with: any rebuild of the work list drops it.
   void drop_graph() {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    graph_exec = nullptr;
-    graph = nullptr;
-    graph_tile = -1;
+    for (int q = 0; q < 2; q++) {
+      if (graph_exec[q]) (void)hipGraphExecDestroy(graph_exec[q]);
+      if (graph[q]) (void)hipGraphDestroy(graph[q]);
+      graph_exec[q] = nullptr;
+      graph[q] = nullptr;
+    }
   }
+
+  SphClock* clocks(int which) { return d_clocks + (size_t)which * h_clocks.size(); }
 
   int build_items(coffee_ctx* c) {
     drop_graph();
@@ -168,13 +177,15 @@ struct SphState : SphStateBase {
   template <typename Tag>
   int launch_step(coffee_ctx* c, hipStream_t s) {
     const int nr = (int)h_runs.size();
-    const dim3 gb((max_n0 + 255) / 256, nr);
-    int rc = timed(c, "sph_axis", s, [&] { sph_axis_kernel<T><<<gb, 256, 0, s>>>(d_runs, nr, 0); });
-    if (rc) return rc;
-    const dim3 gg(std::max(1, std::min(1024, (int)((long)max_n0 * 64 / 256))), nr);
-    rc = timed(c, "sph_guard_copy", s,
-               [&] { sph_guard_copy_kernel<T><<<gg, 256, 0, s>>>(d_runs, nr); });
-    if (rc) return rc;
+    const SphClock* ck = clocks(parity);
+    int rc = COFFEE_OK;
+    // the march kernels leave the axis rows to a launch of their own
+    const dim3 ga((max_n0 + 255) / 256, nr);
+    auto axis = [&](int buf) -> int {
+      if (Tag::kind != 2) return COFFEE_OK;
+      return timed(c, "sph_axis", s,
+                   [&] { sph_axis_kernel<T><<<ga, 256, 0, s>>>(d_runs, ck, nr, buf); });
+    };
     const bool dg = c->diagnostics != 0;
     for (int st = 0; st < 5; st++) {
       const int src = st & 1;
@@ -183,58 +194,73 @@ struct SphState : SphStateBase {
       rc = timed(c, name, s, [&] {
         const int g = grid_blocks, n = nitems;
         if (st == 0) {
-          if (dg) launch_stage<T, Tag, true, false, true>(g, s, d_runs, d_items, n, src, as, bs, cs);
-          else launch_stage<T, Tag, true, false, false>(g, s, d_runs, d_items, n, src, as, bs, cs);
+          if (dg) launch_stage<T, Tag, true, false, true>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
+          else launch_stage<T, Tag, true, false, false>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
         } else if (st == 4) {
-          if (dg) launch_stage<T, Tag, false, true, true>(g, s, d_runs, d_items, n, src, as, bs, cs);
-          else launch_stage<T, Tag, false, true, false>(g, s, d_runs, d_items, n, src, as, bs, cs);
+          if (dg) launch_stage<T, Tag, false, true, true>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
+          else launch_stage<T, Tag, false, true, false>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
         } else {
-          if (dg) launch_stage<T, Tag, false, false, true>(g, s, d_runs, d_items, n, src, as, bs, cs);
-          else launch_stage<T, Tag, false, false, false>(g, s, d_runs, d_items, n, src, as, bs, cs);
+          if (dg) launch_stage<T, Tag, false, false, true>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
+          else launch_stage<T, Tag, false, false, false>(g, s, d_runs, ck, d_items, n, src, as, bs, cs);
         }
       });
-      if (rc) return rc;
-      rc = timed(c, "sph_axis", s,
-                 [&] { sph_axis_kernel<T><<<gb, 256, 0, s>>>(d_runs, nr, src ^ 1); });
-      if (rc) return rc;
+      if (rc || (rc = axis(src ^ 1))) return rc;
     }
-    rc = timed(c, "sph_ko", s,
-               [&] { launch_ko<T, Tag>(grid_blocks, s, d_runs, d_items, nitems, 1); });
-    if (rc) return rc;
-    rc = timed(c, "sph_axis", s, [&] { sph_axis_kernel<T><<<gb, 256, 0, s>>>(d_runs, nr, 0); });
-    if (rc) return rc;
-    return timed(c, "sph_advance", s, [&] {
-      sph_advance_kernel<T><<<(nr + 63) / 64, 64, 0, s>>>(d_runs, nr);
+    rc = timed(c, "sph_ko", s, [&] {
+      launch_ko<T, Tag>(grid_blocks, s, d_runs, ck, d_items, nitems, 1, nr, clocks(parity ^ 1));
+    });
+    return rc ? rc : axis(0);
+  }
+
+  // Before the first step of a call.
+  int prepare(coffee_ctx* c, hipStream_t s) override {
+    const int nr = (int)h_runs.size();
+    const dim3 g((max_guards + 255) / 256, nr);
+    return timed(c, "sph_prepare", s, [&] { sph_prepare_kernel<T><<<g, 256, 0, s>>>(d_runs, clocks(parity), nr); });
+  }
+
+  int prepare_single(coffee_ctx* c, hipStream_t s) {
+    return timed(c, "sph_prepare", s, [&] {
+      sph_prepare_single_kernel<T><<<(max_guards + 255) / 256, 256, 0, s>>>(h_runs[0], d_runs,
+                                                                              h_clocks[0], clocks(parity));
     });
   }
 
-  int step_direct(coffee_ctx* c, hipStream_t s) {
+  int launch_step_tile(coffee_ctx* c, hipStream_t s) {
     return with_tile(tile, [&](auto tag) { return launch_step<decltype(tag)>(c, s); });
+  }
+
+  int step_direct(coffee_ctx* c, hipStream_t s) {
+    const int rc = launch_step_tile(c, s);
+    if (!rc) parity ^= 1;
+    return rc;
   }
 
   int step(coffee_ctx* c, hipStream_t s) override {
     if (!use_graph || c->timing || c->diagnostics) return step_direct(c, s);
-    if (!graph_exec || graph_tile != tile) {
-      drop_graph();
+    const int q = parity;
+    if (!graph_exec[q]) {
       hipStream_t cs;
       HIP_TRY(c, hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
       HIP_TRY(c, hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      int rc = step_direct(c, cs);
+      int rc = launch_step_tile(c, cs);
       hipGraph_t g = nullptr;
       hipError_t e = hipStreamEndCapture(cs, &g);
       (void)hipStreamDestroy(cs);
       if (rc) return rc;
       if (e != hipSuccess) return fail(c, COFFEE_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
-      graph = g;
-      HIP_TRY(c, hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
-      graph_tile = tile;
+      graph[q] = g;
+      HIP_TRY(c, hipGraphInstantiate(&graph_exec[q], g, nullptr, nullptr, 0));
     }
-    HIP_TRY(c, hipGraphLaunch(graph_exec, s));
+    HIP_TRY(c, hipGraphLaunch(graph_exec[q], s));
+    parity ^= 1;
     return COFFEE_OK;
   }
 
   int upload(coffee_ctx* c) {
     HIP_TRY(c, hipMemcpy(d_runs, h_runs.data(), sizeof(SphRun<T>) * h_runs.size(),
+                         hipMemcpyHostToDevice));
+    HIP_TRY(c, hipMemcpy(d_clocks, h_clocks.data(), sizeof(SphClock) * h_clocks.size(),
                          hipMemcpyHostToDevice));
     return COFFEE_OK;
   }
@@ -268,7 +294,7 @@ int validate_sph(coffee_ctx* c, const coffee_grid& g) {
 // Fill one run descriptor (parameters in Scalar, metric tables, buffers).
 template <typename T>
 int make_run(coffee_ctx* c, SphState<T>* S, const coffee_grid& g, const coffee_params& p,
-             const coffee_fields* f, int nsteps, double t0, SphRun<T>& R) {
+             const coffee_fields* f, SphRun<T>& R) {
   int rc = validate_sph(c, g);
   if (rc) return rc;
   if (!(p.dt > 0) || p.tau == 0) return fail(c, COFFEE_ERR_INVALID, "dt must be > 0 and tau != 0");
@@ -321,25 +347,34 @@ int make_run(coffee_ctx* c, SphState<T>* S, const coffee_grid& g, const coffee_p
   R.KO_geometry = p.KO_geometry;
   R.pml_on = p.pml[0] > 0;
   // metric tables r(i) = exp(x_i), sin(theta_j) at the node positions
-  std::vector<T> r(g.dims[0]), sth(g.dims[1]), r3(g.dims[0]), ir2(g.dims[0]);
+  std::vector<T> r(g.dims[0]), sth(g.dims[1]), cth(g.dims[1]), r3(g.dims[0]), ir2(g.dims[0]);
   for (int i = 0; i < g.dims[0]; i++) {
     const double rd = std::exp((double)(R.x0 + R.dx * T(i - R.g0)));
     r[i] = (T)rd;
     r3[i] = (T)(rd * rd * rd);
     ir2[i] = (T)(1.0 / (rd * rd));
   }
-  for (int j = 0; j < g.dims[1]; j++) sth[j] = (T)std::sin((double)(R.y0 + R.dy * T(j - R.g1)));
-  T *dr = nullptr, *ds = nullptr, *dr3 = nullptr, *dir2 = nullptr;
+  for (int j = 0; j < g.dims[1]; j++) {
+    sth[j] = (T)std::sin((double)(R.y0 + R.dy * T(j - R.g1)));
+    cth[j] = (T)std::cos((double)(R.y0 + R.dy * T(j - R.g1)));
+  }
+  // axis rows within half a cell of theta = 0 and pi (.cu:690-748)
+  R.axis0 = std::fabs(R.y0) < R.dy / T(2);
+  R.axis1 = std::fabs(R.y0 + R.dy * T(R.n1) - T(M_PI)) < R.dy / T(2);
+  T *dr = nullptr, *ds = nullptr, *dc = nullptr, *dr3 = nullptr, *dir2 = nullptr;
   if ((rc = alloc_owned(c, S, r.size(), &dr))) return rc;
   if ((rc = alloc_owned(c, S, sth.size(), &ds))) return rc;
+  if ((rc = alloc_owned(c, S, cth.size(), &dc))) return rc;
   if ((rc = alloc_owned(c, S, r3.size(), &dr3))) return rc;
   if ((rc = alloc_owned(c, S, ir2.size(), &dir2))) return rc;
   HIP_TRY(c, hipMemcpy(dr, r.data(), r.size() * sizeof(T), hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(ds, sth.data(), sth.size() * sizeof(T), hipMemcpyHostToDevice));
+  HIP_TRY(c, hipMemcpy(dc, cth.data(), cth.size() * sizeof(T), hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(dr3, r3.data(), r3.size() * sizeof(T), hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(dir2, ir2.data(), ir2.size() * sizeof(T), hipMemcpyHostToDevice));
   R.r = dr;
   R.sth = ds;
+  R.cth = dc;
   R.r3 = dr3;
   R.ir2 = dir2;
   R.inv_tau = (T)(1.0 / p.tau);
@@ -370,10 +405,6 @@ int make_run(coffee_ctx* c, SphState<T>* S, const coffee_grid& g, const coffee_p
       if (!R.dU[q] && (rc = alloc_owned(c, S, n, &R.dU[q]))) return rc;
       if (R.pml_on && !R.Un[q] && (rc = alloc_owned(c, S, n, &R.Un[q]))) return rc;
     }
-  R.t = t0;
-  R.step = 0;
-  R.nsteps = nsteps;
-  R.active = 1;
   return COFFEE_OK;
 }
 
@@ -383,13 +414,18 @@ int batch_create(coffee_ctx* c, int nruns, const coffee_grid* grids, const coffe
   auto* S = new SphState<T>();
   c->state = S;
   S->h_runs.resize(nruns);
+  S->h_clocks.resize(nruns);
   for (int r = 0; r < nruns; r++) {
     int rc = make_run<T>(c, S, grids[r], params[r], fields ? &fields[r] : nullptr,
-                         nsteps ? nsteps[r] : 0, t0 ? t0[r] : 0.0, S->h_runs[r]);
+                         S->h_runs[r]);
     if (rc) return rc;
-    S->max_n0 = std::max(S->max_n0, S->h_runs[r].n0);
+    S->h_clocks[r] = SphClock{t0 ? t0[r] : 0.0, 0, nsteps ? nsteps[r] : 0, 1};
+    const SphRun<T>& R = S->h_runs[r];
+    S->max_n0 = std::max(S->max_n0, R.n0);
+    S->max_guards = std::max(S->max_guards, 2 * R.g1 * R.dims0 + 2 * R.g0 * R.n1 + R.n0);
   }
   HIP_TRY(c, hipMalloc(&S->d_runs, sizeof(SphRun<T>) * nruns));
+  HIP_TRY(c, hipMalloc(&S->d_clocks, sizeof(SphClock) * 2 * nruns));
   int rc = S->upload(c);
   if (rc) return rc;
   return S->build_items(c);
@@ -452,14 +488,9 @@ int sph_step_impl(coffee_ctx* c, const coffee_fields* f, double time, hipStream_
       if (!R.Un[q]) return fail(c, COFFEE_ERR_INVALID, "absorbing layer needs Etmp, Btmp, Ptmp");
   if (c->diagnostics && (!R.J[0] || !R.J[1] || !R.J[2] || !R.divE || !R.divB))
     return fail(c, COFFEE_ERR_INVALID, "diagnostics need J, divE, divB");
-  R.t = time;
-  R.step = 0;
-  R.nsteps = 0;
-  R.active = 1;
-  HIP_TRY(c, hipMemcpyAsync(S->d_runs, &R, sizeof(SphRun<T>), hipMemcpyHostToDevice, s));
-  // the host copy must outlive the asynchronous copy
-  HIP_TRY(c, hipStreamSynchronize(s));
-  return S->step_direct(c, s);
+  S->h_clocks[0] = SphClock{time, 0, 0, 1};
+  int rc = S->prepare_single(c, s);
+  return rc ? rc : S->step_direct(c, s);
 }
 
 int sph_step(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t s) {
@@ -591,7 +622,7 @@ int autotune_impl(coffee_ctx* c, int trials, hipStream_t s, int* best, double* m
     auto launch = [&] {
       with_tile(t, [&](auto tag) {
         launch_stage<T, decltype(tag), true, false, false>(S->grid_blocks, s, S->d_runs,
-                                                           S->d_items, S->nitems, 0, T(0),
+                                                           S->clocks(S->parity), S->d_items, S->nitems, 0, T(0),
                                                            (T)kBs[0], T(0));
         return 0;
       });
@@ -688,11 +719,10 @@ int coffee_sph_batch_destroy(coffee_batch* b) {
 int coffee_sph_batch_step(coffee_batch* c, int nsteps, void* stream) {
   if (!is_batch(c)) return fail(c, COFFEE_ERR_STATE, "not a spherical batch");
   auto* S = static_cast<SphStateBase*>(c->state);
-  for (int k = 0; k < nsteps; k++) {
-    int rc = S->step(c, (hipStream_t)stream);
-    if (rc) return rc;
-  }
-  return COFFEE_OK;
+  if (nsteps < 1) return COFFEE_OK;
+  int rc = S->prepare(c, (hipStream_t)stream);
+  for (int k = 0; k < nsteps && !rc; k++) rc = S->step(c, (hipStream_t)stream);
+  return rc;
 }
 
 int coffee_sph_batch_set_tile(coffee_batch* c, int tile_index) {
@@ -751,24 +781,20 @@ int coffee_sph_batch_residuals(coffee_batch* c, double* out, void* stream) {
 int coffee_sph_batch_status(coffee_batch* c, int* active, double* t, int* step) {
   if (!is_batch(c)) return fail(c, COFFEE_ERR_STATE, "not a spherical batch");
   HIP_TRY(c, hipDeviceSynchronize());
-  if (c->scalar == 4) {
-    auto* S = static_cast<SphState<float>*>(c->state);
-    std::vector<SphRun<float>> h(S->h_runs.size());
-    HIP_TRY(c, hipMemcpy(h.data(), S->d_runs, sizeof(SphRun<float>) * h.size(), hipMemcpyDeviceToHost));
-    for (size_t r = 0; r < h.size(); r++) {
-      if (active) active[r] = h[r].active;
-      if (t) t[r] = h[r].t;
-      if (step) step[r] = h[r].step;
-    }
-  } else {
-    auto* S = static_cast<SphState<double>*>(c->state);
-    std::vector<SphRun<double>> h(S->h_runs.size());
-    HIP_TRY(c, hipMemcpy(h.data(), S->d_runs, sizeof(SphRun<double>) * h.size(), hipMemcpyDeviceToHost));
-    for (size_t r = 0; r < h.size(); r++) {
-      if (active) active[r] = h[r].active;
-      if (t) t[r] = h[r].t;
-      if (step) step[r] = h[r].step;
-    }
+  const SphClock* d;
+  size_t n;
+  auto of = [&](auto* S) {
+    d = S->clocks(S->parity);
+    n = S->h_clocks.size();
+  };
+  if (c->scalar == 4) of(static_cast<SphState<float>*>(c->state));
+  else of(static_cast<SphState<double>*>(c->state));
+  std::vector<SphClock> h(n);
+  HIP_TRY(c, hipMemcpy(h.data(), d, sizeof(SphClock) * n, hipMemcpyDeviceToHost));
+  for (size_t r = 0; r < n; r++) {
+    if (active) active[r] = h[r].active;
+    if (t) t[r] = h[r].t;
+    if (step) step[r] = h[r].step;
   }
   return COFFEE_OK;
 }

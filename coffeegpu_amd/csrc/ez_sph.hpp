@@ -16,8 +16,12 @@
 // 1+2 (.cu:200-359), clean_epar / check_eGTb (.cu:361-442, flag-gated),
 // boundary_pulsar (.cu:617-688) and, in the last stage, the radial absorbing
 // layer (.cu:750-802); U ping-pongs between two buffers.  The theta-axis
-// boundary (.cu:690-748) is a separate small launch after each stage, because
-// it reads interior rows that other workgroups update.
+// boundary (.cu:690-748) only copies new values of the three rows next to an
+// axis, so the thread that computes such a cell also stores its copies
+// (sph_store): a step is six launches.  With the axis, the guard copy and the
+// time step as launches of their own (15 in all) a small batch spent much of its
+// time in them: 64 runs of 128 x 64 FP32 151 -> 118 us per step, one FP64 run of
+// 256 x 128 stepped alone 95 -> 48 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,6 +45,8 @@ struct SphRun {
   const T* sth;   // sin(theta_j), dims1 entries
   const T* r3;    // r(i)^3: sqrt(gamma) = r^3 sin(theta)
   const T* ir2;   // 1 / r(i)^2 = gamma^11 = gamma^22
+  const T* cth;   // cos(theta_j), dims1 entries
+  int axis0, axis1;  // whether theta = 0 (row g1) and pi (row dims1 - g1) are on the grid
   T inv_tau;
   T* U[2][7];     // [0] = caller's state, [1] = ping-pong partner
   T* dU[7];
@@ -48,7 +54,14 @@ struct SphRun {
   T* J[3];
   T* divE;
   T* divB;
-  double t;       // time of the step being taken
+};
+
+// Time and step counter of a run: the part of its state that a step changes.
+// Apart from the descriptor, which the kernels read as constant memory, and
+// kept twice: steps alternate between the two, each step's Kreiss-Oliger launch
+// writing the other one (sph_advance), so that no launch reads what it writes.
+struct SphClock {
+  double t;  // time of the step being taken
   int step, nsteps, active;
 };
 
@@ -102,6 +115,8 @@ __device__ __forceinline__ T wpert_angle(T t, T th, T tps, T tpe, T dw0, T nT, T
     a = b;
     b = tmp;
   }
+  // no pulse: zero without its sines (a zero-length one keeps the expression)
+  if (dw0 == T(0) && tpe != tps && b != a) return T(0);
   const T mu = (a + b) / T(2);
   if (t >= tps && t <= tpe && th >= a && th <= b) {
     const T c = cos((th - mu) * T(M_PI) / (b - a));
@@ -136,15 +151,18 @@ __device__ __forceinline__ void sph_project(const SphRun<T>& R, T g1, T g2, T g3
   }
 }
 
-// boundary_pulsar_sph on one cell (rotating conductor r < R + dx)
+// boundary_pulsar_sph on one cell (rotating conductor r < R + dx).  cos(theta)
+// comes from a per-run table like sin(theta): evaluated here, its range
+// reduction ran in every wavefront that holds a cell of the star, half of them
+// on a 128-cell radial grid.
 template <typename T>
-__device__ __forceinline__ void sph_pulsar(const SphRun<T>& R, T r, T th, T sth, T g1, T g2,
+__device__ __forceinline__ void sph_pulsar(const SphRun<T>& R, T r, T th, T sth, T cth, T g1, T g2,
                                            T g3, T t, T (&u)[7]) {
   if (!(r < R.radius + R.dx)) return;
   const T w = R.omega + wpert_angle(t, th, R.tp_start, R.tp_end, R.dw0, R.nT, R.thp1, R.thp2) +
               wpert_angle(t, th, R.tp_start1, R.tp_end1, R.dw1, R.nT1, R.thp11, R.thp21);
   const T r3 = r * r * r;
-  const T bxn = R.b0 * (T(2) * cos(th) / r3);
+  const T bxn = R.b0 * (T(2) * cth / r3);
   const T byn = R.b0 * (sth / r3);
   const T bzn = T(0);
   const T v3n = w * r * sth;
@@ -165,6 +183,48 @@ __device__ __forceinline__ void sph_pulsar(const SphRun<T>& R, T r, T th, T sth,
     u[1] = eyn / s2;
     u[2] = T(0);
   }
+}
+
+// Copies of a new cell next to an axis (kernel_boundary_axis_sph, .cu:690-748):
+// the cell dist = 1, 2, 3 rows inside the axis row `ja` goes to the row as far
+// on the other side, with parity + for the r components and - for theta and
+// phi (P keeps its guard); the nearest one also fills the axis row itself, E_r,
+// B_r and P copied, the other components zero.
+template <typename T>
+__device__ __forceinline__ void sph_axis_copies(const SphRun<T>& R, T* const* out, int i, int ja,
+                                                int dir, int dist, const T (&u)[7]) {
+  const unsigned m = (unsigned)(i + (ja - dir * dist) * R.dims0);
+#pragma unroll
+  for (int q = 0; q < 6; q++) gst_at(out[q], m, q % 3 == 0 ? u[q] : -u[q]);
+  if (dist == 1) {
+    const unsigned a = (unsigned)(i + ja * R.dims0);
+#pragma unroll
+    for (int q = 0; q < 7; q++) gst_at(out[q], a, q % 3 == 0 ? u[q] : T(0));
+  }
+}
+
+// Stores the new values of interior cell (i, j) and, with AXIS, its copies at
+// the axes (the row theta = 0 is itself a copy; theta = pi lies in the guards).
+// The march kernels leave the axes to sph_axis_kernel: they serve batches
+// whose launches take milliseconds against its 10 us, and ran 10 % slower with
+// the copies' code in their row loop.
+template <typename T, bool AXIS>
+__device__ __forceinline__ void sph_store(const SphRun<T>& R, T* const* out, int i, int j,
+                                          const T (&u)[7]) {
+  if (!AXIS) {
+    const unsigned c = (unsigned)(i + j * R.dims0);
+#pragma unroll
+    for (int q = 0; q < 7; q++) gst_at(out[q], c, u[q]);
+    return;
+  }
+  const int below = j - R.g1, above = R.dims1 - R.g1 - j;  // rows from the axes
+  if (!(R.axis0 && below == 0)) {
+    const unsigned c = (unsigned)(i + j * R.dims0);
+#pragma unroll
+    for (int q = 0; q < 7; q++) gst_at(out[q], c, u[q]);
+    if (R.axis0 && below <= 3) sph_axis_copies(R, out, i, R.g1, 1, below, u);
+  }
+  if (R.axis1 && above <= 3) sph_axis_copies(R, out, i, R.dims1 - R.g1, -1, above, u);
 }
 
 // Stencil operands of one cell.  x(f, d) is field f at radial offset d and
@@ -193,10 +253,11 @@ struct QueueTaps {
 };
 
 // Metric tables around cell (i, j): r, r^3 at radial offsets -H..H, 1/r^2 at
-// the cell (stage only, H = 2), sin(theta) at theta offsets -H..H.
+// the cell (stage only, H = 2), sin(theta) at theta offsets -H..H, cos(theta) at
+// the cell.
 template <typename T, int H>
 struct SphGeo {
-  T r[2 * H + 1], r3[2 * H + 1], s[2 * H + 1], ir2;
+  T r[2 * H + 1], r3[2 * H + 1], s[2 * H + 1], ir2, c;
   __device__ __forceinline__ void radial(const SphRun<T>& R, int i) {
 #pragma unroll
     for (int q = 0; q <= 2 * H; q++) {
@@ -208,21 +269,23 @@ struct SphGeo {
   __device__ __forceinline__ void polar(const SphRun<T>& R, int j) {
 #pragma unroll
     for (int q = 0; q <= 2 * H; q++) s[q] = gld(R.sth + j - H + q);
+    c = gld(R.cth + j);
   }
-  // from a copy of the sin(theta) table, sl[d] = sin(theta_{j + d})
-  __device__ __forceinline__ void polar(const T* sl) {
+  // from copies of the tables: sl[d] = sin(theta_{j + d}), sl[nc] = cos(theta_j)
+  __device__ __forceinline__ void polar(const T* sl, int nc) {
 #pragma unroll
     for (int q = 0; q <= 2 * H; q++) s[q] = sl[q - H];
+    c = sl[nc];
   }
 };
 
 // One LSRK stage at interior cell (i, j) of run R: S supplies the stencil
 // operands, G the metric tables, dprev the cell's LSRK register (ignored in
 // the first stage).
-template <typename T, bool FIRST, bool LAST, bool DIAG, typename Taps>
+template <typename T, bool FIRST, bool LAST, bool DIAG, bool AXIS, typename Taps>
 __device__ __forceinline__ void sph_stage_point(const SphRun<T>& R, int i, int j, int src, T As,
                                                 T Bs, T cs, const Taps& S, const SphGeo<T, 2>& G,
-                                                const T (&dprev)[7]) {
+                                                const T (&dprev)[7], T t) {
   const unsigned c = (unsigned)(i + j * R.dims0);
   enum { EX, EY, EZ, BX, BY, BZ, PP };
   const T r = G.r[2], sth = G.s[2];
@@ -342,8 +405,8 @@ __device__ __forceinline__ void sph_stage_point(const SphRun<T>& R, int i, int j
   for (int q = 0; q < 7; q++) u[q] = fma(Bs, du[q], u[q]);
   sph_project(R, g1, g2, g3, u);
   const T th = R.y0 + R.dy * T(j - R.g1);
-  const T tstage = (T)R.t + cs * dt;
-  sph_pulsar(R, r, th, sth, g1, g2, g3, tstage, u);
+  const T tstage = t + cs * dt;
+  sph_pulsar(R, r, th, sth, G.c, g1, g2, g3, tstage, u);
   if (LAST && R.pml_on && x > R.xh) {
     T sig = T(0);
     if (r > R.rh) {
@@ -359,9 +422,7 @@ __device__ __forceinline__ void sph_stage_point(const SphRun<T>& R, int i, int j
       }
     }
   }
-  T* const* out = R.U[src ^ 1];
-#pragma unroll
-  for (int q = 0; q < 7; q++) gst_at(out[q], c, u[q]);
+  sph_store<T, AXIS>(R, R.U[src ^ 1], i, j, u);
 }
 
 // The LSRK register of cell c (not read in the first stage).
@@ -375,12 +436,14 @@ __device__ __forceinline__ void sph_load_dprev(const SphRun<T>& R, unsigned c, T
 // memory (through the caches).  src = buffer index read (0/1).
 template <typename T, int TX, int TY, bool FIRST, bool LAST, bool DIAG>
 __global__ void __launch_bounds__(TX * TY)
-    sph_stage_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items, int nitems,
+    sph_stage_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items, int nitems,
                      int src, T As, T Bs, T cs) {
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;
     const int li = (int)(threadIdx.x % TX), lj = (int)(threadIdx.x / TX);
     const int ii = it.i0 + li, jj = it.j0 + lj;  // interior-relative
     if (ii >= R.n0 || jj >= R.n1) continue;
@@ -394,8 +457,8 @@ __global__ void __launch_bounds__(TX * TY)
     G.polar(R, j);
     T dp[7];
     sph_load_dprev<T, FIRST>(R, c, dp);
-    sph_stage_point<T, FIRST, LAST, DIAG>(R, i, j, src, As, Bs, cs, StrideTaps<T, true>{F, R.dims0}, G,
-                                          dp);
+    sph_stage_point<T, FIRST, LAST, DIAG, true>(R, i, j, src, As, Bs, cs, StrideTaps<T, true>{F, R.dims0}, G,
+                                          dp, (T)ck.t);
   }
 }
 
@@ -421,7 +484,8 @@ __device__ __forceinline__ void sph_fill_tile(const SphRun<T>& R, const SphItem&
 // per field and cell instead of one per stencil tap.
 template <typename T, int TX, int TY, bool FIRST, bool LAST, bool DIAG>
 __global__ void __launch_bounds__(TX * TY)
-    sph_stage_lds_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items,
+    sph_stage_lds_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items,
                          int nitems, int src, T As, T Bs, T cs) {
   constexpr int RH = 2, LXW = TX + 2 * RH;
   __shared__ T lds[7][LXW * (TY + 2 * RH)];
@@ -429,7 +493,8 @@ __global__ void __launch_bounds__(TX * TY)
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;  // uniform: the whole workgroup works on one item
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;  // uniform: the whole workgroup works on one item
     sph_fill_tile<T, TX, TY, RH>(R, it, src, lds);
     __syncthreads();
     const int ii = it.i0 + li, jj = it.j0 + lj;
@@ -444,8 +509,8 @@ __global__ void __launch_bounds__(TX * TY)
       G.polar(R, j);
       T dp[7];
       sph_load_dprev<T, FIRST>(R, (unsigned)(i + j * R.dims0), dp);
-      sph_stage_point<T, FIRST, LAST, DIAG>(R, i, j, src, As, Bs, cs, StrideTaps<T, false>{F, LXW}, G,
-                                            dp);
+      sph_stage_point<T, FIRST, LAST, DIAG, true>(R, i, j, src, As, Bs, cs, StrideTaps<T, false>{F, LXW}, G,
+                                            dp, (T)ck.t);
     }
     __syncthreads();
   }
@@ -466,7 +531,7 @@ __global__ void __launch_bounds__(TX * TY)
 // indices are clamped to the array; clamped values feed no result.
 template <typename T, int TX, int NJ, int RH, typename Cell>
 __device__ __forceinline__ void sph_march(const SphRun<T>& R, const SphItem& it, int src,
-                                          T (&lds)[2][7][TX + 2 * RH], T (&sl)[NJ + 2 * RH],
+                                          T (&lds)[2][7][TX + 2 * RH], T (&sl)[2 * NJ + 2 * RH],
                                           Cell&& cell) {
   static_assert(TX > 2 * RH, "band narrower than its halo");
   constexpr int NQ = 2 * RH + 1;
@@ -490,6 +555,9 @@ __device__ __forceinline__ void sph_march(const SphRun<T>& R, const SphItem& it,
   const int nj = min(NJ, R.n1 - it.j0);
   // sin(theta) of rows jc - RH .. jc + nj - 1 + RH (within the theta guards)
   for (int t = li; t < nj + 2 * RH; t += TX) sl[t] = gld(R.sth + jc - RH + t);
+  // and cos(theta) of rows jc .. jc + nj - 1: a load in the row loop would wait
+  // for every prefetch in flight (first stage of the sweep 1.06 -> 1.16 ms)
+  for (int t = li; t < nj; t += TX) sl[NJ + 2 * RH + t] = gld(R.cth + jc + t);
   auto load_row = [&](T(&v)[7], int j) {
     const unsigned o = (unsigned)(gi + min(j, jmax) * s);
 #pragma unroll
@@ -553,13 +621,13 @@ __device__ __forceinline__ void sph_march(const SphRun<T>& R, const SphItem& it,
 // Per-cell work of the march kernels: prefetch() requests the cell's own
 // operands that are not stencil values (the LSRK register), operator() runs
 // the cell.
-template <typename T, bool FIRST, bool LAST, bool DIAG>
+template <typename T, int NJ, bool FIRST, bool LAST, bool DIAG>
 struct SphStageCell {
-  static constexpr int RH = 2;
+  static constexpr int RH = 2, NC = NJ + RH;
   const SphRun<T>& R;
   SphGeo<T, 2>& G;
   int src;
-  T As, Bs, cs;
+  T As, Bs, cs, t;
   T dp[7];
   __device__ __forceinline__ void prefetch(int i, int j, bool live) {
     if (live) sph_load_dprev<T, FIRST>(R, (unsigned)(i + j * R.dims0), dp);
@@ -568,27 +636,29 @@ struct SphStageCell {
   __device__ __forceinline__ void operator()(const T (&q)[7][2 * RH + 1], const T (&row)[7][LW],
                                              int lx, int i, int j, bool live, const T* sl) {
     if (!live) return;
-    G.polar(sl);
-    sph_stage_point<T, FIRST, LAST, DIAG>(R, i, j, src, As, Bs, cs,
-                                          QueueTaps<T, RH, LW>{q, row, lx}, G, dp);
+    G.polar(sl, NC);
+    sph_stage_point<T, FIRST, LAST, DIAG, false>(R, i, j, src, As, Bs, cs,
+                                          QueueTaps<T, RH, LW>{q, row, lx}, G, dp, t);
   }
 };
 
 // The stage as a theta march (bands of TX radial cells, up to NJ rows).
 template <typename T, int TX, int NJ, bool FIRST, bool LAST, bool DIAG>
 __global__ void __launch_bounds__(TX)
-    sph_stage_march_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items,
+    sph_stage_march_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items,
                            int nitems, int src, T As, T Bs, T cs) {
   __shared__ T lds[2][7][TX + 4];
-  __shared__ T sl[NJ + 4];
+  __shared__ T sl[2 * NJ + 4];
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;  // uniform: the whole workgroup works on one item
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;  // uniform: the whole workgroup works on one item
     SphGeo<T, 2> G;
     const int ii = it.i0 + (int)threadIdx.x;
     if (ii < R.n0) G.radial(R, ii + R.g0);
-    SphStageCell<T, FIRST, LAST, DIAG> cell{R, G, src, As, Bs, cs, {}};
+    SphStageCell<T, NJ, FIRST, LAST, DIAG> cell{R, G, src, As, Bs, cs, (T)ck.t, {}};
     sph_march<T, TX, NJ, 2>(R, it, src, lds, sl, cell);
   }
 }
@@ -596,10 +666,9 @@ __global__ void __launch_bounds__(TX)
 // Kreiss-Oliger on all 7 fields (kernel_KO_step1/2_sph, .cu:444-555):
 // KO_2d6 (sqrt(g)-weighted, KO_geometry) or KO_2d0, then projections and the
 // pulsar boundary at t + dt.  S supplies the operands, G the metric tables.
-template <typename T, typename Taps>
+template <typename T, bool AXIS, typename Taps>
 __device__ __forceinline__ void sph_ko_point(const SphRun<T>& R, int i, int j, int src,
-                                             const Taps& S, const SphGeo<T, 3>& G) {
-  const unsigned c = (unsigned)(i + j * R.dims0);
+                                             const Taps& S, const SphGeo<T, 3>& G, T t) {
   const T r = G.r[3], sth = G.s[3];
   const T r3c = G.r3[3];
   T gm = r3c * fabs(sth);
@@ -634,20 +703,38 @@ __device__ __forceinline__ void sph_ko_point(const SphRun<T>& R, int i, int j, i
   const T g1 = r * r, g2 = r * r, rs = r * sth, g3 = rs * rs;
   sph_project(R, g1, g2, g3, u);
   const T th = R.y0 + R.dy * T(j - R.g1);
-  sph_pulsar(R, r, th, sth, g1, g2, g3, (T)R.t + R.dt, u);
-  T* const* out = R.U[src ^ 1];
-#pragma unroll
-  for (int q = 0; q < 7; q++) gst_at(out[q], c, u[q]);
+  sph_pulsar(R, r, th, sth, G.c, g1, g2, g3, t + R.dt, u);
+  sph_store<T, AXIS>(R, R.U[src ^ 1], i, j, u);
+}
+
+// End of a step, in the first workgroup of the Kreiss-Oliger launch: the clocks
+// of the next step from this one's, which every launch of the step reads.
+// t += dt, step += 1; a run that reached its target step count becomes inactive.
+template <typename T>
+__device__ __forceinline__ void sph_advance(const SphRun<T>* runs, const SphClock* clocks,
+                                            SphClock* next, int nruns) {
+  if (blockIdx.x) return;
+  for (int run = (int)threadIdx.x; run < nruns; run += (int)blockDim.x) {
+    SphClock c = clocks[run];
+    if (c.active) {
+      c.t = (double)((T)c.t + runs[run].dt);
+      c.step += 1;
+      if (c.nsteps > 0 && c.step >= c.nsteps) c.active = 0;
+    }
+    next[run] = c;
+  }
 }
 
 template <typename T, int TX, int TY>
 __global__ void __launch_bounds__(TX * TY)
-    sph_ko_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items, int nitems,
-                  int src) {
+    sph_ko_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items, int nitems,
+                  int src, int nruns, SphClock* __restrict__ next) {
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;
     const int ii = it.i0 + (int)(threadIdx.x % TX), jj = it.j0 + (int)(threadIdx.x / TX);
     if (ii >= R.n0 || jj >= R.n1) continue;
     const int i = ii + R.g0, j = jj + R.g1;
@@ -658,21 +745,24 @@ __global__ void __launch_bounds__(TX * TY)
     SphGeo<T, 3> G;
     G.radial(R, i);
     G.polar(R, j);
-    sph_ko_point<T>(R, i, j, src, StrideTaps<T, true>{F, R.dims0}, G);
+    sph_ko_point<T, true>(R, i, j, src, StrideTaps<T, true>{F, R.dims0}, G, (T)ck.t);
   }
+  sph_advance(runs, clocks, next, nruns);
 }
 
 template <typename T, int TX, int TY>
 __global__ void __launch_bounds__(TX * TY)
-    sph_ko_lds_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items, int nitems,
-                      int src) {
+    sph_ko_lds_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items, int nitems,
+                      int src, int nruns, SphClock* __restrict__ next) {
   constexpr int RH = 3, LXW = TX + 2 * RH;
   __shared__ T lds[7][LXW * (TY + 2 * RH)];
   const int li = (int)(threadIdx.x % TX), lj = (int)(threadIdx.x / TX);
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;  // uniform: the whole workgroup works on one item
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;  // uniform: the whole workgroup works on one item
     sph_fill_tile<T, TX, TY, RH>(R, it, src, lds);
     __syncthreads();
     const int ii = it.i0 + li, jj = it.j0 + lj;
@@ -685,56 +775,62 @@ __global__ void __launch_bounds__(TX * TY)
       SphGeo<T, 3> G;
       G.radial(R, i);
       G.polar(R, j);
-      sph_ko_point<T>(R, i, j, src, StrideTaps<T, false>{F, LXW}, G);
+      sph_ko_point<T, true>(R, i, j, src, StrideTaps<T, false>{F, LXW}, G, (T)ck.t);
     }
     __syncthreads();
   }
+  sph_advance(runs, clocks, next, nruns);
 }
 
-template <typename T>
+template <typename T, int NJ>
 struct SphKoCell {
-  static constexpr int RH = 3;
+  static constexpr int RH = 3, NC = NJ + RH;
   const SphRun<T>& R;
   SphGeo<T, 3>& G;
   int src;
+  T t;
   __device__ __forceinline__ void prefetch(int, int, bool) {}
   template <int LW>
   __device__ __forceinline__ void operator()(const T (&q)[7][2 * RH + 1], const T (&row)[7][LW],
                                              int lx, int i, int j, bool live, const T* sl) {
     if (!live) return;
-    G.polar(sl);
-    sph_ko_point<T>(R, i, j, src, QueueTaps<T, RH, LW>{q, row, lx}, G);
+    G.polar(sl, NC);
+    sph_ko_point<T, false>(R, i, j, src, QueueTaps<T, RH, LW>{q, row, lx}, G, t);
   }
 };
 
 // Kreiss-Oliger as a theta march (as the stage).
 template <typename T, int TX, int NJ>
 __global__ void __launch_bounds__(TX) __attribute__((amdgpu_waves_per_eu(TX >= 512 ? 4 : 1, 8)))
-    sph_ko_march_kernel(SphRun<T>* __restrict__ runs, const SphItem* __restrict__ items,
-                        int nitems, int src) {
+    sph_ko_march_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                     const SphItem* __restrict__ items,
+                        int nitems, int src, int nruns, SphClock* __restrict__ next) {
   __shared__ T lds[2][7][TX + 6];
-  __shared__ T sl[NJ + 6];
+  __shared__ T sl[2 * NJ + 6];
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
     const SphItem it = items[w];
     const SphRun<T>& R = runs[it.run];
-    if (!R.active) continue;  // uniform: the whole workgroup works on one item
+    const SphClock ck = clocks[it.run];
+    if (!ck.active) continue;  // uniform: the whole workgroup works on one item
     SphGeo<T, 3> G;
     const int ii = it.i0 + (int)threadIdx.x;
     if (ii < R.n0) G.radial(R, ii + R.g0);
-    SphKoCell<T> cell{R, G, src};
+    SphKoCell<T, NJ> cell{R, G, src, (T)ck.t};
     sph_march<T, TX, NJ, 3>(R, it, src, lds, sl, cell);
   }
+  sph_advance(runs, clocks, next, nruns);
 }
 
 // theta-axis boundary (kernel_boundary_axis_sph, .cu:690-748) on buffer `buf`
-// of every active run: one thread per interior radial index.
+// of every active run, after a launch of the march kernels (the others store
+// the copies themselves): one thread per interior radial index.
 template <typename T>
 __global__ void __launch_bounds__(256)
-    sph_axis_kernel(SphRun<T>* __restrict__ runs, int nruns, int buf) {
+    sph_axis_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                    int nruns, int buf) {
   const int run = blockIdx.y;
-  if (run >= nruns) return;
+  if (run >= nruns || !clocks[run].active) return;
   const SphRun<T>& R = runs[run];
-  if (!R.active) return;
   for (int ii = blockIdx.x * blockDim.x + threadIdx.x; ii < R.n0; ii += gridDim.x * blockDim.x) {
     const int i = ii + R.g0;
     const int s = R.dims0;
@@ -769,57 +865,91 @@ __global__ void __launch_bounds__(256)
         gst(U[5] + d, -v[l][5]);
       }
     };
-    int j = R.g1;
-    T y = R.y0 + R.dy * T(j - R.g1);
-    if (fabs(y) < R.dy / T(2)) axis(i + j * s, 1);
-    j = R.dims1 - R.g1;
-    y = R.y0 + R.dy * T(j - R.g1);
-    if (fabs(y - T(M_PI)) < R.dy / T(2)) axis(i + j * s, -1);
+    if (R.axis0) axis(i + R.g1 * s, 1);
+    if (R.axis1) axis(i + (R.dims1 - R.g1) * s, -1);
   }
 }
 
-// Copy every guard cell (radial guard columns and theta guard rows) of the
-// caller's buffer into the partner buffer, so frozen guards are seen by the
-// stages that read the partner.
+// Start of a step or of several by one call: the axis boundary on the caller's
+// state, and every guard cell of it copied into the partner buffer (the
+// frozen guards the stages read; the axis rows are stored by every launch from
+// here on, so later steps of the call need nothing).  One thread per guard
+// cell, then one per cell of the row theta = 0.
 template <typename T>
-__global__ void __launch_bounds__(256)
-    sph_guard_copy_kernel(SphRun<T>* __restrict__ runs, int nruns) {
-  const int run = blockIdx.y;
-  if (run >= nruns) return;
-  const SphRun<T>& R = runs[run];
-  if (!R.active) return;
-  // guard cells only: the g1 full rows below and above the interior, then
-  // the g0 cells left and right of every interior row
-  const int rows = 2 * R.g1 * R.dims0;
-  const int total = rows + 2 * R.g0 * R.n1;
+__device__ __forceinline__ void sph_prepare_run(const SphRun<T>& R) {
+  const int rows = 2 * R.g1 * R.dims0, sides = 2 * R.g0 * R.n1;
+  const int total = rows + sides + (R.axis0 ? R.n0 : 0);
+  T* const* A = R.U[0];
+  T* const* B = R.U[1];
+  const int top = R.dims1 - R.g1;
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
     int i, j;
     if (t < rows) {
       const int r = t / R.dims0;
       i = t % R.dims0;
       j = r < R.g1 ? r : R.dims1 - 2 * R.g1 + r;
-    } else {
+    } else if (t < rows + sides) {
       const int u = t - rows, c = u % (2 * R.g0);
       j = R.g1 + u / (2 * R.g0);
       i = c < R.g0 ? c : R.dims0 - 2 * R.g0 + c;
+    } else {
+      j = R.g1;
+      i = R.g0 + t - rows - sides;
     }
     const unsigned o = (unsigned)(i + j * R.dims0);
+    int ja = 0, dir = 0;  // the axis row this cell belongs to, if any
+    if (i >= R.g0 && i < R.g0 + R.n0) {
+      if (R.axis0 && j <= R.g1 && j >= R.g1 - 3) {
+        ja = R.g1;
+        dir = 1;
+      } else if (R.axis1 && j >= top && j <= top + 3) {
+        ja = top;
+        dir = -1;
+      }
+    }
+    if (dir) {
+      // rows 1..3 inside the axis are read here and written by no thread
+      const int l = dir * (ja - j);  // 0 on the axis
+      const unsigned src = (unsigned)(i + (ja + dir * (l ? l : 1)) * R.dims0);
+      T v[7];
 #pragma unroll
-    for (int q = 0; q < 7; q++) gst_at(R.U[1][q], o, gld_at(R.U[0][q], o));
+      for (int q = 0; q < 6; q++) {
+        const T w = gld_at(A[q], src);
+        v[q] = q % 3 == 0 ? w : (l ? -w : T(0));
+      }
+      v[6] = l ? gld_at(A[6], o) : gld_at(A[6], src);
+#pragma unroll
+      for (int q = 0; q < 7; q++) gst_at(A[q], o, v[q]);
+#pragma unroll
+      for (int q = 0; q < 7; q++) gst_at(B[q], o, v[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 7; q++) gst_at(B[q], o, gld_at(A[q], o));
+    }
   }
 }
 
-// End of a step: t += dt, step += 1; a run that reached its target step
-// count becomes inactive.
 template <typename T>
-__global__ void sph_advance_kernel(SphRun<T>* __restrict__ runs, int nruns) {
-  const int run = blockIdx.x * blockDim.x + threadIdx.x;
-  if (run >= nruns) return;
-  SphRun<T>& R = runs[run];
-  if (!R.active) return;
-  R.t = (double)((T)R.t + R.dt);
-  R.step += 1;
-  if (R.nsteps > 0 && R.step >= R.nsteps) R.active = 0;
+__global__ void __launch_bounds__(256)
+    sph_prepare_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
+                       int nruns) {
+  const int run = blockIdx.y;
+  if (run >= nruns || !clocks[run].active) return;
+  sph_prepare_run(runs[run]);
+}
+
+// The same for a single run whose descriptor comes with the launch (it holds
+// the arrays and the time of this call): also stores it for the launches that
+// follow, so the call neither copies it nor waits for that copy.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    sph_prepare_single_kernel(const SphRun<T> R, SphRun<T>* __restrict__ run, const SphClock c,
+                              SphClock* __restrict__ clock) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *run = R;
+    *clock = c;
+  }
+  sph_prepare_run(R);
 }
 
 // Spin-down luminosity through the sphere r = rad[run] (a diagnostic of this
