@@ -1,13 +1,14 @@
 // U-Net building blocks for gfx950 (include/coffee_unet.h): BF16 activations
 // and weights, FP32 accumulation on the matrix cores.
 //
-// The 3x3 convolution is an implicit GEMM.  With Cin % 32 == 0 it runs on
-// v_mfma_f32_16x16x32_bf16 with the weights staged in LDS (conv3x3_k32
-// below); otherwise (the 16-channel input layer) on v_mfma_f32_16x16x16_bf16: the
-// M dimension is 16 pixels per wavefront (4 wavefronts = 64 pixels per
-// workgroup), N is 16*NB output channels, K runs over the 9 taps times the
-// input channels in steps of 16.  NHWC with channels padded to 16 makes every
-// A and B fragment one 8-byte load per lane (4 consecutive BF16 channels).
+// The 3x3 convolution is an implicit GEMM.  With Cin % 32 == 0 or Cin == 16 it
+// runs on v_mfma_f32_16x16x32_bf16 with the input tile and the weights staged
+// in LDS (conv3x3_tile below); otherwise, or with operands that are not 16-byte
+// aligned, on v_mfma_f32_16x16x16_bf16 from global memory: the M dimension is
+// 16 pixels per wavefront (4 wavefronts = 64 pixels per workgroup), N is 16*NB
+// output channels, K runs over the 9 taps times the input channels in steps of
+// 16.  NHWC with channels padded to 16 makes every A and B fragment one 8-byte
+// load per lane (4 consecutive BF16 channels).
 // Operand layout of the 16x16x16 instruction (wave64):
 //   A[i][k] from lane i + 16*(k/4), element k%4;
 //   B[k][j] from lane j + 16*(k/4), element k%4;
@@ -19,6 +20,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <string>
@@ -33,6 +35,8 @@ namespace {
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint16_t bf16;
+typedef short s8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ float bf2f(bf16 v) { return __uint_as_float((uint32_t)v << 16); }
 
@@ -49,6 +53,12 @@ int launch_check(const char* what) {
   return COFFEE_OK;
 }
 
+// Operand layout of the 16x16x32 instruction (wave64):
+//   A[i][k] from lane i + 16*(k/8), element k%8;
+//   B[k][j] from lane j + 16*(k/8), element k%8;
+//   D[i][j] in lane j + 16*(i/4), element i%4.
+enum ConvForm { kOut, kMasked, kPoolBack, kUpBack };  // see conv_epilogue
+
 struct ConvArgs {
   const bf16* in;
   const bf16* w;
@@ -56,6 +66,15 @@ struct ConvArgs {
   bf16* out;
   float* out32;
   int N, H, W, Cin, Cout, flip, relu;
+  // input forms (conv3x3_tile)
+  const bf16* in2;  // channels c1 .. Cin - 1 (concatenation)
+  int c1, up;       // c1 = Cin without
+  // output forms
+  int form, csplit;
+  const bf16* mask;
+  const bf16* skip;
+  bf16* out2;
+  bf16* pool;
 };
 
 template <int NB>
@@ -117,9 +136,6 @@ __global__ void __launch_bounds__(256) conv3x3_mfma(const ConvArgs a) {
     }
   }
 }
-
-typedef short s8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 // The same convolution on v_mfma_f32_16x16x32_bf16 (twice the K of the
 // 16x16x16 instruction per issue) for Cin % 32 == 0.  A workgroup of 4
@@ -234,89 +250,209 @@ __global__ void __launch_bounds__(256) conv3x3_k32(const ConvArgs a) {
   }
 }
 
-// 16-byte chunk swizzle of the 64-byte (32-channel) LDS rows of conv3x3_tile:
-// chunk c of row k lives at c ^ csw(k).  On gfx950 a ds_read_b128 whose 64
-// lanes read chunk lane / 16 of rows base + lane % 16 then runs as fast as a
-// contiguous 1 KiB read, for every base (measured); unswizzled 64-byte rows,
-// rows padded to 80 bytes and the swizzles (k >> 2) & 3 or k & 3 took 1.35x
-// as long, and the forward convolution counted a third of its LDS cycles as
-// bank conflicts with the padded rows.
-__device__ __forceinline__ int csw(int k) { return (k >> 1) & 3; }
+// Output forms of conv3x3_tile, from a wavefront's accumulators: acc[m][b][v] is
+// image row y0 + m, column x0 + lane % 16, channel co0 + 16 b + 4 (lane / 16) + v,
+// so a lane holds 4 consecutive channels of a pixel (one 8-byte store each) and
+// needs no LDS; the pixel beside it is in lane ^ 1, the one below in acc[m + 1].
+// The values rounded to BF16 between the operations are those the separate
+// kernels store, so the fused forms give the same bits.
+//   kOut: bias and ReLU, to `out` (BF16) and `out32`; with `pool`, also the 2x2
+//     averages of the stored values (coffee_unet_pool2).
+//   kMasked (backward data): the first csplit channels to `out` (stride
+//     csplit), zero where `mask` (the ReLU output they are the gradient of) is not
+//     positive; the others to `out2` unmasked (coffee_unet_combine).
+//   kPoolBack: the gradient of a 2x2 average pool, a quarter of the value to
+//     each of the four pixels of the finer grid, plus `skip`, masked
+//     (coffee_unet_pool2_bwd, then combine).
+//   kUpBack: the gradient of a nearest 2x upsampling, the sum of 2x2 stored
+//     values, masked (coffee_unet_up2_bwd, then combine).
+template <int MB, int NB>
+__device__ __forceinline__ void conv_epilogue(const ConvArgs& a, const f4 (&acc)[MB][NB],
+                                              const f4 (&bias)[NB], int img, int y0, int x, int co0) {
+  const int lk = ((int)threadIdx.x & 63) >> 4;
+  auto masked = [&](s4 o, const bf16* m) {
+    const s4 mv = *(const s4*)m;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (!(bf2f((bf16)mv[e]) > 0.f)) o[e] = 0;
+    return o;
+  };
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int c = co0 + 16 * b + 4 * lk;
+    s4 o[MB];
+#pragma unroll
+    for (int m = 0; m < MB; m++) {
+      const int y = y0 + m;
+      const bool live = y < a.H && x < a.W;
+      const long p = (long)(img * a.H + y) * a.W + x;
+      f4 v = acc[m][b];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        v[e] += bias[b][e];
+        if (a.relu) v[e] = v[e] > 0.f ? v[e] : 0.f;
+        o[m][e] = (short)f2bf(v[e]);
+      }
+      if (a.form == kOut && live) {
+        if (a.out) *(s4*)(a.out + p * a.Cout + c) = o[m];
+        if (a.out32) *(f4*)(a.out32 + p * a.Cout + c) = v;
+      } else if (a.form == kMasked && live) {
+        const bool first = c < a.csplit;
+        const long w = first ? p * a.csplit + c : p * (a.Cout - a.csplit) + c - a.csplit;
+        *(s4*)((first ? a.out : a.out2) + w) = first && a.mask ? masked(o[m], a.mask + w) : o[m];
+      } else if (a.form == kPoolBack && live) {
+        s4 d;
+#pragma unroll
+        for (int e = 0; e < 4; e++) d[e] = (short)f2bf(0.25f * bf2f((bf16)o[m][e]));
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const long w = ((long)(img * 2 * a.H + 2 * y + q / 2) * (2 * a.W) + 2 * x + q % 2) * a.Cout + c;
+          s4 r = d;
+          if (a.skip) {
+            const s4 sk = *(const s4*)(a.skip + w);
+#pragma unroll
+            for (int e = 0; e < 4; e++) r[e] = (short)f2bf(bf2f((bf16)d[e]) + bf2f((bf16)sk[e]));
+          }
+          *(s4*)(a.out + w) = a.mask ? masked(r, a.mask + w) : r;
+        }
+      }
+    }
+    if constexpr (MB % 2 == 0) {
+      if (a.form == kUpBack || a.pool) {
+        bf16* const dst = a.form == kUpBack ? a.out : a.pool;
+#pragma unroll
+        for (int m = 0; m < MB; m += 2) {
+          s4 r;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float u = bf2f((bf16)o[m][e]), d = bf2f((bf16)o[m + 1][e]);
+            const float s = (u + __shfl_xor(u, 1)) + (d + __shfl_xor(d, 1));
+            r[e] = (short)f2bf(a.form == kUpBack ? s : 0.25f * s);
+          }
+          const int y = y0 + m;
+          if (y >= a.H || x >= a.W || (x & 1)) continue;
+          const long w = ((long)(img * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1)) * a.Cout + c;
+          *(s4*)(dst + w) = a.form == kUpBack && a.mask ? masked(r, a.mask + w) : r;
+        }
+      }
+    }
+  }
+}
 
-// The same convolution with the input tile in LDS, for Cin % 32 == 0,
-// Cout % 64 == 0 and W % 16 == 0.  A workgroup (4 wavefronts) computes a tile
-// of TR image rows x 16 columns of one image x 64 output channels.  For each
-// chunk of 32 input channels it stages the (TR + 2) x 18 input pixels (zero
-// outside the image) and the 9 x 64 x 32 weights in LDS once, and all nine taps
-// read their A fragments (one 16-pixel row segment, shifted by the tap) and B
-// fragments from there, so every input value crosses the memory hierarchy
-// once per chunk instead of once per tap.  The next chunk's global loads are
-// issued before the current chunk's MFMAs, into registers; NBUF = 2
-// double-buffers the LDS, NBUF = 1 stores after a barrier (half the LDS, so two
-// workgroups share a CU).  LDS rows
-// are the 32 channels (64 bytes) with their 16-byte chunks swizzled by csw,
-// so the 16-byte fragment reads of consecutive lanes fall in distinct banks.
-// Wavefront w owns rows
-// w*TR/4 .. (w+1)*TR/4 - 1: TR/4 M fragments x 4 N fragments of
-// v_mfma_f32_16x16x32_bf16.  The epilogue goes through LDS, so every output
-// pixel's 64 channels are written as 16-byte stores.
-template <int TR, int NBUF>
-__global__ void __launch_bounds__(256) conv3x3_tile(const ConvArgs a) {
-  constexpr int TW = 16, CP = 32, IH = TR + 2, IW = TW + 2, NIN = IH * IW;
-  constexpr int MB = TR / 4, NB = 4;
-  constexpr int IN_E = NIN * CP, W_E = 9 * 64 * CP, BUF_E = IN_E + W_E;
-  constexpr int IN_LD = (NIN * 4 + 255) / 256;  // 16-byte input loads per thread
-  constexpr int W_LD = 9;                       // 9 x 64 x 4 16-byte weight loads / 256
-  constexpr int EP = 68;                        // epilogue row pitch (floats)
-  constexpr int LDS_E = NBUF * BUF_E > TR * TW * EP * 2 ? NBUF * BUF_E : TR * TW * EP * 2;
+// 16-byte chunk swizzle of the LDS rows of conv3x3_tile: chunk c of row k lives
+// at c ^ csw(k).  On gfx950 a ds_read_b128 whose 64 lanes read chunk lane / 16 of
+// 64-byte rows base + lane % 16 then runs as fast as a contiguous 1 KiB read,
+// for every base (measured); unswizzled 64-byte rows, rows padded to 80 bytes
+// and the swizzles (k >> 2) & 3 or k & 3 took 1.35x as long, and the forward
+// convolution counted a third of its LDS cycles as bank conflicts with the
+// padded rows.  Rows of 64 channels or more swizzle each 8 chunks.
+template <int PARTS>
+__device__ __forceinline__ int csw(int k) {
+  return PARTS >= 8 ? k & 7 : PARTS == 4 ? (k >> 1) & 3 : (k >> 2) & 1;
+}
+
+// The convolution with the input tile in LDS.  A workgroup (4 wavefronts)
+// computes a tile of TR image rows x 16 columns of one image x 16 NB output channels.
+// For each chunk of CP input channels it stages the (TR + 2) x 18 input pixels
+// (zero outside the image) and the 9 x 16 NB x CP weights in LDS once, so every
+// input value crosses the memory hierarchy once per chunk instead of once per
+// tap.  The next chunk's global loads are in flight, in registers, during the
+// current chunk's MFMAs; the LDS is single-buffered, so that two workgroups share
+// a CU (double-buffered, one workgroup per CU, measured 25-35 % slower).
+//
+// The order in which an output value takes its products is part of the result
+// (the BF16 rounding of a layer feeds the next ones): chunks of 32 channels, and
+// the taps within a chunk, for images of whole 16-pixel rows and whole 64-channel
+// blocks (CP = 32, any Cin % 32 == 0); the taps, and the 32-channel chunks within
+// a tap, otherwise, as conv3x3_k32 (CP = Cin = 32, 64, 128 or 256 here); Cin = 16
+// takes the taps with v_mfma_f32_16x16x16_bf16, as conv3x3_mfma.  So every shape has one
+// result, whatever tile or kernel computes it.
+//
+// With few output channels the LDS read rate counts: one 16-byte-per-lane read
+// takes 8 cycles of the CU's LDS, in which its SIMDs finish two MFMAs.  Where the
+// registers allow (SHARE) a wavefront (rows wave MB .. + MB - 1) reads each input
+// fragment of its MB + 2 rows and three column shifts once and applies all row
+// shifts of the taps to it: 3 (MB + 2) + 9 NB reads per 9 MB NB MFMAs instead of 9
+// (MB + NB).
+//
+// Input forms: `in2` continues the channels of `in` (concatenation without a
+// copy); `up` reads the input of a nearest 2x upsampling at its coarse pixels.
+// Output forms: conv_epilogue.
+template <int TR, int NB, int CP, bool FLIP>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CP > 64 ? 1 : TR == 16 || NB == 4 || CP == 64 ? 2 : 4)))
+    conv3x3_tile(const ConvArgs a) {
+  constexpr int TW = 16, IH = TR + 2, IW = TW + 2, NIN = IH * IW;
+  constexpr int PARTS = CP / 8;                 // 16-byte chunks of an LDS row
+  constexpr int SUB = CP < 32 ? 1 : CP / 32;    // MFMA steps per tap
+  constexpr int MB = TR / 4, COB = 16 * NB, NW = 9 * COB * PARTS;
+  constexpr int IN_E = NIN * CP, W_E = 9 * COB * CP;
+  constexpr int IN_LD = (NIN * PARTS + 255) / 256;  // 16-byte input loads per thread
+  constexpr int W_LD = (NW + 255) / 256;            // 16-byte weight loads per thread
+  constexpr bool SHARE = CP >= 32 && NB > 1 && 3 * (MB + 2) * SUB <= (NB == 2 ? 12 : 24);
   static_assert(TR % 4 == 0, "rows per wavefront");
-  __shared__ __attribute__((aligned(16))) bf16 lds[LDS_E];
+  __shared__ __attribute__((aligned(16))) bf16 lds[IN_E + W_E];
 
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int li = lane & 15, lk = lane >> 4;
-  const int tiles_x = a.W / TW, tiles_y = (a.H + TR - 1) / TR;
+  const int tiles_x = (a.W + TW - 1) / TW, tiles_y = (a.H + TR - 1) / TR;
   const int tile = blockIdx.x;
   const int img = tile / (tiles_x * tiles_y);
   const int rest = tile - img * tiles_x * tiles_y;
   const int y0 = (rest / tiles_x) * TR, x0 = (rest % tiles_x) * TW;
-  const int co0 = blockIdx.y * 64;
-  const int nch = a.Cin / 32;
+  const int co0 = blockIdx.y * COB;
+  const int nch = a.Cin / CP;
 
+  int ipix[IN_LD];  // input pixel of this thread's u-th load, -1 outside the image
+#pragma unroll
+  for (int u = 0; u < IN_LD; u++) {
+    const int idx = t + 256 * u, pix = idx / PARTS;
+    const int yy = y0 - 1 + pix / IW, xx = x0 - 1 + pix % IW;
+    ipix[u] = -1;
+    if (idx < NIN * PARTS && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
+      ipix[u] = a.up ? (img * (a.H >> 1) + (yy >> 1)) * (a.W >> 1) + (xx >> 1)
+                     : (img * a.H + yy) * a.W + xx;
+  }
   s8 rin[IN_LD], rw[W_LD];
   auto load_chunk = [&](int ch) __attribute__((always_inline)) {
-    const int c0 = ch * 32;
+    const int c0 = ch * CP;
 #pragma unroll
     for (int u = 0; u < IN_LD; u++) {
-      const int idx = t + 256 * u;
+      const int part = (t + 256 * u) % PARTS, c = c0 + 8 * part;
+      const bool second = c >= a.c1;
       rin[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (idx < NIN * 4) {
-        const int pix = idx >> 2, part = idx & 3;
-        const int yy = y0 - 1 + pix / IW, xx = x0 - 1 + pix % IW;
-        if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-          rin[u] = *(const s8*)(a.in + ((long)(img * a.H + yy) * a.W + xx) * a.Cin + c0 + 8 * part);
-      }
+      if (ipix[u] >= 0)
+        rin[u] = *(const s8*)(second ? a.in2 + (long)ipix[u] * (a.Cin - a.c1) + c - a.c1
+                                     : a.in + (long)ipix[u] * a.c1 + c);
     }
 #pragma unroll
     for (int u = 0; u < W_LD; u++) {
-      const int idx = t + 256 * u;  // < 9 * 64 * 4
-      const int row = idx >> 2, part = idx & 3;  // row = tap * 64 + co
-      const int tap = row >> 6, co = row & 63;
-      rw[u] = *(const s8*)(a.w + ((long)tap * a.Cout + co0 + co) * a.Cin + c0 + 8 * part);
+      const int idx = t + 256 * u;
+      const int row = idx / PARTS, part = idx % PARTS;  // row = tap * COB + co
+      const int tap = row / COB, co = row % COB;
+      if (NW % 256 == 0 || idx < NW)
+        rw[u] = *(const s8*)(a.w + ((long)tap * a.Cout + co0 + co) * a.Cin + c0 + 8 * part);
     }
   };
-  auto store_chunk = [&](bf16* buf) __attribute__((always_inline)) {
+  auto store_chunk = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < IN_LD; u++) {
-      const int idx = t + 256 * u;
-      if (idx < NIN * 4) *(s8*)&buf[(idx >> 2) * CP + 8 * ((idx & 3) ^ csw(idx >> 2))] = rin[u];
+      const int idx = t + 256 * u, k = idx / PARTS;
+      if (idx < NIN * PARTS) *(s8*)&lds[k * CP + 8 * ((idx % PARTS) ^ csw<PARTS>(k))] = rin[u];
     }
 #pragma unroll
     for (int u = 0; u < W_LD; u++) {
-      const int idx = t + 256 * u;
-      *(s8*)&buf[IN_E + (idx >> 2) * CP + 8 * ((idx & 3) ^ csw(idx >> 2))] = rw[u];
+      const int idx = t + 256 * u, k = idx / PARTS;
+      if (NW % 256 == 0 || idx < NW)
+        *(s8*)&lds[IN_E + k * CP + 8 * ((idx % PARTS) ^ csw<PARTS>(k))] = rw[u];
     }
+  };
+  // 16-byte fragment of row k, channels 32 s + 8 lk ..
+  auto frag = [&](const bf16* base, int k, int s) {
+    return __builtin_bit_cast(bf8, *(const s8*)&base[k * CP + 8 * ((4 * s + lk) ^ csw<PARTS>(k))]);
   };
 
+  // D[i = channel][j = pixel]: the weights are operand A, so that a lane ends
+  // up with consecutive channels of one pixel (conv_epilogue)
   f4 acc[MB][NB];
 #pragma unroll
   for (int m = 0; m < MB; m++)
@@ -324,77 +460,73 @@ __global__ void __launch_bounds__(256) conv3x3_tile(const ConvArgs a) {
     for (int b = 0; b < NB; b++) acc[m][b] = f4{0.f, 0.f, 0.f, 0.f};
 
   load_chunk(0);
-  store_chunk(lds);
-  __syncthreads();
-  for (int ch = 0; ch < nch; ch++) {
-    const bf16* buf = lds + (NBUF == 2 ? (ch & 1) * BUF_E : 0);
-    if (ch + 1 < nch) load_chunk(ch + 1);
-#pragma unroll
-    for (int tap = 0; tap < 9; tap++) {
-      int dy = tap / 3 - 1, dx = tap % 3 - 1;
-      if (a.flip) {
-        dy = -dy;
-        dx = -dx;
-      }
-      bf8 bfr[NB];
-#pragma unroll
-      for (int b = 0; b < NB; b++)  // csw(tap * 64 + b * 16 + li) = csw(li)
-        bfr[b] = __builtin_bit_cast(
-            bf8, *(const s8*)&buf[IN_E + (tap * 64 + b * 16 + li) * CP + 8 * (lk ^ csw(li))]);
-#pragma unroll
-      for (int m = 0; m < MB; m++) {
-        const int r = wave * MB + m;
-        const int row = (r + 1 + dy) * IW + (li + 1 + dx);
-        const bf8 af = __builtin_bit_cast(bf8, *(const s8*)&buf[row * CP + 8 * (lk ^ csw(row))]);
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-          acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[b], acc[m][b], 0, 0, 0);
-      }
-    }
-    if (NBUF == 2) {
-      // the other buffer was last read in the previous chunk, before its barrier
-      if (ch + 1 < nch) store_chunk(lds + ((ch + 1) & 1) * BUF_E);
-    } else if (ch + 1 < nch) {
-      __syncthreads();  // every wavefront is done with this chunk
-      store_chunk(lds);
-    }
-    __syncthreads();
-  }
-
-  // epilogue: accumulators -> LDS (pixel-major, 64 channels) -> 16-byte stores
-  float* ep = (float*)lds;
-#pragma unroll
-  for (int m = 0; m < MB; m++)
+  f4 bias[NB];
+  auto load_bias = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < NB; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        ep[((wave * MB + m) * TW + 4 * lk + v) * EP + b * 16 + li] = acc[m][b][v];
+      bias[b] = a.bias ? *(const f4*)(a.bias + co0 + 16 * b + 4 * lk) : f4{0.f, 0.f, 0.f, 0.f};
+  };
+  if constexpr (NB < 4) load_bias();  // where the registers are free, not after the MFMAs
+  store_chunk();
   __syncthreads();
-  for (int idx = t; idx < TR * TW * 8; idx += 256) {
-    const int px = idx >> 3, c8 = idx & 7;
-    const int yy = y0 + px / TW, xx = x0 + px % TW;
-    if (yy >= a.H) continue;
-    const long p = (long)(img * a.H + yy) * a.W + xx;
-    float v[8];
+  for (int ch = 0; ch < nch; ch++) {
+    if (ch + 1 < nch) load_chunk(ch + 1);
+    bf8 shared[SHARE ? SUB : 1][3][SHARE ? MB + 2 : 1];
+    if constexpr (SHARE) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      float val = ep[px * EP + 8 * c8 + e] + (a.bias ? a.bias[co0 + 8 * c8 + e] : 0.f);
-      if (a.relu) val = val > 0.f ? val : 0.f;
-      v[e] = val;
-    }
-    if (a.out) {
-      s8 o;
+      for (int s = 0; s < SUB; s++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) o[e] = (short)f2bf(v[e]);
-      *(s8*)(a.out + p * a.Cout + co0 + 8 * c8) = o;
+        for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+          for (int r = 0; r < MB + 2; r++)
+            shared[s][dx][r] = frag(lds, (wave * MB + r) * IW + li + dx, s);
     }
-    if (a.out32) {
-      f4* dst = (f4*)(a.out32 + p * a.Cout + co0 + 8 * c8);
-      dst[0] = f4{v[0], v[1], v[2], v[3]};
-      dst[1] = f4{v[4], v[5], v[6], v[7]};
+#pragma unroll
+    for (int tap = 0; tap < 9; tap++) {
+      // input offset (0..2, 0..2) of the tap's weights
+      const int dy = FLIP ? 2 - tap / 3 : tap / 3, dx = FLIP ? 2 - tap % 3 : tap % 3;
+      if constexpr (CP == 16) {
+        // 8-byte fragments: channels 4 lk .. of a 32-byte row
+        auto frag4 = [&](const bf16* base, int k) {
+          return *(const s4*)&base[k * CP + 8 * ((lk >> 1) ^ csw<PARTS>(k)) + 4 * (lk & 1)];
+        };
+        s4 bfr[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) bfr[b] = frag4(lds + IN_E, tap * COB + b * 16 + li);
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+          const s4 af = frag4(lds, (wave * MB + m + dy) * IW + li + dx);
+#pragma unroll
+          for (int b = 0; b < NB; b++)
+            acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bfr[b], af, acc[m][b], 0, 0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < SUB; s++) {
+          bf8 bfr[NB];
+#pragma unroll
+          for (int b = 0; b < NB; b++) bfr[b] = frag(lds + IN_E, tap * COB + b * 16 + li, s);
+#pragma unroll
+          for (int m = 0; m < MB; m++) {
+            bf8 af;
+            if constexpr (SHARE) af = shared[s][dx][m + dy];
+            else af = frag(lds, (wave * MB + m + dy) * IW + li + dx, s);
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+              acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[b], af, acc[m][b], 0, 0, 0);
+          }
+        }
+      }
+    }
+    if (ch + 1 < nch) {
+      __syncthreads();  // every wavefront is done with this chunk
+      store_chunk();
+      __syncthreads();
     }
   }
+
+  if constexpr (NB == 4) load_bias();
+  conv_epilogue<MB, NB>(a, acc, bias, img, y0 + wave * MB, x0 + li, co0);
 }
 
 // One wavefront per (pixel range, tap, 16x16 tile of (co, ci)).
@@ -440,91 +572,6 @@ __global__ void __launch_bounds__(64)
   for (int v = 0; v < 4; v++) dst[(long)(cob * 16 + 4 * lk + v) * Cin + cib * 16 + li] = acc[v];
 }
 
-// Weight gradient on v_mfma_f32_16x16x32_bf16: for one tap and one pixel
-// range a workgroup (4 wavefronts) computes a 64 (co) x 64 (ci) tile of
-// dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] (GEMM with K = pixels).
-// Each step stages 32 pixels of dz and of the shifted input in LDS, transposed
-// to channel-major rows so that a lane's 8 consecutive pixels (one MFMA
-// fragment) are one 16-byte read; the global loads (16 B = 8 channels of one
-// pixel per thread) for the next step are issued before the current step's
-// MFMAs.  Wavefront w computes channels co0 + 16 w .. + 15 against the 64
-// input channels (4 MFMAs per step).  Channels beyond Cout / Cin and pixels
-// beyond the range or the image are zero.
-__global__ void __launch_bounds__(256)
-    wgrad_k32(const bf16* __restrict__ x, const bf16* __restrict__ dz, float* __restrict__ part,
-              int N, int H, int W, int Cin, int Cout, long chunk) {
-  constexpr int LDP = 40;  // LDS row: 32 pixels + 8 of padding (bank spread)
-  __shared__ __attribute__((aligned(16))) bf16 dzt[2][64 * LDP];
-  __shared__ __attribute__((aligned(16))) bf16 xt[2][64 * LDP];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const int split = blockIdx.x, tap = blockIdx.y;
-  const int ncib = (Cin + 63) / 64;
-  const int co0 = (blockIdx.z / ncib) * 64, ci0 = (blockIdx.z % ncib) * 64;
-  const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-  const long P = (long)N * H * W;
-  const long p_begin = (long)split * chunk;
-  const long p_end = p_begin + chunk < P ? p_begin + chunk : P;
-  // staging: thread t moves 8 channels (16 B) of pixel t % 32 of the step,
-  // channels 8 (t / 32) ..; consecutive lanes write consecutive LDS columns
-  const int sp = threadIdx.x & 31, sc = (threadIdx.x >> 5) * 8;
-  const bool dz_ok = co0 + sc < Cout, x_ok = ci0 + sc < Cin;
-  auto fetch = [&](long k0, s8& vdz, s8& vx) {
-    vdz = s8{0, 0, 0, 0, 0, 0, 0, 0};
-    vx = s8{0, 0, 0, 0, 0, 0, 0, 0};
-    const long p = k0 + sp;
-    if (p >= p_end) return;
-    if (dz_ok) vdz = *(const s8*)(dz + p * Cout + co0 + sc);
-    const int px = (int)(p % W);
-    const long t = p / W;
-    const int py = (int)(t % H), pn = (int)(t / H);
-    const int yy = py + dy, xx = px + dx;
-    if (x_ok && yy >= 0 && yy < H && xx >= 0 && xx < W)
-      vx = *(const s8*)(x + ((long)(pn * H + yy) * W + xx) * Cin + ci0 + sc);
-  };
-  auto stage = [&](int buf, const s8& vdz, const s8& vx) {
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      dzt[buf][(sc + e) * LDP + sp] = (bf16)vdz[e];
-      xt[buf][(sc + e) * LDP + sp] = (bf16)vx[e];
-    }
-  };
-  f4 acc[4];
-#pragma unroll
-  for (int b = 0; b < 4; b++) acc[b] = f4{0.f, 0.f, 0.f, 0.f};
-  s8 ndz, nx;
-  fetch(p_begin, ndz, nx);
-  stage(0, ndz, nx);
-  __syncthreads();
-  int buf = 0;
-  for (long k0 = p_begin; k0 < p_end; k0 += 32) {
-    const bool more = k0 + 32 < p_end;
-    if (more) fetch(k0 + 32, ndz, nx);
-    const bf8 af = __builtin_bit_cast(bf8, *(const s8*)&dzt[buf][(wave * 16 + li) * LDP + 8 * lk]);
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-      const bf8 bfr = __builtin_bit_cast(bf8, *(const s8*)&xt[buf][(b * 16 + li) * LDP + 8 * lk]);
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr, acc[b], 0, 0, 0);
-    }
-    // buffer buf ^ 1 was last read in the previous step, before its barrier
-    if (more) stage(buf ^ 1, ndz, nx);
-    __syncthreads();
-    buf ^= 1;
-  }
-  // D[i = co][j = ci]: lane holds co = co0 + 16 wave + 4 lk + v, ci = ci0 + 16 b + li
-  float* dst = part + ((long)split * 9 + tap) * Cout * Cin;
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    const int ci = ci0 + b * 16 + li;
-    if (ci >= Cin) continue;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int co = co0 + wave * 16 + 4 * lk + v;
-      if (co < Cout) dst[(long)co * Cin + ci] = acc[b][v];
-    }
-  }
-}
-
 // Transposing 64-bit LDS read of gfx950 (ds_read_b64_tr_b16).  Within each
 // group of 16 lanes, lane 4 r + q names 4 consecutive 16-bit values (columns
 // 4 q .. 4 q + 3 of "row" r); lane i of the group receives column i of rows
@@ -535,53 +582,75 @@ __device__ __forceinline__ s4 lds_read_tr(const bf16* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
 }
 
-// 16-byte chunk swizzle of the dz tile of wgrad_tr (pixel rows of 64
-// channels = 8 chunks, 128 bytes): chunk c of pixel k lives at c ^ wswz(k),
-// which puts the 32 lanes of every transposing read (pixel rows 8 g + 4 h + r
-// of a 32-pixel step) on distinct banks with no padding.  The bits it uses
-// (1 and 3) come only from the lane's own part of the pixel index.
-__device__ __forceinline__ int wswz(int k) { return (k & 2) | ((k >> 1) & 4); }
+// 16-byte chunk swizzle of the dz tile of wgrad_tr (pixel rows of C8 chunks):
+// chunk c of pixel k lives at c ^ wswz(k).  With 32 channels (4 chunks, 64 bytes)
+// it puts the 32 lanes of every transposing read (pixel rows 8 g + 4 h + r of a
+// 32-pixel step) on distinct banks with no padding; the bits it uses (1 and 3) come
+// only from the lane's own part of the pixel index.
+template <int C8>
+__device__ __forceinline__ int wswz(int k) {
+  return C8 == 4 ? (k & 2) | ((k >> 3) & 1) : 0;
+}
 
-// Weight gradient with spatial tiles in LDS, for Cin % 64 == 0, Cout % 64 == 0
-// and W % 16 == 0: a workgroup computes the 9 x 64 (co) x 64 (ci) block of
-// dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] over a range of tiles of
-// TR image rows x 16 columns.  dz (TR x 16 pixels x 64 co) and the input
-// with its one-pixel halo are staged in LDS as they lie in memory (pixel
-// rows, channels contiguous; 16-byte stores), and both MFMA operands are read
-// with the transposing LDS read, so a tap's shift is only another row
-// address (a constant offset from the lane's base) and every staged value
-// serves all nine taps.  Input rows are padded to XS = 72 values.  Wavefront
-// w owns input channels ci0 + 16 w .. + 15 against the 64 output channels:
-// per 32-pixel step it reads 4 A fragments (shared by the taps) and 9 B
-// fragments for 36 MFMAs (v_mfma_f32_16x16x32_bf16).  The next tile's
-// global loads are in flight during the current tile's MFMAs.  Pixels beyond
-// the image are zero.  Partial blocks per range go to
-// part[range][tap][co][ci] (summed by wgrad_reduce in range order); when
-// bpart is given, the workgroups of the first input-channel block also sum dz
-// over their range, per output channel in a fixed order, into
+struct WgradArgs {
+  const bf16* x;
+  const bf16* dz;
+  float* part;
+  float* bpart;  // per-range sums of dz per output channel, or null
+  int N, H, W, Cin, Cout;
+  // input forms, as ConvArgs
+  const bf16* x2;
+  int c1, up;
+  int tiles_per_range, ntiles;
+};
+
+// Weight gradient with spatial tiles in LDS: a workgroup computes the 9 x COB
+// (co) x CIB (ci) block of dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] over a
+// range of tiles of TR image rows x 16 columns (GEMM with K = pixels).  dz (TR x 16
+// pixels x COB) and the input with its one-pixel halo are staged in LDS as they
+// lie in memory (pixel rows, channels contiguous; 16-byte stores), and both MFMA
+// operands are read with the transposing LDS read, so a tap's shift is only
+// another row address (a constant offset from the lane's base) and every staged
+// value serves all nine taps.  Input rows are padded by 8 values.
+//
+// A wavefront owns 16 input channels (CIB / 16 wavefronts side by side) against
+// all COB output channels: per 32-pixel step it reads COB / 16 A fragments (shared
+// by the taps) and 9 B fragments for 9 COB / 16 MFMAs (v_mfma_f32_16x16x32_bf16).
+// The four wavefronts are 2 (CIB = 32) or 4 (16) groups that take the steps of a
+// tile in turn, and their sums are added in group order through LDS at the end.  The next tile's global loads are in flight
+// during the current tile's MFMAs.  Pixels beyond the image are zero.  Partial
+// blocks per range go to part[range][tap][co][ci] (summed in range order by
+// wgrad_reduce); when bpart is given, the workgroups of the first input-channel
+// block also sum dz over their range, per output channel in a fixed order, into
 // bpart[range][co].
-template <int TR>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    wgrad_tr(const bf16* __restrict__ x, const bf16* __restrict__ dz, float* __restrict__ part,
-             float* __restrict__ bpart, int N, int H, int W, int Cin, int Cout,
-             int tiles_per_range, int ntiles) {
-  constexpr int TW = 16, TP = TR * TW, XW = TW + 2, XP = (TR + 2) * XW, XS = 72;
-  constexpr int NDZ = TP * 8 / 256;            // 16-byte dz loads per thread
-  constexpr int NX = (XP * 8 + 255) / 256;     // 16-byte input loads per thread
-  static_assert(TP % 32 == 0, "whole 32-pixel steps per tile");
-  static_assert(32 * 64 <= XP * XS, "bias reduction fits in the input tile");
-  __shared__ __attribute__((aligned(16))) bf16 dzs[TP * 64];
-  __shared__ __attribute__((aligned(16))) bf16 xs[XP * XS];
+template <int TR, int CIB, int COB>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    wgrad_tr(const WgradArgs a) {
+  constexpr int TW = 16, TP = TR * TW, XW = TW + 2, XP = (TR + 2) * XW, XS = CIB + 8;
+  constexpr int D8 = COB / 8, X8 = CIB / 8;          // 16-byte chunks per pixel
+  constexpr int NDZ = (TP * D8 + 255) / 256;         // 16-byte dz loads per thread
+  constexpr int NX = (XP * X8 + 255) / 256;          // 16-byte input loads per thread
+  constexpr int WC = CIB / 16, KS = 4 / WC;          // wavefronts along ci, step groups
+  constexpr int MC = COB / 16, STEPS = TP / 32;
+  constexpr int RED = KS > 1 ? 4 * 64 * MC * 4 * 2 : 0;  // one tap's sums, in bf16 units
+  constexpr int LDS_E = TP * COB + XP * XS;
+  static_assert(TP % 32 == 0 && STEPS % KS == 0, "whole 32-pixel steps per tile and group");
+  static_assert(RED <= LDS_E && 256 * 8 * 2 <= LDS_E, "reductions fit in the tiles");
+  __shared__ __attribute__((aligned(16))) bf16 lds[LDS_E];
+  bf16* const dzs = lds;
+  bf16* const xs = lds + TP * COB;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int wc = wave % WC, ks = wave / WC;
   const int li = lane & 15, lk = lane >> 4;
   const int g = lane >> 4, r = (lane >> 2) & 3, q = lane & 3;
   const int range = blockIdx.x;
-  const int ncib = Cin / 64;
-  const int co0 = (blockIdx.y / ncib) * 64, ci0 = (blockIdx.y % ncib) * 64;
-  const bool do_bias = bpart && blockIdx.y % ncib == 0;
-  const int tiles_x = W / TW, tiles_y = (H + TR - 1) / TR;
-  const int t_begin = range * tiles_per_range;
-  const int t_end = min(t_begin + tiles_per_range, ntiles);
+  const int ncib = a.Cin / CIB;
+  const int co0 = (blockIdx.y / ncib) * COB, ci0 = (blockIdx.y % ncib) * CIB;
+  const bool do_bias = a.bpart && blockIdx.y % ncib == 0;
+  const int H = a.H, W = a.W, Cin = a.Cin, Cout = a.Cout;
+  const int tiles_x = (W + TW - 1) / TW, tiles_y = (H + TR - 1) / TR;
+  const int t_begin = range * a.tiles_per_range;
+  const int t_end = min(t_begin + a.tiles_per_range, a.ntiles);
 
   s8 rdz[NDZ], rx[NX];
   auto load_tile = [&](int tile) __attribute__((always_inline)) {
@@ -590,50 +659,57 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int y0 = (rest / tiles_x) * TR, x0 = (rest % tiles_x) * TW;
 #pragma unroll
     for (int u = 0; u < NDZ; u++) {
-      const int idx = t + 256 * u, px = idx >> 3, c8 = idx & 7;
+      const int idx = t + 256 * u, px = idx / D8, c8 = idx % D8;
       const int yy = y0 + px / TW, xx = x0 + px % TW;
       rdz[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (yy < H) rdz[u] = *(const s8*)(dz + ((long)(img * H + yy) * W + xx) * Cout + co0 + 8 * c8);
+      if ((TP * D8 % 256 == 0 || idx < TP * D8) && yy < H && xx < W)
+        rdz[u] = *(const s8*)(a.dz + ((long)(img * H + yy) * W + xx) * Cout + co0 + 8 * c8);
     }
 #pragma unroll
     for (int u = 0; u < NX; u++) {
       const int idx = t + 256 * u;
       rx[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (idx < XP * 8) {
-        const int pix = idx >> 3, c8 = idx & 7;
+      if (idx < XP * X8) {
+        const int pix = idx / X8, c = ci0 + 8 * (idx % X8);
         const int yy = y0 - 1 + pix / XW, xx = x0 - 1 + pix % XW;
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-          rx[u] = *(const s8*)(x + ((long)(img * H + yy) * W + xx) * Cin + ci0 + 8 * c8);
+        if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
+          const long p = a.up ? (long)(img * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)
+                              : (long)(img * H + yy) * W + xx;
+          if (c >= a.c1) rx[u] = *(const s8*)(a.x2 + p * (Cin - a.c1) + c - a.c1);
+          else rx[u] = *(const s8*)(a.x + p * a.c1 + c);
+        }
       }
     }
   };
   auto store_tile = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < NDZ; u++) {
-      const int idx = t + 256 * u, px = idx >> 3, c8 = idx & 7;
-      *(s8*)&dzs[px * 64 + 8 * (c8 ^ wswz(px))] = rdz[u];
+      const int idx = t + 256 * u, px = idx / D8, c8 = idx % D8;
+      if (TP * D8 % 256 == 0 || idx < TP * D8)
+        *(s8*)&dzs[px * COB + 8 * (c8 ^ wswz<D8>(px))] = rdz[u];
     }
 #pragma unroll
     for (int u = 0; u < NX; u++) {
       const int idx = t + 256 * u;
-      if (idx < XP * 8) *(s8*)&xs[(idx >> 3) * XS + 8 * (idx & 7)] = rx[u];
+      if (idx < XP * X8) *(s8*)&xs[(idx / X8) * XS + 8 * (idx % X8)] = rx[u];
     }
   };
   // A: K index 8 g + 4 h + r of step st is pixel 32 st + 16 (g / 2) + 8 (g % 2)
-  // + 4 h + r; the lane's part ka fixes the swizzle, st and h add 64-value rows.
+  // + 4 h + r; the lane's part ka fixes the swizzle, st and h add whole rows.
   const int ka = 16 * (g >> 1) + 8 * (g & 1) + r;
-  const bf16* abase[4];
+  const bf16* abase[MC];
 #pragma unroll
-  for (int m = 0; m < 4; m++) abase[m] = &dzs[ka * 64 + 8 * ((2 * m + (q >> 1)) ^ wswz(ka)) + 4 * (q & 1)];
+  for (int m = 0; m < MC; m++)
+    abase[m] = &dzs[ka * COB + 8 * ((2 * m + (q >> 1)) ^ wswz<D8>(ka)) + 4 * (q & 1)];
   // B: the same pixel shifted by the tap, in the haloed input tile
-  const bf16* xbase = &xs[(((g >> 1) + 1) * XW + 8 * (g & 1) + r + 1) * XS + 8 * (2 * wave + (q >> 1)) +
+  const bf16* xbase = &xs[(((g >> 1) + 1) * XW + 8 * (g & 1) + r + 1) * XS + 8 * (2 * wc + (q >> 1)) +
                           4 * (q & 1)];
 
-  f4 acc[9][4];
+  f4 acc[9][MC];
 #pragma unroll
   for (int k = 0; k < 9; k++)
 #pragma unroll
-    for (int m = 0; m < 4; m++) acc[k][m] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MC; m++) acc[k][m] = f4{0.f, 0.f, 0.f, 0.f};
   float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (t_begin < t_end) load_tile(t_begin);
   for (int tile = t_begin; tile < t_end; tile++) {
@@ -642,22 +718,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     __syncthreads();
     if (tile + 1 < t_end) load_tile(tile + 1);
     if (do_bias) {
-      // thread (pixel group t / 8, chunk t % 8): pixels t / 8, t / 8 + 32, ...
+      // thread (pixel group t / D8, chunk t % D8): pixels t / D8, + 256 / D8, ...
 #pragma unroll
-      for (int i = 0; i < TP / 32; i++) {
-        const int px = (t >> 3) + 32 * i, c8 = t & 7;
-        const s8 v = *(const s8*)&dzs[px * 64 + 8 * (c8 ^ wswz(px))];
+      for (int i = 0; i < (TP * D8 + 255) / 256; i++) {
+        const int px = t / D8 + 256 / D8 * i, c8 = t % D8;
+        if (TP * D8 % 256 == 0 || px < TP) {
+          const s8 v = *(const s8*)&dzs[px * COB + 8 * (c8 ^ wswz<D8>(px))];
 #pragma unroll
-        for (int e = 0; e < 8; e++) bsum[e] += bf2f((bf16)v[e]);
+          for (int e = 0; e < 8; e++) bsum[e] += bf2f((bf16)v[e]);
+        }
       }
     }
 #pragma unroll 1
-    for (int st = 0; st < TP / 32; st++) {
-      bf8 af[4];
+    for (int st = ks; st < STEPS; st += KS) {
+      bf8 af[MC];
 #pragma unroll
-      for (int m = 0; m < 4; m++) {
-        const s4 lo = lds_read_tr(abase[m] + (32 * st) * 64);
-        const s4 hi = lds_read_tr(abase[m] + (32 * st + 4) * 64);
+      for (int m = 0; m < MC; m++) {
+        const s4 lo = lds_read_tr(abase[m] + (32 * st) * COB);
+        const s4 hi = lds_read_tr(abase[m] + (32 * st + 4) * COB);
         af[m] = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
       }
 #pragma unroll
@@ -668,32 +746,46 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         const s4 hi = lds_read_tr(xbase + off + 4 * XS);
         const bf8 bfr = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
 #pragma unroll
-        for (int m = 0; m < 4; m++)
+        for (int m = 0; m < MC; m++)
           acc[tap][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[m], bfr, acc[tap][m], 0, 0, 0);
       }
     }
   }
-  // D[i = co][j = ci]: lane holds co = co0 + 16 m + 4 lk + v, ci = ci0 + 16 wave + li
-  const int ci = ci0 + wave * 16 + li;
+  // D[i = co][j = ci]: lane holds co = co0 + 16 m + 4 lk + v, ci = ci0 + 16 wc + li
+  const int ci = ci0 + wc * 16 + li;
 #pragma unroll
   for (int k = 0; k < 9; k++) {
-    float* dst = part + ((long)range * 9 + k) * Cout * Cin;
+    if constexpr (KS > 1) {  // groups 1.. hand their sums of this tap to group 0
+      f4* red = (f4*)lds;    // [m][wavefront][lane]
+      __syncthreads();       // the tiles, or the previous tap, are done with
 #pragma unroll
-    for (int m = 0; m < 4; m++)
+      for (int m = 0; m < MC; m++)
+        if (ks) red[(m * 4 + wave) * 64 + lane] = acc[k][m];
+      __syncthreads();
+      if (!ks)
+#pragma unroll
+        for (int m = 0; m < MC; m++)
+#pragma unroll
+          for (int o = 1; o < KS; o++) acc[k][m] += red[(m * 4 + o * WC + wc) * 64 + lane];
+    }
+    if (ks) continue;
+    float* dst = a.part + ((long)range * 9 + k) * Cout * Cin;
+#pragma unroll
+    for (int m = 0; m < MC; m++)
 #pragma unroll
       for (int v = 0; v < 4; v++) dst[(long)(co0 + m * 16 + 4 * lk + v) * Cin + ci] = acc[k][m][v];
   }
   if (do_bias) {
-    // the 32 pixel groups' sums of each channel, added in group order
+    // the pixel groups' sums of each channel, added in group order
     __syncthreads();  // every wavefront is done with the last tile
-    float* red = (float*)xs;  // 32 x 64 floats, inside the input tile
+    float* red = (float*)lds;
 #pragma unroll
-    for (int e = 0; e < 8; e++) red[(t >> 3) * 64 + 8 * (t & 7) + e] = bsum[e];
+    for (int e = 0; e < 8; e++) red[(t / D8) * COB + 8 * (t % D8) + e] = bsum[e];
     __syncthreads();
-    if (t < 64) {
+    if (t < COB) {
       float b = 0.f;
-      for (int k = 0; k < 32; k++) b += red[k * 64 + t];
-      bpart[(long)range * Cout + co0 + t] = b;
+      for (int k = 0; k < 256 / D8; k++) b += red[k * COB + t];
+      a.bpart[(long)range * Cout + co0 + t] = b;
     }
   }
 }
@@ -980,6 +1072,104 @@ int grid_for(long total, int block = 256) {
   return (int)(b < 1 ? 1 : (b > 65535 ? 65535 : b));
 }
 
+bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
+
+// The order of products of a shape (see conv3x3_tile): by 32-channel chunks, or
+// by taps.
+bool conv_by_chunks(const ConvArgs& a) {
+  return a.Cin % 32 == 0 && a.Cout % 64 == 0 && a.W % 16 == 0;
+}
+
+// Whether conv3x3_tile takes the convolution: 16-byte aligned operands, pixel
+// indices in 32 bits, and a channel count it has the shape's order for.
+bool conv_tiled(const ConvArgs& a) {
+  return (conv_by_chunks(a) || a.Cin == 16 || a.Cin == 32 || a.Cin == 64 || a.Cin == 128 ||
+          a.Cin == 256) &&
+         (long)a.N * a.H * a.W < 2147483647L / 4 && aligned16(a.in) && aligned16(a.w) &&
+         aligned16(a.out) && aligned16(a.out32) && aligned16(a.bias);
+}
+
+template <int TR, int NB, int CP>
+void launch_conv_tile(const ConvArgs& a, hipStream_t s) {
+  const dim3 g((unsigned)((long)a.N * ((a.W + 15) / 16) * ((a.H + TR - 1) / TR)),
+               (unsigned)(a.Cout / (16 * NB)));
+  if (a.flip) conv3x3_tile<TR, NB, CP, true><<<g, 256, 0, s>>>(a);
+  else conv3x3_tile<TR, NB, CP, false><<<g, 256, 0, s>>>(a);
+}
+
+// Tile of a convolution: the largest (most MFMAs per LDS read, least halo) that
+// still gives two workgroups per CU, else one with more workgroups.
+template <int CP>
+int launch_conv(const ConvArgs& a, hipStream_t s) {
+  auto blocks = [&](int tr, int nb) {
+    return (long)a.N * ((a.W + 15) / 16) * ((a.H + tr - 1) / tr) * (a.Cout / (16 * nb));
+  };
+  const bool c32 = a.Cout % 32 == 0;
+  if (a.Cout % 64 == 0 && CP == 32 && a.H > 8 && blocks(16, 4) >= 512) launch_conv_tile<16, 4, 32>(a, s);
+  else if (a.Cout % 64 == 0 && CP == 32 && blocks(8, 4) >= 512) launch_conv_tile<8, 4, 32>(a, s);
+  else if (c32 && a.H > 4 && blocks(8, 2) >= 256) launch_conv_tile<8, 2, CP>(a, s);
+  else if (c32) launch_conv_tile<4, 2, CP>(a, s);
+  else launch_conv_tile<8, 1, CP>(a, s);
+  return launch_check("conv3x3");
+}
+
+int launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
+  if (conv_by_chunks(a)) return launch_conv<32>(a, s);
+  if (a.Cin == 256) {  // all channels staged at once: 129 KB of LDS
+    launch_conv_tile<4, 1, 256>(a, s);
+    return launch_check("conv3x3");
+  }
+  if (a.Cin == 128) {  // 101 (64) KB
+    if (a.Cout % 32 == 0) launch_conv_tile<4, 2, 128>(a, s);
+    else launch_conv_tile<4, 1, 128>(a, s);
+    return launch_check("conv3x3");
+  }
+  if (a.Cin == 64) return launch_conv<64>(a, s);
+  return a.Cin == 32 ? launch_conv<32>(a, s) : launch_conv<16>(a, s);
+}
+
+template <int CIB, int COB>
+void launch_wgrad_tr(const WgradArgs& a, int used, hipStream_t s) {
+  wgrad_tr<8, CIB, COB><<<dim3((unsigned)used, (unsigned)((a.Cout / COB) * (a.Cin / CIB))), 256, 0, s>>>(a);
+}
+
+// Partial weight gradients (and per-range bias sums, when `bias` and they fit)
+// into `part`: at most nsplit ranges of whole tiles; *used of them.
+//
+// Blocks of 32 x 32 channels (16 where the count asks for it): the partials of a
+// workgroup are 37 KB, and four times as many workgroups share a tile range as with
+// 64 x 64, so fewer ranges fill the chip and fewer partials are written and summed.
+// Two workgroups per CU, three from 32 blocks on, where the reduction has the
+// threads for more ranges (16 x 32 x 64, 256 -> 128: 42.9 us with two, 40.4 with
+// three; 16 x 64 x 128, 64 -> 64: 30.4 and 38.0).  With the reduction, against 64 x 64 blocks (and
+// one 32-pixel step at a time from global memory for the 32-channel layers): 8 x
+// 128 x 64, 128 -> 128 44 -> 42 us; 8 x 256 x 128, 64 -> 64 53 -> 45; 8 x 64 x 128, 32
+// -> 32 41 -> 21; 16 x 128 x 256, 32 -> 32 166 -> 45.
+int launch_wgrad(WgradArgs a, float* part, int nsplit, bool bias, int* used, bool* with_bias,
+                 hipStream_t s) {
+  const long ntiles = (long)a.N * ((a.W + 15) / 16) * ((a.H + 7) / 8);
+  if (ntiles > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3_wgrad: too many tiles");
+  a.ntiles = (int)ntiles;
+  const int cib = a.Cin % 32 == 0 ? 32 : 16, cob = a.Cout % 32 == 0 ? 32 : 16;
+  const long blocks = (long)(a.Cin / cib) * (a.Cout / cob);
+  const long want = std::max<long>(1, (blocks >= 32 ? 768 : 512) / blocks);
+  // room after the weight partials for one row of bias partials per range
+  long nr = std::min<long>(std::min<long>(ntiles, want), nsplit);
+  *with_bias = bias && nsplit >= 2;
+  if (*with_bias)
+    while (nr > 1 && (nsplit - nr) * 9L * a.Cin < nr) nr--;
+  *with_bias = *with_bias && (nsplit - nr) * 9L * a.Cin >= nr;
+  a.tiles_per_range = (int)((ntiles + nr - 1) / nr);
+  *used = (int)((ntiles + a.tiles_per_range - 1) / a.tiles_per_range);
+  a.part = part;
+  a.bpart = *with_bias ? part + (long)*used * 9 * a.Cout * a.Cin : nullptr;
+  if (cib == 32 && cob == 32) launch_wgrad_tr<32, 32>(a, *used, s);
+  else if (cib == 32) launch_wgrad_tr<32, 16>(a, *used, s);
+  else if (cob == 32) launch_wgrad_tr<16, 32>(a, *used, s);
+  else launch_wgrad_tr<16, 16>(a, *used, s);
+  return launch_check("conv3x3_wgrad");
+}
+
 }  // namespace
 }  // namespace coffee
 
@@ -992,29 +1182,25 @@ int coffee_unet_conv3x3(const void* in, const void* w, const float* bias, void* 
   if (!in || !w || (!out && !out32) || n < 1 || h < 1 || wd < 1 || cin < 16 || cout < 16 ||
       cin % 16 || cout % 16)
     return fail(nullptr, COFFEE_ERR_INVALID, "conv3x3: bad arguments (channels must be multiples of 16)");
-  ConvArgs a{(const bf16*)in, (const bf16*)w, bias, (bf16*)out, out32, n, h, wd, cin, cout, flip, relu};
-  hipStream_t s = (hipStream_t)stream;
+  ConvArgs a{};
+  a.in = (const bf16*)in;
+  a.w = (const bf16*)w;
+  a.bias = bias;
+  a.out = (bf16*)out;
+  a.out32 = out32;
+  a.N = n;
+  a.H = h;
+  a.W = wd;
+  a.Cin = a.c1 = cin;
+  a.Cout = a.csplit = cout;
+  a.flip = flip;
+  a.relu = relu;
+  const hipStream_t s = (hipStream_t)stream;
   const long P = (long)n * h * wd;
   const long bx = (P + 63) / 64;
   if (bx > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3: too many pixels");
-  const bool aligned16 = ((uintptr_t)in % 16 == 0) && ((uintptr_t)w % 16 == 0);
-  const bool out_aligned = ((uintptr_t)out % 16 == 0) && ((uintptr_t)out32 % 16 == 0);
-  if (cin % 32 == 0 && cout % 64 == 0 && wd % 16 == 0 && aligned16 && out_aligned) {
-    // LDS-tiled kernel: 16-row tiles where the image has them, else 8-row
-    // single-buffered LDS (72 / 60 KB), two workgroups per CU; 16-row tiles
-    // where they still give two workgroups per CU, else 8-row tiles (measured
-    // at the U-Net shapes: 8x256x128 64->64 44 us, 8x128x64 128->128 32 us,
-    // 8x64x32 256->256 31 us; the double-buffered variant, one workgroup per
-    // CU, was 25-35 % slower on the first two)
-    const long cb = cout / 64;
-    int tr = 16;
-    if (h < 16 || (long)n * (wd / 16) * ((h + 15) / 16) * cb < 512) tr = 8;
-    const long tiles = (long)n * (wd / 16) * ((h + tr - 1) / tr);
-    if (tiles > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3: too many tiles");
-    const dim3 g((unsigned)tiles, (unsigned)cb);
-    if (tr == 16) conv3x3_tile<16, 1><<<g, 256, 0, s>>>(a);
-    else conv3x3_tile<8, 1><<<g, 256, 0, s>>>(a);
-  } else if (cin % 32 == 0 && aligned16) {
+  if (conv_tiled(a)) return launch_conv_tiled(a, s);
+  if (cin % 32 == 0 && aligned16(in) && aligned16(w)) {
     // K = 32 kernel; two 16-pixel row blocks per wavefront when that still
     // leaves two workgroups per CU
     const int nb = cout % 64 == 0 ? 4 : (cout % 32 == 0 ? 2 : 1);
@@ -1047,38 +1233,27 @@ int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int
     return fail(nullptr, COFFEE_ERR_INVALID, "conv3x3_wgrad: bad arguments");
   hipStream_t s = (hipStream_t)stream;
   const long P = (long)n * h * wd;
-  long chunk = (P + nsplit - 1) / nsplit;
-  chunk = (chunk + 15) / 16 * 16;
-  int used = (int)((P + chunk - 1) / chunk);
-  const bool al16 = (uintptr_t)x % 16 == 0 && (uintptr_t)dz % 16 == 0;
+  WgradArgs a{};
+  a.x = (const bf16*)x;
+  a.dz = (const bf16*)dz;
+  a.N = n;
+  a.H = h;
+  a.W = wd;
+  a.Cin = a.c1 = cin;
+  a.Cout = cout;
+  int used = 0;
   bool fused_bias = false;
-  if (al16 && cin % 64 == 0 && cout % 64 == 0 && wd % 16 == 0) {
-    // spatial tiles of 8 rows (4 where the image is shorter), split over at
-    // most nsplit ranges of whole tiles
-    const int tr = h >= 8 ? 8 : 4;
-    const long ntiles = (long)n * (wd / 16) * ((h + tr - 1) / tr);
-    if (ntiles > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3_wgrad: too many tiles");
-    // with a bias gradient, the ranges leave room after their weight partials
-    // for one row of cout bias partials each: at most nsplit - 1 ranges
-    fused_bias = db && nsplit >= 2 && nsplit - 1 <= 9 * cin;
-    const long nr = fused_bias ? nsplit - 1 : nsplit;
-    const int per = (int)((ntiles + nr - 1) / nr);
-    used = (int)((ntiles + per - 1) / per);
-    const dim3 g((unsigned)used, (unsigned)((cout / 64) * (cin / 64)));
-    float* bpart = fused_bias ? partial + (long)used * 9 * cout * cin : nullptr;
-    if (tr == 8)
-      wgrad_tr<8><<<g, 256, 0, s>>>((const bf16*)x, (const bf16*)dz, partial, bpart, n, h, wd, cin,
-                                     cout, per, (int)ntiles);
-    else
-      wgrad_tr<4><<<g, 256, 0, s>>>((const bf16*)x, (const bf16*)dz, partial, bpart, n, h, wd, cin,
-                                     cout, per, (int)ntiles);
-  } else if (al16)
-    wgrad_k32<<<dim3(used, 9, ((cout + 63) / 64) * ((cin + 63) / 64)), 256, 0, s>>>(
-        (const bf16*)x, (const bf16*)dz, partial, n, h, wd, cin, cout, chunk);
-  else
+  int rc;
+  if (aligned16(x) && aligned16(dz)) {
+    rc = launch_wgrad(a, partial, nsplit, db != nullptr, &used, &fused_bias, s);
+  } else {
+    long chunk = (P + nsplit - 1) / nsplit;
+    chunk = (chunk + 15) / 16 * 16;
+    used = (int)((P + chunk - 1) / chunk);
     wgrad_mfma<<<dim3(used, 9, (cout / 16) * (cin / 16)), 64, 0, s>>>(
         (const bf16*)x, (const bf16*)dz, partial, n, h, wd, cin, cout, chunk);
-  int rc = launch_check("conv3x3_wgrad");
+    rc = launch_check("conv3x3_wgrad");
+  }
   if (rc) return rc;
   const long nw = 9L * cout * cin;
   // with the bias partials of wgrad_tr, one pass reduces both
