@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <vector>
 
 #include "coffee_hip.h"
 #include "coffee_unet.h"
@@ -582,6 +583,8 @@ __device__ __forceinline__ s4 lds_read_tr(const bf16* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
 }
 
+constexpr int kWgradLds = 128 * 32 + 180 * 40;  // tiles of 8 x 16 pixels, 32 x 32 channels
+
 // 16-byte chunk swizzle of the dz tile of wgrad_tr (pixel rows of C8 chunks):
 // chunk c of pixel k lives at c ^ wswz(k).  With 32 channels (4 chunks, 64 bytes)
 // it puts the 32 lanes of every transposing read (pixel rows 8 g + 4 h + r of a
@@ -597,12 +600,26 @@ struct WgradArgs {
   const bf16* dz;
   float* part;
   float* bpart;  // per-range sums of dz per output channel, or null
-  int N, H, W, Cin, Cout;
-  // input forms, as ConvArgs
-  const bf16* x2;
-  int c1, up;
-  int tiles_per_range, ntiles;
+  const bf16* x2;  // input forms, as ConvArgs
+  int N, H, W, Cin, Cout, c1, up;
+  int tiles_per_range, ntiles, ranges;
 };
+
+// Layers of one launch (at most MAX: a single layer has no table to send and search,
+// 1 us of its two launches), with the first workgroup of each (first[n] = total).
+constexpr int kWgradLayers = 32;
+template <int MAX>
+struct WgradMany {
+  int n, first[MAX + 1];
+  WgradArgs l[MAX];
+};
+
+// Entry k of ascending first workgroups that workgroup b belongs to.
+__device__ __forceinline__ int entry_of(const int* first, int n, int b) {
+  int k = 0;
+  while (k + 1 < n && b >= first[k + 1]) k++;
+  return k;
+}
 
 // Weight gradient with spatial tiles in LDS: a workgroup computes the 9 x COB
 // (co) x CIB (ci) block of dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] over a
@@ -624,8 +641,7 @@ struct WgradArgs {
 // block also sum dz over their range, per output channel in a fixed order, into
 // bpart[range][co].
 template <int TR, int CIB, int COB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-    wgrad_tr(const WgradArgs a) {
+__device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int block, bf16* lds) {
   constexpr int TW = 16, TP = TR * TW, XW = TW + 2, XP = (TR + 2) * XW, XS = CIB + 8;
   constexpr int D8 = COB / 8, X8 = CIB / 8;          // 16-byte chunks per pixel
   constexpr int NDZ = (TP * D8 + 255) / 256;         // 16-byte dz loads per thread
@@ -636,17 +652,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
   constexpr int LDS_E = TP * COB + XP * XS;
   static_assert(TP % 32 == 0 && STEPS % KS == 0, "whole 32-pixel steps per tile and group");
   static_assert(RED <= LDS_E && 256 * 8 * 2 <= LDS_E, "reductions fit in the tiles");
-  __shared__ __attribute__((aligned(16))) bf16 lds[LDS_E];
+  static_assert(LDS_E <= kWgradLds, "shared memory of wgrad_tr");
   bf16* const dzs = lds;
   bf16* const xs = lds + TP * COB;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int wc = wave % WC, ks = wave / WC;
   const int li = lane & 15, lk = lane >> 4;
   const int g = lane >> 4, r = (lane >> 2) & 3, q = lane & 3;
-  const int range = blockIdx.x;
   const int ncib = a.Cin / CIB;
-  const int co0 = (blockIdx.y / ncib) * COB, ci0 = (blockIdx.y % ncib) * CIB;
-  const bool do_bias = a.bpart && blockIdx.y % ncib == 0;
+  const int co0 = (block / ncib) * COB, ci0 = (block % ncib) * CIB;
+  const bool do_bias = a.bpart && block % ncib == 0;
   const int H = a.H, W = a.W, Cin = a.Cin, Cout = a.Cout;
   const int tiles_x = (W + TW - 1) / TW, tiles_y = (H + TR - 1) / TR;
   const int t_begin = range * a.tiles_per_range;
@@ -790,6 +805,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
   }
 }
 
+template <int MAX>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    wgrad_tr(const WgradMany<MAX> m) {
+  __shared__ __attribute__((aligned(16))) bf16 lds[kWgradLds];
+  const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
+  const WgradArgs a = m.l[k];
+  const int b = blockIdx.x - m.first[k], range = b % a.ranges, block = b / a.ranges;
+  if (a.Cin % 32 == 0) {
+    if (a.Cout % 32 == 0) wgrad_block<8, 32, 32>(a, range, block, lds);
+    else wgrad_block<8, 32, 16>(a, range, block, lds);
+  } else {
+    if (a.Cout % 32 == 0) wgrad_block<8, 16, 32>(a, range, block, lds);
+    else wgrad_block<8, 16, 16>(a, range, block, lds);
+  }
+}
+
 // Sum of m values v(k), k = 0 .. m-1, as 8 interleaved partial sums (k mod 8)
 // combined pairwise: a fixed order (deterministic results) whose loads do
 // not wait on each other.
@@ -804,15 +835,30 @@ __device__ __forceinline__ float sum8(int m, F&& v) {
   return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
-// dW[i] = sum over ranges of part[range][i]; with bpart, also db[c] = sum
-// over ranges of bpart[range][c] (threads n .. n + nb - 1), in range order.
-__global__ void wgrad_reduce(const float* __restrict__ part, float* __restrict__ dW, long n,
-                             int nsplit, const float* __restrict__ bpart, float* __restrict__ db,
-                             int nb) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n + nb; i += (long)gridDim.x * blockDim.x) {
-    if (i < n) dW[i] = sum8(nsplit, [&](int k) { return part[(long)k * n + i]; });
-    else db[i - n] = sum8(nsplit, [&](int k) { return bpart[(long)k * nb + (i - n)]; });
-  }
+struct ReduceArgs {
+  const float* part;
+  const float* bpart;
+  float* dW;
+  float* db;
+  long n;
+  int nb, ranges;
+};
+template <int MAX>
+struct ReduceMany {
+  int n, first[MAX + 1];
+  ReduceArgs l[MAX];
+};
+
+// dW[i] = sum over ranges of part[range][i], and db[c] = sum over ranges of
+// bpart[range][c] (threads n .. n + nb - 1 of a layer), in range order.
+template <int MAX>
+__global__ void __launch_bounds__(256) wgrad_reduce(const ReduceMany<MAX> m) {
+  const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
+  const ReduceArgs& a = m.l[k];
+  const long i = (blockIdx.x - m.first[k]) * 256L + threadIdx.x;
+  if (i < a.n) a.dW[i] = sum8(a.ranges, [&](int r) { return a.part[r * a.n + i]; });
+  else if (i < a.n + a.nb)
+    a.db[i - a.n] = sum8(a.ranges, [&](int r) { return a.bpart[(long)r * a.nb + (i - a.n)]; });
 }
 
 // Bias gradient db[c] = sum_p dz[p][c] in two deterministic passes.  Pass 1:
@@ -938,6 +984,14 @@ __global__ void up2_bwd_kernel(const bf16* __restrict__ dy, bf16* __restrict__ d
   }
 }
 
+constexpr int kMseBlocks = COFFEE_UNET_MSE_WORK;
+
+double mse_sum(const double* part, long npix, int nc) {
+  double tot = 0.0;
+  for (int b = 0; b < kMseBlocks; b++) tot += part[b];
+  return tot / ((double)npix * nc);
+}
+
 __global__ void __launch_bounds__(256)
     mse_kernel(const float* __restrict__ out32, int cst, const float* __restrict__ target, int nc,
                long npix, bf16* __restrict__ dout, double* __restrict__ part) {
@@ -975,6 +1029,64 @@ __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, 
     m[i] = mi;
     v[i] = vi;
     p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  }
+}
+
+struct AdamArgs {
+  float* p;
+  const float* g;
+  float* m;
+  float* v;
+  bf16* wb;  // [9][cout][cin] and its transpose, or null
+  bf16* wbt;
+  int n, cout, cin;
+};
+constexpr int kAdamTensors = 48;
+struct AdamMany {
+  int n, first[kAdamTensors + 1];
+  float lr, b1, b2, eps, c1, c2;
+  AdamArgs l[kAdamTensors];
+};
+
+// Adam step of many tensors and the BF16 copies of their new weights: a
+// workgroup takes 32 x 32 channels of one tap (1024 values of a bias), whose
+// transpose goes through LDS so that both copies are stored along their rows.
+__global__ void __launch_bounds__(256) adam_many_kernel(const AdamMany t) {
+  __shared__ bf16 tile[32][34];
+  const int k = entry_of(t.first, t.n, blockIdx.x);
+  const AdamArgs& a = t.l[k];
+  const int b = blockIdx.x - t.first[k];
+  auto step = [&](int i) {
+    const float gi = a.g[i];
+    const float mi = t.b1 * a.m[i] + (1.f - t.b1) * gi;
+    const float vi = t.b2 * a.v[i] + (1.f - t.b2) * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    const float p = a.p[i] - t.lr * (mi / t.c1) / (sqrtf(vi / t.c2) + t.eps);
+    a.p[i] = p;
+    return p;
+  };
+  if (!a.wb) {
+    for (int i = b * 1024 + threadIdx.x; i < min(a.n, (b + 1) * 1024); i += 256) step(i);
+    return;
+  }
+  const int nci = (a.cin + 31) / 32, nco = (a.cout + 31) / 32;
+  const int ci0 = (b % nci) * 32, co0 = (b / nci % nco) * 32, tap = b / (nci * nco);
+  const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int co = co0 + y + 8 * u, ci = ci0 + x;
+    if (co >= a.cout || ci >= a.cin) continue;
+    const int i = (tap * a.cout + co) * a.cin + ci;
+    const bf16 w = f2bf(step(i));
+    a.wb[i] = w;
+    tile[y + 8 * u][x] = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int ci = ci0 + y + 8 * u, co = co0 + x;
+    if (co < a.cout && ci < a.cin) a.wbt[(tap * a.cin + ci) * a.cout + co] = tile[x][y + 8 * u];
   }
 }
 
@@ -1089,6 +1201,9 @@ bool conv_tiled(const ConvArgs& a) {
          aligned16(a.out) && aligned16(a.out32) && aligned16(a.bias);
 }
 
+// Outputs of 2 x 2 pixels: a wavefront has to hold both rows (tiles of 8 rows).
+bool conv_pairs(const ConvArgs& a) { return a.form == kUpBack || a.pool; }
+
 template <int TR, int NB, int CP>
 void launch_conv_tile(const ConvArgs& a, hipStream_t s) {
   const dim3 g((unsigned)((long)a.N * ((a.W + 15) / 16) * ((a.H + TR - 1) / TR)),
@@ -1104,10 +1219,10 @@ int launch_conv(const ConvArgs& a, hipStream_t s) {
   auto blocks = [&](int tr, int nb) {
     return (long)a.N * ((a.W + 15) / 16) * ((a.H + tr - 1) / tr) * (a.Cout / (16 * nb));
   };
-  const bool c32 = a.Cout % 32 == 0;
+  const bool c32 = a.Cout % 32 == 0, pairs = conv_pairs(a);
   if (a.Cout % 64 == 0 && CP == 32 && a.H > 8 && blocks(16, 4) >= 512) launch_conv_tile<16, 4, 32>(a, s);
   else if (a.Cout % 64 == 0 && CP == 32 && blocks(8, 4) >= 512) launch_conv_tile<8, 4, 32>(a, s);
-  else if (c32 && a.H > 4 && blocks(8, 2) >= 256) launch_conv_tile<8, 2, CP>(a, s);
+  else if (c32 && (pairs || (a.H > 4 && blocks(8, 2) >= 256))) launch_conv_tile<8, 2, CP>(a, s);
   else if (c32) launch_conv_tile<4, 2, CP>(a, s);
   else launch_conv_tile<8, 1, CP>(a, s);
   return launch_check("conv3x3");
@@ -1119,8 +1234,10 @@ int launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
     launch_conv_tile<4, 1, 256>(a, s);
     return launch_check("conv3x3");
   }
-  if (a.Cin == 128) {  // 101 (64) KB
-    if (a.Cout % 32 == 0) launch_conv_tile<4, 2, 128>(a, s);
+  if (a.Cin == 128) {  // 101 (64, 121, 84) KB
+    if (conv_pairs(a) && a.Cout % 32 == 0) launch_conv_tile<8, 2, 128>(a, s);
+    else if (conv_pairs(a)) launch_conv_tile<8, 1, 128>(a, s);
+    else if (a.Cout % 32 == 0) launch_conv_tile<4, 2, 128>(a, s);
     else launch_conv_tile<4, 1, 128>(a, s);
     return launch_check("conv3x3");
   }
@@ -1128,46 +1245,55 @@ int launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
   return a.Cin == 32 ? launch_conv<32>(a, s) : launch_conv<16>(a, s);
 }
 
-template <int CIB, int COB>
-void launch_wgrad_tr(const WgradArgs& a, int used, hipStream_t s) {
-  wgrad_tr<8, CIB, COB><<<dim3((unsigned)used, (unsigned)((a.Cout / COB) * (a.Cin / CIB))), 256, 0, s>>>(a);
+int wgrad_blocks(const WgradArgs& a) {
+  return (a.Cin / (a.Cin % 32 == 0 ? 32 : 16)) * (a.Cout / (a.Cout % 32 == 0 ? 32 : 16));
 }
 
-// Partial weight gradients (and per-range bias sums, when `bias` and they fit)
-// into `part`: at most nsplit ranges of whole tiles; *used of them.
-//
+// 8 x 16-pixel tiles of a layer, -1 if they do not fit an int.
+int wgrad_tiles(const WgradArgs& a) {
+  const long t = (long)a.N * ((a.W + 15) / 16) * ((a.H + 7) / 8);
+  return t > 2147483647L ? -1 : (int)t;
+}
+
+// At most `ranges` ranges of whole tiles.
+void wgrad_set_ranges(WgradArgs& a, long ranges) {
+  ranges = std::max<long>(1, std::min<long>(ranges, a.ntiles));
+  a.tiles_per_range = (int)((a.ntiles + ranges - 1) / ranges);
+  a.ranges = (int)((a.ntiles + a.tiles_per_range - 1) / a.tiles_per_range);
+}
+
 // Blocks of 32 x 32 channels (16 where the count asks for it): the partials of a
 // workgroup are 37 KB, and four times as many workgroups share a tile range as with
 // 64 x 64, so fewer ranges fill the chip and fewer partials are written and summed.
 // Two workgroups per CU, three from 32 blocks on, where the reduction has the
 // threads for more ranges (16 x 32 x 64, 256 -> 128: 42.9 us with two, 40.4 with
-// three; 16 x 64 x 128, 64 -> 64: 30.4 and 38.0).  With the reduction, against 64 x 64 blocks (and
-// one 32-pixel step at a time from global memory for the 32-channel layers): 8 x
-// 128 x 64, 128 -> 128 44 -> 42 us; 8 x 256 x 128, 64 -> 64 53 -> 45; 8 x 64 x 128, 32
-// -> 32 41 -> 21; 16 x 128 x 256, 32 -> 32 166 -> 45.
-int launch_wgrad(WgradArgs a, float* part, int nsplit, bool bias, int* used, bool* with_bias,
-                 hipStream_t s) {
-  const long ntiles = (long)a.N * ((a.W + 15) / 16) * ((a.H + 7) / 8);
-  if (ntiles > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3_wgrad: too many tiles");
-  a.ntiles = (int)ntiles;
-  const int cib = a.Cin % 32 == 0 ? 32 : 16, cob = a.Cout % 32 == 0 ? 32 : 16;
-  const long blocks = (long)(a.Cin / cib) * (a.Cout / cob);
-  const long want = std::max<long>(1, (blocks >= 32 ? 768 : 512) / blocks);
-  // room after the weight partials for one row of bias partials per range
-  long nr = std::min<long>(std::min<long>(ntiles, want), nsplit);
-  *with_bias = bias && nsplit >= 2;
-  if (*with_bias)
-    while (nr > 1 && (nsplit - nr) * 9L * a.Cin < nr) nr--;
-  *with_bias = *with_bias && (nsplit - nr) * 9L * a.Cin >= nr;
-  a.tiles_per_range = (int)((ntiles + nr - 1) / nr);
-  *used = (int)((ntiles + a.tiles_per_range - 1) / a.tiles_per_range);
-  a.part = part;
-  a.bpart = *with_bias ? part + (long)*used * 9 * a.Cout * a.Cin : nullptr;
-  if (cib == 32 && cob == 32) launch_wgrad_tr<32, 32>(a, *used, s);
-  else if (cib == 32) launch_wgrad_tr<32, 16>(a, *used, s);
-  else if (cob == 32) launch_wgrad_tr<16, 32>(a, *used, s);
-  else launch_wgrad_tr<16, 16>(a, *used, s);
-  return launch_check("conv3x3_wgrad");
+// three; 16 x 64 x 128, 64 -> 64: 30.4 and 38.0).  With the reduction, against 64 x
+// 64 blocks (and one 32-pixel step at a time from global memory for the 32-channel
+// layers): 8 x 128 x 64, 128 -> 128 44 -> 42 us; 8 x 256 x 128, 64 -> 64 53 -> 45; 8 x
+// 64 x 128, 32 -> 32 41 -> 21; 16 x 128 x 256, 32 -> 32 166 -> 45.
+long wgrad_want(int blocks) { return std::max(1, (blocks >= 32 ? 768 : 512) / blocks); }
+
+// Partials of layers with ntiles, ranges and part set (db: bias gradients or null),
+// then their sums: two launches.
+template <int MAX>
+int launch_wgrad(const WgradArgs* l, float* const* dW, float* const* db, int n, hipStream_t s) {
+  WgradMany<MAX> m;
+  ReduceMany<MAX> r;
+  m.n = r.n = n;
+  m.first[0] = r.first[0] = 0;
+  for (int k = 0; k < n; k++) {
+    const WgradArgs& a = m.l[k] = l[k];
+    const long nw = 9L * a.Cout * a.Cin;
+    const int nb = a.bpart ? a.Cout : 0;
+    m.first[k + 1] = m.first[k] + a.ranges * wgrad_blocks(a);
+    r.first[k + 1] = r.first[k] + (int)((nw + nb + 255) / 256);
+    r.l[k] = {a.part, a.bpart, dW[k], db[k], nw, nb, a.ranges};
+  }
+  wgrad_tr<MAX><<<m.first[n], 256, 0, s>>>(m);
+  const int rc = launch_check("conv3x3_wgrad");
+  if (rc) return rc;
+  wgrad_reduce<MAX><<<r.first[n], 256, 0, s>>>(r);
+  return launch_check("wgrad_reduce");
 }
 
 }  // namespace
@@ -1227,6 +1353,59 @@ int coffee_unet_conv3x3(const void* in, const void* w, const float* bias, void* 
   return launch_check("conv3x3");
 }
 
+int coffee_unet_conv3x3_fusable(int n, int h, int wd, int cin, int cout, int pairs) {
+  if (n < 1 || h < 1 || wd < 1 || cin < 16 || cout < 16 || cin % 16 || cout % 16) return 0;
+  ConvArgs a{};
+  a.N = n;
+  a.H = h;
+  a.W = wd;
+  a.Cin = cin;
+  a.Cout = cout;
+  // all of 256 channels leave no room for tiles of 8 rows
+  return conv_tiled(a) && (!pairs || conv_by_chunks(a) || cin != 256);
+}
+
+int coffee_unet_conv3x3_fused(const coffee_unet_conv* c, void* stream) {
+  if (!c || !c->in || !c->w || (!c->out && !c->out32) ||
+      !coffee_unet_conv3x3_fusable(c->n, c->h, c->wd, c->cin, c->cout,
+                                   c->form == kUpBack || c->pool != nullptr))
+    return fail(nullptr, COFFEE_ERR_INVALID, "conv3x3_fused: bad arguments");
+  const bool even = c->h % 2 == 0 && c->wd % 2 == 0;
+  if (c->form < kOut || c->form > kUpBack || c->cin1 < 16 || c->cin1 % 16 || c->cin1 > c->cin ||
+      (c->cin1 < c->cin && !c->in2) || ((c->up || c->form == kUpBack || c->pool) && !even) ||
+      (c->form != kOut && (!c->out || c->out32 || c->pool)) ||
+      (c->form == kMasked && (c->csplit < 16 || c->csplit % 16 || c->csplit > c->cout ||
+                              (c->csplit < c->cout && !c->out2))))
+    return fail(nullptr, COFFEE_ERR_INVALID, "conv3x3_fused: inconsistent forms");
+  for (const void* p : {c->in, c->in2, c->w, (const void*)c->bias, (const void*)c->out,
+                        (const void*)c->out2, (const void*)c->out32, c->mask, c->skip,
+                        (const void*)c->pool})
+    if (!aligned16(p)) return fail(nullptr, COFFEE_ERR_INVALID, "conv3x3_fused: 16-byte alignment required");
+  ConvArgs a{};
+  a.in = (const bf16*)c->in;
+  a.in2 = (const bf16*)c->in2;
+  a.c1 = c->cin1;
+  a.up = c->up;
+  a.w = (const bf16*)c->w;
+  a.bias = c->bias;
+  a.out = (bf16*)c->out;
+  a.out2 = (bf16*)c->out2;
+  a.out32 = c->out32;
+  a.mask = (const bf16*)c->mask;
+  a.skip = (const bf16*)c->skip;
+  a.pool = (bf16*)c->pool;
+  a.form = c->form;
+  a.csplit = c->csplit;
+  a.N = c->n;
+  a.H = c->h;
+  a.W = c->wd;
+  a.Cin = c->cin;
+  a.Cout = c->cout;
+  a.flip = c->flip;
+  a.relu = c->relu;
+  return launch_conv_tiled(a, (hipStream_t)stream);
+}
+
 int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int nsplit, float* dW,
                               float* db, int n, int h, int wd, int cin, int cout, void* stream) {
   if (!x || !dz || !partial || !dW || nsplit < 1 || cin % 16 || cout % 16 || cin < 16 || cout < 16)
@@ -1241,26 +1420,39 @@ int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int
   a.W = wd;
   a.Cin = a.c1 = cin;
   a.Cout = cout;
-  int used = 0;
-  bool fused_bias = false;
-  int rc;
+  const long nw = 9L * cout * cin;
+  bool bias = false;  // summed with the weights
   if (aligned16(x) && aligned16(dz)) {
-    rc = launch_wgrad(a, partial, nsplit, db != nullptr, &used, &fused_bias, s);
+    if ((a.ntiles = wgrad_tiles(a)) < 0)
+      return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3_wgrad: too many tiles");
+    // room after the weight partials for one row of bias partials per range
+    long nr = std::min<long>(std::min<long>(a.ntiles, wgrad_want(wgrad_blocks(a))), nsplit);
+    if (db && nsplit >= 2) {
+      while (nr > 1 && (nsplit - nr) * 9L * cin < nr) nr--;
+      bias = (nsplit - nr) * 9L * cin >= nr;
+    }
+    wgrad_set_ranges(a, nr);
+    a.part = partial;
+    a.bpart = bias ? partial + a.ranges * nw : nullptr;
+    const int rc = launch_wgrad<1>(&a, &dW, &db, 1, s);
+    if (rc || !db || bias) return rc;
   } else {
     long chunk = (P + nsplit - 1) / nsplit;
     chunk = (chunk + 15) / 16 * 16;
-    used = (int)((P + chunk - 1) / chunk);
+    const int used = (int)((P + chunk - 1) / chunk);
     wgrad_mfma<<<dim3(used, 9, (cout / 16) * (cin / 16)), 64, 0, s>>>(
         (const bf16*)x, (const bf16*)dz, partial, n, h, wd, cin, cout, chunk);
-    rc = launch_check("conv3x3_wgrad");
+    int rc = launch_check("conv3x3_wgrad");
+    if (rc) return rc;
+    ReduceMany<1> r;
+    r.n = 1;
+    r.first[0] = 0;
+    r.first[1] = (int)((nw + 255) / 256);
+    r.l[0] = {partial, nullptr, dW, nullptr, nw, 0, used};
+    wgrad_reduce<1><<<r.first[1], 256, 0, s>>>(r);
+    rc = launch_check("wgrad_reduce");
+    if (rc || !db) return rc;
   }
-  if (rc) return rc;
-  const long nw = 9L * cout * cin;
-  // with the bias partials of wgrad_tr, one pass reduces both
-  const int nb = fused_bias ? cout : 0;
-  wgrad_reduce<<<grid_for(nw + nb), 256, 0, s>>>(partial, dW, nw, used, partial + nw * used, db, nb);
-  rc = launch_check("wgrad_reduce");
-  if (rc || !db || fused_bias) return rc;
   // the weight partials have been reduced: their buffer holds the bias
   // partials, one row of cout per block (at most nsplit x 9 x cin rows); a
   // block covers 64 pixels per thread row
@@ -1273,10 +1465,66 @@ int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int
     nbb = (P + bchunk - 1) / bchunk;
   }
   bias_grad_part<<<(unsigned)nbb, 256, 0, s>>>((const bf16*)dz, partial, P, cout, bchunk);
-  rc = launch_check("bias_grad_part");
+  int rc = launch_check("bias_grad_part");
   if (rc) return rc;
   bias_grad_sum<<<(cout + 63) / 64, 256, 0, s>>>(partial, db, (int)nbb, cout);
   return launch_check("bias_grad_sum");
+}
+
+int coffee_unet_wgrad_many(const coffee_unet_wgrad* l, int count, float* partial, long floats,
+                           long* need, void* stream) {
+  if (!l || count < 1 || (!partial && !need))
+    return fail(nullptr, COFFEE_ERR_INVALID, "wgrad_many: bad arguments");
+  std::vector<WgradArgs> a(count);
+  std::vector<float*> dW(count), db(count);
+  long work = 0;
+  for (int k = 0; k < count; k++) {
+    const coffee_unet_wgrad& q = l[k];
+    if (!q.x || !q.dz || !q.dw || !q.db || q.n < 1 || q.h < 1 || q.wd < 1 || q.cin < 16 ||
+        q.cout < 16 || q.cin % 16 || q.cout % 16 || q.cin1 < 16 || q.cin1 % 16 || q.cin1 > q.cin ||
+        (q.cin1 < q.cin && !q.x2) || (q.up && (q.h % 2 || q.wd % 2)) || !aligned16(q.x) ||
+        !aligned16(q.x2) || !aligned16(q.dz) || 9L * q.cout * q.cin > 2147483647L / 2)
+      return fail(nullptr, COFFEE_ERR_INVALID, "wgrad_many: bad arguments of layer " + std::to_string(k));
+    WgradArgs& w = a[k];
+    w = WgradArgs{};
+    w.x = (const bf16*)q.x;
+    w.x2 = (const bf16*)q.x2;
+    w.dz = (const bf16*)q.dz;
+    w.N = q.n;
+    w.H = q.h;
+    w.W = q.wd;
+    w.Cin = q.cin;
+    w.Cout = q.cout;
+    w.c1 = q.cin1;
+    w.up = q.up;
+    if ((w.ntiles = wgrad_tiles(w)) < 0)
+      return fail(nullptr, COFFEE_ERR_SIZE, "wgrad_many: too many tiles");
+    work += (long)w.ntiles * wgrad_blocks(w);
+    dW[k] = q.dw;
+    db[k] = q.db;
+  }
+  // One tile count for every workgroup of every layer, so that three per CU end
+  // together: base 32, 4 levels on 8 x 64 x 128: 59 us and 16 us of sums for the 18
+  // layers, against 346 one layer at a time (two launches each).
+  const long per = std::max<long>(1, (work + 767) / 768);
+  long used = 0;
+  for (int k = 0; k < count; k++) {
+    WgradArgs& w = a[k];
+    const long nw = 9L * w.Cout * w.Cin;
+    wgrad_set_ranges(w, (w.ntiles + per - 1) / per);
+    w.part = partial + used;
+    w.bpart = w.part + w.ranges * nw;
+    used += w.ranges * (nw + w.Cout);
+  }
+  if (need) *need = used;
+  if (!partial) return COFFEE_OK;
+  if (floats < used) return fail(nullptr, COFFEE_ERR_INVALID, "wgrad_many: workspace too small");
+  for (int k = 0; k < count; k += kWgradLayers) {
+    const int rc = launch_wgrad<kWgradLayers>(&a[k], &dW[k], &db[k], std::min(count - k, kWgradLayers),
+                                              (hipStream_t)stream);
+    if (rc) return rc;
+  }
+  return COFFEE_OK;
 }
 
 int coffee_unet_combine(void* out, int ost, int ooff, const void* a, int ast, int aoff,
@@ -1324,20 +1572,31 @@ int coffee_unet_mse(const float* out32, int cst, const float* target, int nc, lo
   if (!out32 || !target || !dout || !loss || nc < 1 || nc > cst)
     return fail(nullptr, COFFEE_ERR_INVALID, "mse: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  const int blocks = 1024;
   double* part = nullptr;
-  if (hipMalloc(&part, sizeof(double) * blocks) != hipSuccess)
+  if (hipMalloc(&part, sizeof(double) * kMseBlocks) != hipSuccess)
     return fail(nullptr, COFFEE_ERR_HIP, "mse: hipMalloc failed");
-  mse_kernel<<<blocks, 256, 0, s>>>(out32, cst, target, nc, npix, (bf16*)dout, part);
+  mse_kernel<<<kMseBlocks, 256, 0, s>>>(out32, cst, target, nc, npix, (bf16*)dout, part);
   hipError_t e = hipGetLastError();
-  double h[1024];
-  if (e == hipSuccess) e = hipMemcpyAsync(h, part, sizeof(double) * blocks, hipMemcpyDeviceToHost, s);
+  double h[kMseBlocks];
+  if (e == hipSuccess) e = hipMemcpyAsync(h, part, sizeof(h), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   (void)hipFree(part);
   if (e != hipSuccess) return fail(nullptr, COFFEE_ERR_HIP, std::string("mse: ") + hipGetErrorString(e));
-  double tot = 0.0;
-  for (int b = 0; b < blocks; b++) tot += h[b];
-  *loss = tot / ((double)npix * nc);
+  *loss = mse_sum(h, npix, nc);
+  return COFFEE_OK;
+}
+
+int coffee_unet_mse_pinned(const float* out32, int cst, const float* target, int nc, long npix,
+                           void* dout, double* work, double* loss, void* stream) {
+  if (!out32 || !target || !dout || !work || !loss || nc < 1 || nc > cst || npix < 1)
+    return fail(nullptr, COFFEE_ERR_INVALID, "mse_pinned: bad arguments");
+  hipStream_t s = (hipStream_t)stream;
+  mse_kernel<<<kMseBlocks, 256, 0, s>>>(out32, cst, target, nc, npix, (bf16*)dout, work);
+  int rc = launch_check("mse_pinned");
+  if (rc) return rc;
+  const hipError_t e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return fail(nullptr, COFFEE_ERR_HIP, std::string("mse_pinned: ") + hipGetErrorString(e));
+  *loss = mse_sum(work, npix, nc);
   return COFFEE_OK;
 }
 
@@ -1353,6 +1612,36 @@ int coffee_unet_adam(float* p, const float* g, float* m, float* v, long n, float
   if (!wbt || 9L * cout * cin != n) return fail(nullptr, COFFEE_ERR_INVALID, "adam: weight shape mismatch");
   weights_bf16_kernel<<<grid_for(n), 256, 0, s>>>(p, (bf16*)wb, (bf16*)wbt, cout, cin);
   return launch_check("weights_bf16");
+}
+
+int coffee_unet_adam_many(const coffee_unet_tensor* l, int count, float lr, float beta1, float beta2,
+                          float eps, int t, void* stream) {
+  if (!l || count < 1 || t < 1) return fail(nullptr, COFFEE_ERR_INVALID, "adam_many: bad arguments");
+  for (int k = 0; k < count; k++)
+    if (!l[k].p || !l[k].g || !l[k].m || !l[k].v || l[k].n < 1 || l[k].n > 1 << 30 ||
+        (l[k].wb && (!l[k].wbt || l[k].cout < 1 || l[k].cin < 1 || 9L * l[k].cout * l[k].cin != l[k].n)))
+      return fail(nullptr, COFFEE_ERR_INVALID, "adam_many: bad arguments of tensor " + std::to_string(k));
+  AdamMany a;
+  a.lr = lr;
+  a.b1 = beta1;
+  a.b2 = beta2;
+  a.eps = eps;
+  a.c1 = 1.f - powf(beta1, (float)t);
+  a.c2 = 1.f - powf(beta2, (float)t);
+  for (int k0 = 0; k0 < count; k0 += kAdamTensors) {
+    a.n = std::min(count - k0, kAdamTensors);
+    a.first[0] = 0;
+    for (int k = 0; k < a.n; k++) {
+      const coffee_unet_tensor& q = l[k0 + k];
+      a.l[k] = {q.p, q.g, q.m, q.v, (bf16*)q.wb, (bf16*)q.wbt, (int)q.n, q.cout, q.cin};
+      a.first[k + 1] = a.first[k] + (q.wb ? 9 * ((q.cout + 31) / 32) * ((q.cin + 31) / 32)
+                                          : (int)((q.n + 1023) / 1024));
+    }
+    adam_many_kernel<<<a.first[a.n], 256, 0, (hipStream_t)stream>>>(a);
+    const int rc = launch_check("adam_many");
+    if (rc) return rc;
+  }
+  return COFFEE_OK;
 }
 
 int coffee_unet_weights_bf16(const float* w32, void* wb, void* wbt, int cout, int cin, void* stream) {

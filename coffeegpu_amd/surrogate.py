@@ -17,6 +17,7 @@ padded to multiples of 16 on the device (padded weights stay zero).
 from __future__ import annotations
 
 import ctypes
+import struct
 from typing import Dict, List, Optional, Tuple
 
 import numpy as np
@@ -58,6 +59,17 @@ def _p(t) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+# coffee_unet_conv, coffee_unet_wgrad and coffee_unet_tensor of include/coffee_unet.h
+_CONV = struct.Struct("10P11i4x")
+_WGRAD = struct.Struct("5P8i")
+_TENSOR = struct.Struct("6Pl2i")
+_OUT, _MASKED, _POOL_BACK, _UP_BACK = range(4)
+
+
+def _a(t) -> int:
+    return t.data_ptr() if t is not None else 0
+
+
 class UNet:
     """U-Net on the device.  Parameters: FP32 masters W[tap][co][ci] (padded),
     biases, Adam moments, BF16 copies W and WT."""
@@ -80,6 +92,9 @@ class UNet:
             self.params[name] = self._alloc_param(w, b, ci, co, relu)
         self.t = 0
         self._bufs: Dict[tuple, object] = {}
+        self._fusable: Dict[tuple, bool] = {}  # by (n, h, w)
+        # partial sums of the loss: written by the device, summed here
+        self._work = _torch().empty(1024, dtype=_torch().float64, pin_memory=True)
 
     # ---- parameters ------------------------------------------------------
     def _alloc_param(self, w: np.ndarray, b: np.ndarray, ci: int, co: int, relu: bool) -> dict:
@@ -156,9 +171,138 @@ class UNet:
             _p(x), _p(P["wb"]), _p(P["b"]), _p(out), _p(out32), n, h, w, P["cip"], P["cop"], 0,
             int(P["relu"] if relu is None else relu), self._s()))
 
+    def _fused(self, x, n: int, h: int, w: int) -> bool:
+        """Whether every convolution of the two passes can take its neighbours
+        (pools, upsamplings, concatenations, masks) into its loads and stores."""
+        if h % (1 << self.levels - 1) or w % (1 << self.levels - 1) or x.data_ptr() % 16:
+            return False
+        ok = self._fusable.get((n, h, w))
+        if ok is None:
+            ok = True
+            for name, _, _, _ in self.specs:
+                P = self.params[name]
+                l = 0 if name == "head" else int(name[3:].rstrip("abup"))
+                up = name.endswith("up")
+                pool = name.startswith("enc") and name.endswith("b") and l < self.levels - 1
+                joins = name.startswith("dec") and name.endswith("a")
+                fits = self._lib.coffee_unet_conv3x3_fusable
+                ok = (ok and fits(n, h >> l, w >> l, P["cip"], P["cop"], int(pool)) == 1
+                      and fits(n, h >> l, w >> l, P["cop"], P["cip"], int(up)) == 1
+                      and (not joins or P["cip"] == 2 * P["cop"]))
+            self._fusable[n, h, w] = ok
+        return ok
+
     def forward(self, x, n: int, h: int, w: int):
         """x: BF16 (int16 storage) NHWC tensor with pad16(cin) channels.
         Returns the FP32 NHWC output (pad16(cout) channels, first cout valid)."""
+        if self._fused(x, n, h, w):
+            return self._forward_fused(x, n, h, w)
+        return self._forward_by_parts(x, n, h, w)
+
+    def _conv_fused(self, s, x, x2, c1, up, P, n, h, w, out=None, out32=None, pool=None, *,
+                    form=_OUT, out2=None, csplit=0, mask=None, skip=None):
+        """forward (form _OUT) or, with the other forms, the backward data pass"""
+        back = form != _OUT or c1 is None
+        ci, co = (P["cop"], P["cip"]) if back else (P["cip"], P["cop"])
+        c = _CONV.pack(_a(x), _a(x2), _a(P["wbt" if back else "wb"]), 0 if back else _a(P["b"]),
+                       _a(out), _a(out2), _a(out32), _a(mask), _a(skip), _a(pool), n, h, w, ci,
+                       c1 or ci, co, csplit or co, int(back), int(P["relu"] and not back), up, form)
+        _lib.check(self._lib.coffee_unet_conv3x3_fused(c, s))
+
+    def _forward_fused(self, x, n, h, w):
+        """One launch per convolution.  The pool of an encoder level is stored by
+        the convolution before it; upsampled and concatenated inputs are read in
+        place.  The tape holds (name, x, x2, cin1, up, y, h, w) per convolution."""
+        torch = _torch()
+        s = self._s()
+        tape = []
+        it = iter(self.specs)
+        skips = []
+
+        def conv(x, hh, ww, x2=None, c1=None, up=0, pool=None):
+            name = next(it)[0]
+            P = self.params[name]
+            y = self._buf(("y", name), n * hh * ww * P["cop"], torch.int16)
+            c1 = c1 or P["cip"]
+            self._conv_fused(s, x, x2, c1, up, P, n, hh, ww, y, pool=pool)
+            tape.append((name, x, x2, c1, up, y, hh, ww))
+            return y, P["cop"]
+
+        cur, hh, ww = x, h, w
+        for l in range(self.levels):
+            if l > 0:
+                cur, hh, ww = pool, hh // 2, ww // 2
+            cur, cc = conv(cur, hh, ww)
+            pool = None
+            if l < self.levels - 1:
+                pool = self._buf(("pool", l + 1), n * (hh // 2) * (ww // 2) * cc, torch.int16)
+            cur, cc = conv(cur, hh, ww, pool=pool)
+            skips.append(cur)
+        for l in range(self.levels - 2, -1, -1):
+            hh, ww = hh * 2, ww * 2
+            cur, cc = conv(cur, hh, ww, up=1)
+            cur, cc = conv(cur, hh, ww, x2=skips[l], c1=cc)
+            cur, cc = conv(cur, hh, ww)
+        name = next(it)[0]
+        P = self.params[name]
+        out32 = self._buf(("out32",), n * hh * ww * P["cop"], torch.float32)
+        self._conv_fused(s, cur, None, P["cip"], 0, P, n, hh, ww, out32=out32)
+        tape.append((name, cur, None, P["cip"], 0, None, hh, ww))
+        self._tape = (tape, n, True)
+        return out32[: n * hh * ww * P["cop"]]
+
+    def _backward_fused(self, dout):
+        """One launch per convolution for the activation gradients, which leave
+        each of them as the dz of the convolution before, then two for all
+        parameter gradients."""
+        torch = _torch()
+        s = self._s()
+        tape, n, _ = self._tape
+        npix = lambda k: n * tape[k][6] * tape[k][7]  # noqa: E731
+        if dout.data_ptr() % 16:
+            dout = self._buf(("dout16",), dout.numel(), torch.int16).copy_(dout.view(torch.int16))
+        dzs = {len(tape) - 1: dout}
+        pos = {t[0]: k for k, t in enumerate(tape)}
+        dskip = {}
+
+        def dz_of(k):
+            dzs[k] = self._buf(("dz", tape[k][0]), npix(k) * self.params[tape[k][0]]["cop"], torch.int16)
+            return dzs[k]
+
+        for k in range(len(tape) - 1, -1, -1):
+            name, _, _, c1, up, _, hh, ww = tape[k]
+            P = self.params[name]
+            kw = {}
+            if k == 0:
+                out = self._buf(("dx", name), npix(k) * P["cip"], torch.int16)
+                self._conv_fused(s, dzs[k], None, None, 0, P, n, hh, ww, out)
+                self.dx = out
+                break
+            mask, out = tape[k - 1][5], dz_of(k - 1)
+            if up:
+                form = _UP_BACK
+            elif name.startswith("enc") and name.endswith("a"):
+                form = _POOL_BACK
+                kw["skip"] = dskip[int(name[3:-1]) - 1]
+            else:
+                form = _MASKED
+                if c1 < P["cip"]:
+                    l = int(name[3:-1])
+                    kw["csplit"] = c1
+                    kw["out2"] = dskip[l] = self._buf(("dskip", l), npix(k) * (P["cip"] - c1), torch.int16)
+            self._conv_fused(s, dzs[k], None, None, 0, P, n, hh, ww, out, form=form, mask=mask, **kw)
+        layers = b"".join(
+            _WGRAD.pack(_a(x), _a(x2), _a(dzs[k]), _a(self.params[name]["gw"]),
+                        _a(self.params[name]["gb"]), n, hh, ww, self.params[name]["cip"], c1,
+                        self.params[name]["cop"], up, 0)
+            for k, (name, x, x2, c1, up, _, hh, ww) in enumerate(tape))
+        need = ctypes.c_long()
+        _lib.check(self._lib.coffee_unet_wgrad_many(layers, len(tape), None, 0, ctypes.byref(need), s))
+        part = self._buf(("part",), need.value, torch.float32)
+        _lib.check(self._lib.coffee_unet_wgrad_many(layers, len(tape), _p(part), part.numel(), None, s))
+        return self.dx
+
+    def _forward_by_parts(self, x, n, h, w):
         torch = _torch()
         L = self.levels
         tape = []
@@ -208,14 +352,16 @@ class UNet:
         out32 = self._buf(("out32",), n * hh * ww * P["cop"], torch.float32)
         self._conv(cur, P, n, hh, ww, None, out32=out32, relu=False)
         tape.append((name, cur, None, hh, ww))
-        self._tape = (tape, n)
+        self._tape = (tape, n, False)
         return out32[: n * hh * ww * P["cop"]]
 
     def backward(self, dout):
         """dout: BF16 gradient of the loss w.r.t. the FP32 output (same layout).
         Fills every parameter's gradient (gw, gb)."""
+        if self._tape[2]:
+            return self._backward_fused(dout)
         torch = _torch()
-        tape, n = self._tape
+        tape, n, _ = self._tape
         pos = [len(tape) - 1]
 
         def conv_back(dz):
@@ -284,17 +430,19 @@ class UNet:
         cop = pad16(self.cout)
         dout = self._buf(("dout",), n * h * w * cop, torch.int16)
         loss = ctypes.c_double()
-        _lib.check(self._lib.coffee_unet_mse(_p(out32), cop, _p(target), self.cout, n * h * w,
-                                             _p(dout), ctypes.byref(loss), self._s()))
+        _lib.check(self._lib.coffee_unet_mse_pinned(_p(out32), cop, _p(target), self.cout,
+                                                    n * h * w, _p(dout), _p(self._work),
+                                                    ctypes.byref(loss), self._s()))
         return loss.value, dout
 
     def adam_step(self, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999,
                   eps: float = 1e-8):
         self.t += 1
-        for P in self.params.values():
-            _lib.check(self._lib.coffee_unet_adam(
-                _p(P["w"]), _p(P["gw"]), _p(P["mw"]), _p(P["vw"]), P["w"].numel(), lr, beta1,
-                beta2, eps, self.t, _p(P["wb"]), _p(P["wbt"]), P["cop"], P["cip"], self._s()))
-            _lib.check(self._lib.coffee_unet_adam(
-                _p(P["b"]), _p(P["gb"]), _p(P["mb"]), _p(P["vb"]), P["b"].numel(), lr, beta1,
-                beta2, eps, self.t, None, None, 0, 0, self._s()))
+        tensors = b"".join(
+            _TENSOR.pack(_a(P["w"]), _a(P["gw"]), _a(P["mw"]), _a(P["vw"]), _a(P["wb"]),
+                         _a(P["wbt"]), P["w"].numel(), P["cop"], P["cip"])
+            + _TENSOR.pack(_a(P["b"]), _a(P["gb"]), _a(P["mb"]), _a(P["vb"]), 0, 0,
+                           P["b"].numel(), 0, 0)
+            for P in self.params.values())
+        _lib.check(self._lib.coffee_unet_adam_many(tensors, 2 * len(self.params), lr, beta1, beta2,
+                                                   eps, self.t, self._s()))

@@ -29,11 +29,51 @@ extern "C" {
 int coffee_unet_conv3x3(const void *in, const void *w, const float *bias, void *out, float *out32,
                         int n, int h, int wd, int cin, int cout, int flip, int relu, void *stream);
 
+/* The same convolution with its neighbours in the network folded into its loads
+ * and stores.  Results are those of the separate calls, roundings included.
+ *   input   channels [0, cin1) from in (stride cin1), the rest from in2 (stride
+ *           cin - cin1): a concatenation; with up, the tensors have h/2 x wd/2
+ *           pixels and are read as their nearest 2x upsampling
+ *   form 0  out and/or out32 as above; pool (may be NULL): BF16 2x2 average of out
+ *   form 1  channels [0, csplit) to out (stride csplit), zeroed where mask (same
+ *           layout, may be NULL) is not positive; the rest to out2 (stride
+ *           cout - csplit)
+ *   form 2  out (2h x 2wd pixels) = adjoint of the 2x2 average + skip (may be
+ *           NULL), zeroed by mask (may be NULL; both in out's layout)
+ *   form 3  out (h/2 x wd/2 pixels) = adjoint of the upsampling, zeroed by mask
+ * Every pointer 16-byte aligned; cin1 and csplit multiples of 16 (cin and cout
+ * without a concatenation or split). */
+typedef struct {
+  const void *in, *in2, *w;
+  const float *bias;
+  void *out, *out2;
+  float *out32;
+  const void *mask, *skip;
+  void *pool;
+  int n, h, wd, cin, cin1, cout, csplit, flip, relu, up, form;
+} coffee_unet_conv;
+int coffee_unet_conv3x3_fused(const coffee_unet_conv *c, void *stream);
+
+/* 1 if coffee_unet_conv3x3_fused takes a convolution of these sizes (pairs: with
+ * pool or form 3), else 0. */
+int coffee_unet_conv3x3_fusable(int n, int h, int wd, int cin, int cout, int pairs);
+
 /* Weight gradient: dW[tap][co][ci] = sum_p dz[p][co] * x[p + (dy,dx)][ci],
  * split over `nsplit` pixel ranges into `partial` (nsplit*9*cout*cin FP32),
  * then reduced into dW (FP32); db[co] = sum_p dz[p][co] (FP32, may be NULL). */
 int coffee_unet_conv3x3_wgrad(const void *x, const void *dz, float *partial, int nsplit, float *dW,
                               float *db, int n, int h, int wd, int cin, int cout, void *stream);
+
+/* Weight and bias gradients of many layers in two launches; x, x2, cin1 and up are
+ * the input as in coffee_unet_conv.  partial holds `floats` FP32 values; with
+ * partial NULL only *need (the number required) is set. */
+typedef struct {
+  const void *x, *x2, *dz;
+  float *dw, *db;
+  int n, h, wd, cin, cin1, cout, up, pad;
+} coffee_unet_wgrad;
+int coffee_unet_wgrad_many(const coffee_unet_wgrad *l, int count, float *partial, long floats,
+                           long *need, void *stream);
 
 /* out[p][ooff+c] = (a[p][aoff+c] + b[p][boff+c]) * (mask[p][moff+c] > 0), c < nc,
  * over p < npix; b and mask may be NULL (then 0 and 1).  *st = channel
@@ -57,12 +97,29 @@ int coffee_unet_up2_bwd(const void *dy, void *dx, int n, int h, int wd, int c, v
 int coffee_unet_mse(const float *out32, int cst, const float *target, int nc, long npix,
                     void *dout, double *loss, void *stream);
 
+/* The same with COFFEE_UNET_MSE_WORK doubles of pinned host memory as workspace. */
+#define COFFEE_UNET_MSE_WORK 1024
+int coffee_unet_mse_pinned(const float *out32, int cst, const float *target, int nc, long npix,
+                           void *dout, double *work, double *loss, void *stream);
+
 /* Adam step on one tensor of n FP32 parameters (t = step number, 1-based);
  * when wb is given the tensor is a 3x3 weight [9][cout][cin] and its BF16
  * copies W and WT are refreshed. */
 int coffee_unet_adam(float *p, const float *g, float *m, float *v, long n, float lr, float beta1,
                      float beta2, float eps, int t, void *wb, void *wbt, int cout, int cin,
                      void *stream);
+
+/* The same step on many tensors in one launch. */
+typedef struct {
+  float *p;
+  const float *g;
+  float *m, *v;
+  void *wb, *wbt;
+  long n;
+  int cout, cin;
+} coffee_unet_tensor;
+int coffee_unet_adam_many(const coffee_unet_tensor *l, int count, float lr, float beta1, float beta2,
+                          float eps, int t, void *stream);
 
 /* FP32 -> BF16 weight copies W[tap][co][ci] and WT[tap][ci][co]. */
 int coffee_unet_weights_bf16(const float *w32, void *wb, void *wbt, int cout, int cin,
