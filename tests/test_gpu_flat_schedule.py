@@ -1,5 +1,5 @@
-"""The schedule the flat solver picks by grid size (thread-per-cell, 64 x 8 or
-128 x 8 tiles, one or several z chunks) against forced ones: bitwise the same
+"""The schedule the flat solver picks by grid size (thread-per-cell, 64 x 4, 64 x 8
+or 128 x 8 tiles, one or several z chunks, tiles not in eights) against forced ones: bitwise the same
 state, guards included.  Sizes on both sides of each line of the rule, with
 remainders in every axis."""
 
@@ -19,7 +19,8 @@ from coffeegpu_amd.solver import FieldSolverEZ, SimData, SimEnvironment  # noqa:
 
 @pytest.mark.parametrize("n", [(50, 51, 50), (52, 51, 50), (66, 67, 68), (67, 67, 68), (81, 83, 81),
                                (82, 83, 81), (127, 40, 70), (129, 190, 33), (256, 130, 9),
-                               (192, 160, 64)])
+                               (192, 160, 64), (75, 77, 78), (92, 93, 94), (127, 126, 126),
+                               (136, 136, 136)])
 @pytest.mark.parametrize("problem", [0, 1])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_picked_schedule_is_bitwise_the_same(n, problem, dtype):
