@@ -821,6 +821,13 @@ __global__ void __launch_bounds__(TX) __attribute__((amdgpu_waves_per_eu(TX >= 5
   sph_advance(runs, clocks, next, nruns);
 }
 
+// cos(theta_j) as the cells would evaluate it (the host's may round differently).
+template <typename T>
+__global__ void __launch_bounds__(256) sph_cos_table(T* __restrict__ cth, T y0, T dy, int g1, int n) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < n) cth[j] = cos(y0 + dy * T(j - g1));
+}
+
 // theta-axis boundary (kernel_boundary_axis_sph, .cu:690-748) on buffer `buf`
 // of every active run, after a launch of the march kernels (the others store
 // the copies themselves): one thread per interior radial index.
