@@ -583,31 +583,39 @@ __device__ __forceinline__ s4 lds_read_tr(const bf16* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
 }
 
-constexpr int kWgradLds = 128 * 32 + 180 * 40;  // tiles of 8 x 16 pixels, 32 x 32 channels
+template <int CIB, int COB, bool LIN>
+constexpr int wgrad_lds() {  // bf16 values of its tiles
+  return 128 * COB + (LIN ? 391 : 180) * (CIB + 8);
+}
 
-// 16-byte chunk swizzle of the dz tile of wgrad_tr (pixel rows of C8 chunks):
-// chunk c of pixel k lives at c ^ wswz(k).  With 32 channels (4 chunks, 64 bytes)
-// it puts the 32 lanes of every transposing read (pixel rows 8 g + 4 h + r of a
+// 16-byte chunk swizzle of the dz tile of wgrad_block (pixel rows of C8 chunks):
+// chunk c of pixel k lives at c ^ wswz(k).  With 32 or 64 channels it puts the 32 lanes of every transposing read (pixel rows 8 g + 4 h + r of a
 // 32-pixel step) on distinct banks with no padding; the bits it uses (1 and 3) come
 // only from the lane's own part of the pixel index.
 template <int C8>
 __device__ __forceinline__ int wswz(int k) {
-  return C8 == 4 ? (k & 2) | ((k >> 3) & 1) : 0;
+  return C8 == 8 ? (k & 2) | ((k >> 1) & 4) : C8 == 4 ? (k & 2) | ((k >> 3) & 1) : 0;
 }
+
+// Order of the pixels of a weight gradient (part of its FP32 result): tiles of 8 x
+// 16 or 4 x 16 pixels, or the pixels as they lie in memory.
+enum WgradOrder { kTile8, kTile4, kLinear };
 
 struct WgradArgs {
   const bf16* x;
   const bf16* dz;
   float* part;
-  float* bpart;  // per-range sums of dz per output channel, or null
+  float* bpart;    // bias partials, or null
   const bf16* x2;  // input forms, as ConvArgs
   int N, H, W, Cin, Cout, c1, up;
-  int tiles_per_range, ntiles, ranges;
+  int order, ranges, per, ntiles;  // per: tiles (kLinear: pixels) per range
+  int bblocks, bchunk;             // kept apart from the ranges: bias_part
+  int split;                       // kLinear: workgroups that share out the taps (1 or 3)
 };
 
 // Layers of one launch (at most MAX: a single layer has no table to send and search,
 // 1 us of its two launches), with the first workgroup of each (first[n] = total).
-constexpr int kWgradLayers = 32;
+constexpr int kWgradLayers = 20;
 template <int MAX>
 struct WgradMany {
   int n, first[MAX + 1];
@@ -621,64 +629,90 @@ __device__ __forceinline__ int entry_of(const int* first, int n, int b) {
   return k;
 }
 
-// Weight gradient with spatial tiles in LDS: a workgroup computes the 9 x COB
+// v / d for 0 <= v < d + 130, mul = 2^20 / d + 1 (exact for d < 256; from there on v /
+// d is 0 or 1).
+__device__ __forceinline__ int small_div(int v, int d, int mul) {
+  return d < 256 ? (int)((unsigned)v * (unsigned)mul >> 20) : (int)(v >= d);
+}
+
+// Weight gradient with the pixels staged in LDS: a workgroup computes the 9 x COB
 // (co) x CIB (ci) block of dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] over a
-// range of tiles of TR image rows x 16 columns (GEMM with K = pixels).  dz (TR x 16
-// pixels x COB) and the input with its one-pixel halo are staged in LDS as they
-// lie in memory (pixel rows, channels contiguous; 16-byte stores), and both MFMA
-// operands are read with the transposing LDS read, so a tap's shift is only
-// another row address (a constant offset from the lane's base) and every staged
-// value serves all nine taps.  Input rows are padded by 8 values.
+// range of pixels (GEMM with K = pixels), TP at a time.  dz (TP pixels x COB) and
+// the input with its one-pixel halo lie in LDS as in memory (pixel rows, channels
+// contiguous; 16-byte stores), and both MFMA operands are read with the transposing
+// LDS read, so a tap's shift is only another row address and every staged value
+// serves all nine taps.  Input rows are padded by 8 values.  The next tile's global
+// loads are in flight during the current tile's MFMAs.
 //
-// A wavefront owns 16 input channels (CIB / 16 wavefronts side by side) against
-// all COB output channels: per 32-pixel step it reads COB / 16 A fragments (shared
-// by the taps) and 9 B fragments for 9 COB / 16 MFMAs (v_mfma_f32_16x16x32_bf16).
-// The four wavefronts are 2 (CIB = 32) or 4 (16) groups that take the steps of a
-// tile in turn, and their sums are added in group order through LDS at the end.  The next tile's global loads are in flight
-// during the current tile's MFMAs.  Pixels beyond the image are zero.  Partial
-// blocks per range go to part[range][tap][co][ci] (summed in range order by
-// wgrad_reduce); when bpart is given, the workgroups of the first input-channel
-// block also sum dz over their range, per output channel in a fixed order, into
-// bpart[range][co].
-template <int TR, int CIB, int COB>
-__device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int block, bf16* lds) {
-  constexpr int TW = 16, TP = TR * TW, XW = TW + 2, XP = (TR + 2) * XW, XS = CIB + 8;
-  constexpr int D8 = COB / 8, X8 = CIB / 8;          // 16-byte chunks per pixel
-  constexpr int NDZ = (TP * D8 + 255) / 256;         // 16-byte dz loads per thread
-  constexpr int NX = (XP * X8 + 255) / 256;          // 16-byte input loads per thread
-  constexpr int WC = CIB / 16, KS = 4 / WC;          // wavefronts along ci, step groups
-  constexpr int MC = COB / 16, STEPS = TP / 32;
-  constexpr int RED = KS > 1 ? 4 * 64 * MC * 4 * 2 : 0;  // one tap's sums, in bf16 units
-  constexpr int LDS_E = TP * COB + XP * XS;
-  static_assert(TP % 32 == 0 && STEPS % KS == 0, "whole 32-pixel steps per tile and group");
-  static_assert(RED <= LDS_E && 256 * 8 * 2 <= LDS_E, "reductions fit in the tiles");
-  static_assert(LDS_E <= kWgradLds, "shared memory of wgrad_tr");
+// The pixels are summed in the order `order` names, 32 per instruction
+// (v_mfma_f32_16x16x32_bf16) and one chain per range, so that a training step gives
+// the same gradients whatever the block shape: a sum in another order moves a BF16
+// weight of the next step now and then, and with it every activation.
+//   TR rows x 16 columns: the halo tile is (TR + 2) x 18 pixels.
+//   kLinear: TP consecutive pixels; three strips of them, a row of the image above
+//   and below (zero outside the image); where a tap leaves the row, or the pixel
+//   the range, the lane reads a row of zeros instead.
+// A wavefront owns 16 input channels against all COB output channels: with CIB = 64
+// for all nine taps; with 32 or 16, 2 or 4 wavefronts share them out.  With DY (kLinear)
+// a workgroup takes the three taps of row dy, one strip, and the wavefronts share
+// out the output channels.  FORMS: x2 and up are looked at.  Pixels beyond
+// the image are zero.  Partial blocks go to part[range][tap][co][ci] (summed in
+// range order by wgrad_reduce); in the tile orders with bpart given, the workgroups
+// of the first input-channel block also sum dz over their range, per output channel
+// in a fixed order, into bpart[range][co].
+template <int CIB, int COB, int ORDER, bool FORMS, bool DY = false>
+__device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int block, bf16* lds,
+                                            int row0 = 0) {
+  constexpr bool LIN = ORDER == kLinear;
+  constexpr int TR = ORDER == kTile4 ? 4 : 8, TW = 16, TP = TR * TW;
+  constexpr int XW = LIN ? TP + 2 : TW + 2, XP = (DY ? 1 : LIN ? 3 : TR + 2) * XW, XS = CIB + 8;
+  constexpr int D8 = COB / 8, X8 = CIB / 8;       // 16-byte chunks per pixel
+  constexpr int NDZ = (TP * D8 + 255) / 256;      // 16-byte dz loads per thread
+  constexpr int NX = (XP * X8 + 255) / 256;       // 16-byte input loads per thread
+  constexpr int WC = CIB / 16, TG = 4 / WC;       // wavefronts along ci, groups of taps
+  constexpr int MC = DY ? 1 : COB / 16, NT = DY ? 3 : (9 + TG - 1) / TG;
   bf16* const dzs = lds;
   bf16* const xs = lds + TP * COB;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int wc = wave % WC, ks = wave / WC;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const int wc = wave % WC, tg = wave / WC, m0 = DY ? tg : 0;  // m0: first 16 of COB
+  const bool works = m0 < COB / 16;
   const int li = lane & 15, lk = lane >> 4;
   const int g = lane >> 4, r = (lane >> 2) & 3, q = lane & 3;
   const int ncib = a.Cin / CIB;
   const int co0 = (block / ncib) * COB, ci0 = (block % ncib) * CIB;
-  const bool do_bias = a.bpart && block % ncib == 0;
+  const bool do_bias = !LIN && a.bpart && !a.bblocks && block % ncib == 0;
   const int H = a.H, W = a.W, Cin = a.Cin, Cout = a.Cout;
-  const int tiles_x = (W + TW - 1) / TW, tiles_y = (H + TR - 1) / TR;
-  const int t_begin = range * a.tiles_per_range;
-  const int t_end = min(t_begin + a.tiles_per_range, a.ntiles);
+  const int tiles_x = LIN ? 1 : W / TW, tiles_y = (H + TR - 1) / TR;
+  // kLinear: pixels, at most 2^31 - 1
+  const int begin = range * a.per;
+  const int end = (int)min((long)begin + a.per, (long)a.ntiles), stride = LIN ? TP : 1;
+  const int mulW = (1 << 20) / W + 1, mulH = (1 << 20) / H + 1;
 
   s8 rdz[NDZ], rx[NX];
+  int col0 = 0;  // column of the first pixel of the tile being loaded (kLinear)
   auto load_tile = [&](int tile) __attribute__((always_inline)) {
-    const int img = tile / (tiles_x * tiles_y);
-    const int rest = tile - img * tiles_x * tiles_y;
-    const int y0 = (rest / tiles_x) * TR, x0 = (rest % tiles_x) * TW;
+    // first pixel (kLinear) or corner of the tile
+    int img, y0, x0;
+    if constexpr (LIN) {
+      const unsigned row = (unsigned)tile / (unsigned)W;
+      col0 = x0 = (int)((unsigned)tile - row * W);
+      img = (int)(row / (unsigned)H);
+      y0 = (int)row - img * H;
+    } else {
+      img = tile / (tiles_x * tiles_y);
+      const int rest = tile - img * tiles_x * tiles_y;
+      y0 = (rest / tiles_x) * TR;
+      x0 = (rest % tiles_x) * TW;
+    }
 #pragma unroll
     for (int u = 0; u < NDZ; u++) {
       const int idx = t + 256 * u, px = idx / D8, c8 = idx % D8;
       const int yy = y0 + px / TW, xx = x0 + px % TW;
+      const bool in = LIN ? px < end - tile : yy < H;
+      const long p = LIN ? (long)tile + px : (long)(img * H + yy) * W + xx;
       rdz[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
-      if ((TP * D8 % 256 == 0 || idx < TP * D8) && yy < H && xx < W)
-        rdz[u] = *(const s8*)(a.dz + ((long)(img * H + yy) * W + xx) * Cout + co0 + 8 * c8);
+      if ((TP * D8 % 256 == 0 || idx < TP * D8) && in)
+        rdz[u] = *(const s8*)(a.dz + p * Cout + co0 + 8 * c8);
     }
 #pragma unroll
     for (int u = 0; u < NX; u++) {
@@ -686,12 +720,27 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int b
       rx[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
       if (idx < XP * X8) {
         const int pix = idx / X8, c = ci0 + 8 * (idx % X8);
-        const int yy = y0 - 1 + pix / XW, xx = x0 - 1 + pix % XW;
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
-          const long p = a.up ? (long)(img * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)
-                              : (long)(img * H + yy) * W + xx;
-          if (c >= a.c1) rx[u] = *(const s8*)(a.x2 + p * (Cin - a.c1) + c - a.c1);
-          else rx[u] = *(const s8*)(a.x + p * a.c1 + c);
+        int yy, xx, im = img;
+        bool in;
+        if constexpr (LIN) {
+          // pixel tile - 1 + pix % XW of the strip, a row up or down; the one
+          // before column 0 serves no tap
+          const int v = x0 + pix % XW - 1, down = small_div(max(v, 0), W, mulW);
+          const int rr = y0 + down, next = small_div(rr, H, mulH);
+          im += next;
+          yy = rr - next * H + pix / XW + row0 - 1;
+          xx = v - down * W;
+          in = v >= 0 && im < a.N && yy >= 0 && yy < H;
+        } else {
+          yy = y0 - 1 + pix / XW;
+          xx = x0 - 1 + pix % XW;
+          in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+        }
+        if (in) {
+          const long p = FORMS && a.up ? (long)(im * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)
+                                       : (long)(im * H + yy) * W + xx;
+          if (FORMS && c >= a.c1) rx[u] = *(const s8*)(a.x2 + p * (Cin - a.c1) + c - a.c1);
+          else rx[u] = *(const s8*)(a.x + p * (FORMS ? a.c1 : Cin) + c);
         }
       }
     }
@@ -709,22 +758,282 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int b
       if (idx < XP * X8) *(s8*)&xs[(idx / X8) * XS + 8 * (idx % X8)] = rx[u];
     }
   };
-  // A: K index 8 g + 4 h + r of step st is pixel 32 st + 16 (g / 2) + 8 (g % 2)
-  // + 4 h + r; the lane's part ka fixes the swizzle, st and h add whole rows.
-  const int ka = 16 * (g >> 1) + 8 * (g & 1) + r;
-  const bf16* abase[MC];
+  // A: K index 8 g + 4 h + r of step st is pixel 32 st + 8 g + 4 h + r; the lane's
+  // part ka fixes the swizzle, st and h add whole rows.
+  const int ka = 8 * g + r;
+  int abase[MC];  // offsets in dzs, as xbase and zero in xs
 #pragma unroll
   for (int m = 0; m < MC; m++)
-    abase[m] = &dzs[ka * COB + 8 * ((2 * m + (q >> 1)) ^ wswz<D8>(ka)) + 4 * (q & 1)];
+    abase[m] = (ka * COB + 8 * ((2 * (works ? m0 + m : 0) + (q >> 1)) ^ wswz<D8>(ka)) + 4 * (q & 1));
+  // B: the same pixel, in the middle of the haloed input
+  const int xchunk = 8 * (2 * wc + (q >> 1)) + 4 * (q & 1);
+  const int xbase = xchunk + (LIN ? (DY ? 0 : XW) + ka + 1
+                                  : ((g >> 1) + 1) * XW + 8 * (g & 1) + r + 1) * XS;
+  const int zero = XP * XS + xchunk;
+  if (LIN && t < CIB) xs[XP * XS + t] = 0;
+
+  f4 acc[NT][MC];
+#pragma unroll
+  for (int k = 0; k < NT; k++)
+#pragma unroll
+    for (int m = 0; m < MC; m++) acc[k][m] = f4{0.f, 0.f, 0.f, 0.f};
+  float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (begin < end) load_tile(begin);
+  for (int tile = begin; tile < end; tile += stride) {
+    const int left = LIN ? end - tile : TP;  // pixels of the tile in the range
+    const int colt = col0;
+    __syncthreads();  // every wavefront is done with the previous tile
+    store_tile();
+    __syncthreads();
+    if (LIN ? left > TP : tile + 1 < end) load_tile(tile + stride);
+    if (do_bias && t < 32 * D8) {
+      // thread (pixel group t / D8, chunk t % D8): pixels t / D8, t / D8 + 32, ...
+#pragma unroll
+      for (int i = 0; i < TP / 32; i++) {
+        const int px = t / D8 + 32 * i, c8 = t % D8;
+        const s8 v = *(const s8*)&dzs[px * COB + 8 * (c8 ^ wswz<D8>(px))];
+#pragma unroll
+        for (int e = 0; e < 8; e++) bsum[e] += bf2f((bf16)v[e]);
+      }
+    }
+#pragma unroll 1
+    for (int st = 0; st < TP / 32 && 32 * st < left && works; st++) {
+      bf8 af[MC];
+#pragma unroll
+      for (int m = 0; m < MC; m++) {
+        const s4 lo = lds_read_tr(dzs + abase[m] + (32 * st) * COB);
+        const s4 hi = lds_read_tr(dzs + abase[m] + (32 * st + 4) * COB);
+        af[m] = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+      }
+      // whether the lane's two pixels in the step have a neighbour to the left and
+      // right
+      const int row = (LIN ? 32 * st : 2 * st * XW) * XS;
+      bool mid[2], lft[2], rgt[2];
+      if constexpr (LIN) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int k = 32 * st + ka + 4 * h, v = colt + k, col = v - small_div(v, W, mulW) * W;
+          mid[h] = k < left;
+          lft[h] = mid[h] && col > 0;
+          rgt[h] = mid[h] && col < W - 1;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NT; i++) {
+        const int tap = DY ? i : tg + TG * i;
+        if (!DY && TG > 1 && tap >= 9) continue;
+        const int dy = DY ? 0 : tap / 3 - 1, dx = tap % 3 - 1, off = (dy * XW + dx) * XS;
+        auto from = [&](int h) {
+          const int at = xbase + (row + off) + 4 * h * XS;
+          if constexpr (!LIN) return at;
+          const bool ok = dx == 0 ? mid[h] : (dx < 0 ? lft[h] : rgt[h]);
+          return ok ? at : zero;
+        };
+        const s4 lo = lds_read_tr(xs + from(0)), hi = lds_read_tr(xs + from(1));
+        const bf8 bfr = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+#pragma unroll
+        for (int m = 0; m < MC; m++)
+          acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[m], bfr, acc[i][m], 0, 0, 0);
+      }
+    }
+  }
+  // D[i = co][j = ci]: lane holds co = co0 + 16 m + 4 lk + v, ci = ci0 + 16 wc + li
+  const int ci = ci0 + wc * 16 + li;
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    const int tap = DY ? 3 * row0 + i : tg + TG * i;
+    if (tap >= 9 || !works) continue;
+    float* dst = a.part + ((long)range * 9 + tap) * Cout * Cin;
+#pragma unroll
+    for (int m = 0; m < MC; m++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) dst[(long)(co0 + (m0 + m) * 16 + 4 * lk + v) * Cin + ci] = acc[i][m][v];
+  }
+  if (do_bias) {
+    // the 32 pixel groups' sums of each channel, added in group order
+    __syncthreads();  // every wavefront is done with the last tile
+    float* red = (float*)lds;
+    if (t < 32 * D8)
+#pragma unroll
+      for (int e = 0; e < 8; e++) red[(t / D8) * COB + 8 * (t % D8) + e] = bsum[e];
+    __syncthreads();
+    if (t < COB) {
+      float b = 0.f;
+      for (int k = 0; k < 32; k++) b += red[k * COB + t];
+      a.bpart[(long)range * Cout + co0 + t] = b;
+    }
+  }
+}
+
+// Bias gradient db[c] = sum_p dz[p][c] in two deterministic passes, for the orders
+// that do not sum it with the weights.  Pass 1: block b sums the pixels [b chunk, (b
+// + 1) chunk) of every channel, threads laid out channel-fastest so that a pixel's
+// channels are one coalesced row (channel groups of up to 256; 256 / group pixel
+// rows in parallel, summed in a fixed order).  Pass 2 adds the block partials in
+// block order.
+__device__ __forceinline__ void bias_part(const bf16* __restrict__ dz, float* __restrict__ part,
+                                          long P, int C, long chunk, int b, float* red) {
+  const long p0 = b * chunk;
+  const long p1 = p0 + chunk < P ? p0 + chunk : P;
+  for (int cb = 0; cb < C; cb += 256) {
+    const int cw = C - cb < 256 ? C - cb : 256;
+    const int rows = 256 / cw;
+    const int c = (int)threadIdx.x % cw, r = (int)threadIdx.x / cw;
+    float s = 0.f;
+    if (r < rows)
+      for (long p = p0 + r; p < p1; p += rows) s += bf2f(dz[p * C + cb + c]);
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if ((int)threadIdx.x < cw) {
+      float t = 0.f;
+      for (int k = 0; k < rows; k++) t += red[k * cw + threadIdx.x];
+      part[(long)b * C + cb + threadIdx.x] = t;
+    }
+    __syncthreads();
+  }
+}
+
+// Workgroups of a layer in the launch of its order: its bias_part
+// blocks, then ranges x channel blocks.
+template <int MAX, int ORDER>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    wgrad_tiles(const WgradMany<MAX> m) {
+  __shared__ __attribute__((aligned(16))) bf16 lds[wgrad_lds<64, 32, false>()];
+  const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
+  const WgradArgs a = m.l[k];
+  const int b = blockIdx.x - m.first[k] - a.bblocks;
+  if (b < 0) {
+    bias_part(a.dz, a.bpart, (long)a.N * a.H * a.W, a.Cout, a.bchunk, b + a.bblocks, (float*)lds);
+    return;
+  }
+  const int range = b % a.ranges, block = b / a.ranges;
+  wgrad_block<64, 32, ORDER, true>(a, range, block, lds);
+}
+
+template <int MAX>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    wgrad_linear(const WgradMany<MAX> m) {
+  __shared__ __attribute__((aligned(16))) bf16 lds[wgrad_lds<32, 32, true>()];
+  const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
+  const WgradArgs a = m.l[k];
+  const int b = blockIdx.x - m.first[k] - a.bblocks;
+  if (b < 0) {
+    bias_part(a.dz, a.bpart, (long)a.N * a.H * a.W, a.Cout, a.bchunk, b + a.bblocks, (float*)lds);
+    return;
+  }
+  const int range = b % a.ranges, block = b / a.ranges;
+  constexpr bool F = MAX > 1;
+  if (MAX == 1 && a.split == 3) {
+    if (a.Cin % 32 == 0) {
+      if (a.Cout % 32 == 0) wgrad_block<32, 32, kLinear, F, true>(a, range, block / 3, lds, block % 3);
+      else wgrad_block<32, 16, kLinear, F, true>(a, range, block / 3, lds, block % 3);
+    } else {
+      if (a.Cout % 32 == 0) wgrad_block<16, 32, kLinear, F, true>(a, range, block / 3, lds, block % 3);
+      else wgrad_block<16, 16, kLinear, F, true>(a, range, block / 3, lds, block % 3);
+    }
+  } else if (a.Cin % 32 == 0) {
+    if (a.Cout % 32 == 0) wgrad_block<32, 32, kLinear, F>(a, range, block, lds);
+    else wgrad_block<32, 16, kLinear, F>(a, range, block, lds);
+  } else {
+    if (a.Cout % 32 == 0) wgrad_block<16, 32, kLinear, F>(a, range, block, lds);
+    else wgrad_block<16, 16, kLinear, F>(a, range, block, lds);
+  }
+}
+
+// One layer in a tile order, blocks of 64 x 64 channels (wgrad_block's chains, bit for
+// bit; from it they spill 17 registers, and with 64 x 32 blocks 1.6 times the bytes are
+// staged: 16 x 64 x 128, 128 -> 64 45 -> 62 and 72 us), for Cin % 64 == 0, Cout % 64 == 0
+// and W % 16 == 0: a workgroup computes the 9 x 64 (co) x 64 (ci) block of
+// dW[tap][co][ci] = sum_p dz[p][co] x[p + tap][ci] over a range of tiles of
+// TR image rows x 16 columns.  dz (TR x 16 pixels x 64 co) and the input
+// with its one-pixel halo are staged in LDS as they lie in memory (pixel
+// rows, channels contiguous; 16-byte stores), and both MFMA operands are read
+// with the transposing LDS read, so a tap's shift is only another row
+// address (a constant offset from the lane's base) and every staged value
+// serves all nine taps.  Input rows are padded to XS = 72 values.  Wavefront
+// w owns input channels ci0 + 16 w .. + 15 against the 64 output channels:
+// per 32-pixel step it reads 4 A fragments (shared by the taps) and 9 B
+// fragments for 36 MFMAs (v_mfma_f32_16x16x32_bf16).  The next tile's
+// global loads are in flight during the current tile's MFMAs.  Pixels beyond
+// the image are zero.  Partial blocks per range go to
+// part[range][tap][co][ci] (summed by wgrad_reduce in range order); when
+// bpart is given, the workgroups of the first input-channel block also sum dz
+// over their range, per output channel in a fixed order, into
+// bpart[range][co].
+template <int TR>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    wgrad_tr(const bf16* __restrict__ x, const bf16* __restrict__ dz, float* __restrict__ part,
+             float* __restrict__ bpart, int N, int H, int W, int Cin, int Cout,
+             int tiles_per_range, int ntiles) {
+  constexpr int TW = 16, TP = TR * TW, XW = TW + 2, XP = (TR + 2) * XW, XS = 72;
+  constexpr int NDZ = TP * 8 / 256;            // 16-byte dz loads per thread
+  constexpr int NX = (XP * 8 + 255) / 256;     // 16-byte input loads per thread
+  static_assert(TP % 32 == 0, "whole 32-pixel steps per tile");
+  static_assert(32 * 64 <= XP * XS, "bias reduction fits in the input tile");
+  __shared__ __attribute__((aligned(16))) bf16 dzs[TP * 64];
+  __shared__ __attribute__((aligned(16))) bf16 xs[XP * XS];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int g = lane >> 4, r = (lane >> 2) & 3, q = lane & 3;
+  const int range = blockIdx.x;
+  const int ncib = Cin / 64;
+  const int co0 = (blockIdx.y / ncib) * 64, ci0 = (blockIdx.y % ncib) * 64;
+  const bool do_bias = bpart && blockIdx.y % ncib == 0;
+  const int tiles_x = W / TW, tiles_y = (H + TR - 1) / TR;
+  const int t_begin = range * tiles_per_range;
+  const int t_end = min(t_begin + tiles_per_range, ntiles);
+
+  s8 rdz[NDZ], rx[NX];
+  auto load_tile = [&](int tile) __attribute__((always_inline)) {
+    const int img = tile / (tiles_x * tiles_y);
+    const int rest = tile - img * tiles_x * tiles_y;
+    const int y0 = (rest / tiles_x) * TR, x0 = (rest % tiles_x) * TW;
+#pragma unroll
+    for (int u = 0; u < NDZ; u++) {
+      const int idx = t + 256 * u, px = idx >> 3, c8 = idx & 7;
+      const int yy = y0 + px / TW, xx = x0 + px % TW;
+      rdz[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (yy < H) rdz[u] = *(const s8*)(dz + ((long)(img * H + yy) * W + xx) * Cout + co0 + 8 * c8);
+    }
+#pragma unroll
+    for (int u = 0; u < NX; u++) {
+      const int idx = t + 256 * u;
+      rx[u] = s8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (idx < XP * 8) {
+        const int pix = idx >> 3, c8 = idx & 7;
+        const int yy = y0 - 1 + pix / XW, xx = x0 - 1 + pix % XW;
+        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
+          rx[u] = *(const s8*)(x + ((long)(img * H + yy) * W + xx) * Cin + ci0 + 8 * c8);
+      }
+    }
+  };
+  auto store_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NDZ; u++) {
+      const int idx = t + 256 * u, px = idx >> 3, c8 = idx & 7;
+      *(s8*)&dzs[px * 64 + 8 * (c8 ^ wswz<8>(px))] = rdz[u];
+    }
+#pragma unroll
+    for (int u = 0; u < NX; u++) {
+      const int idx = t + 256 * u;
+      if (idx < XP * 8) *(s8*)&xs[(idx >> 3) * XS + 8 * (idx & 7)] = rx[u];
+    }
+  };
+  // A: K index 8 g + 4 h + r of step st is pixel 32 st + 16 (g / 2) + 8 (g % 2)
+  // + 4 h + r; the lane's part ka fixes the swizzle, st and h add 64-value rows.
+  const int ka = 16 * (g >> 1) + 8 * (g & 1) + r;
+  const bf16* abase[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) abase[m] = &dzs[ka * 64 + 8 * ((2 * m + (q >> 1)) ^ wswz<8>(ka)) + 4 * (q & 1)];
   // B: the same pixel shifted by the tap, in the haloed input tile
-  const bf16* xbase = &xs[(((g >> 1) + 1) * XW + 8 * (g & 1) + r + 1) * XS + 8 * (2 * wc + (q >> 1)) +
+  const bf16* xbase = &xs[(((g >> 1) + 1) * XW + 8 * (g & 1) + r + 1) * XS + 8 * (2 * wave + (q >> 1)) +
                           4 * (q & 1)];
 
-  f4 acc[9][MC];
+  f4 acc[9][4];
 #pragma unroll
   for (int k = 0; k < 9; k++)
 #pragma unroll
-    for (int m = 0; m < MC; m++) acc[k][m] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < 4; m++) acc[k][m] = f4{0.f, 0.f, 0.f, 0.f};
   float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (t_begin < t_end) load_tile(t_begin);
   for (int tile = t_begin; tile < t_end; tile++) {
@@ -733,24 +1042,22 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int b
     __syncthreads();
     if (tile + 1 < t_end) load_tile(tile + 1);
     if (do_bias) {
-      // thread (pixel group t / D8, chunk t % D8): pixels t / D8, + 256 / D8, ...
+      // thread (pixel group t / 8, chunk t % 8): pixels t / 8, t / 8 + 32, ...
 #pragma unroll
-      for (int i = 0; i < (TP * D8 + 255) / 256; i++) {
-        const int px = t / D8 + 256 / D8 * i, c8 = t % D8;
-        if (TP * D8 % 256 == 0 || px < TP) {
-          const s8 v = *(const s8*)&dzs[px * COB + 8 * (c8 ^ wswz<D8>(px))];
+      for (int i = 0; i < TP / 32; i++) {
+        const int px = (t >> 3) + 32 * i, c8 = t & 7;
+        const s8 v = *(const s8*)&dzs[px * 64 + 8 * (c8 ^ wswz<8>(px))];
 #pragma unroll
-          for (int e = 0; e < 8; e++) bsum[e] += bf2f((bf16)v[e]);
-        }
+        for (int e = 0; e < 8; e++) bsum[e] += bf2f((bf16)v[e]);
       }
     }
 #pragma unroll 1
-    for (int st = ks; st < STEPS; st += KS) {
-      bf8 af[MC];
+    for (int st = 0; st < TP / 32; st++) {
+      bf8 af[4];
 #pragma unroll
-      for (int m = 0; m < MC; m++) {
-        const s4 lo = lds_read_tr(abase[m] + (32 * st) * COB);
-        const s4 hi = lds_read_tr(abase[m] + (32 * st + 4) * COB);
+      for (int m = 0; m < 4; m++) {
+        const s4 lo = lds_read_tr(abase[m] + (32 * st) * 64);
+        const s4 hi = lds_read_tr(abase[m] + (32 * st + 4) * 64);
         af[m] = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
       }
 #pragma unroll
@@ -761,63 +1068,33 @@ __device__ __forceinline__ void wgrad_block(const WgradArgs& a, int range, int b
         const s4 hi = lds_read_tr(xbase + off + 4 * XS);
         const bf8 bfr = __builtin_bit_cast(bf8, s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
 #pragma unroll
-        for (int m = 0; m < MC; m++)
+        for (int m = 0; m < 4; m++)
           acc[tap][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[m], bfr, acc[tap][m], 0, 0, 0);
       }
     }
   }
-  // D[i = co][j = ci]: lane holds co = co0 + 16 m + 4 lk + v, ci = ci0 + 16 wc + li
-  const int ci = ci0 + wc * 16 + li;
+  // D[i = co][j = ci]: lane holds co = co0 + 16 m + 4 lk + v, ci = ci0 + 16 wave + li
+  const int ci = ci0 + wave * 16 + li;
 #pragma unroll
   for (int k = 0; k < 9; k++) {
-    if constexpr (KS > 1) {  // groups 1.. hand their sums of this tap to group 0
-      f4* red = (f4*)lds;    // [m][wavefront][lane]
-      __syncthreads();       // the tiles, or the previous tap, are done with
+    float* dst = part + ((long)range * 9 + k) * Cout * Cin;
 #pragma unroll
-      for (int m = 0; m < MC; m++)
-        if (ks) red[(m * 4 + wave) * 64 + lane] = acc[k][m];
-      __syncthreads();
-      if (!ks)
-#pragma unroll
-        for (int m = 0; m < MC; m++)
-#pragma unroll
-          for (int o = 1; o < KS; o++) acc[k][m] += red[(m * 4 + o * WC + wc) * 64 + lane];
-    }
-    if (ks) continue;
-    float* dst = a.part + ((long)range * 9 + k) * Cout * Cin;
-#pragma unroll
-    for (int m = 0; m < MC; m++)
+    for (int m = 0; m < 4; m++)
 #pragma unroll
       for (int v = 0; v < 4; v++) dst[(long)(co0 + m * 16 + 4 * lk + v) * Cin + ci] = acc[k][m][v];
   }
   if (do_bias) {
-    // the pixel groups' sums of each channel, added in group order
+    // the 32 pixel groups' sums of each channel, added in group order
     __syncthreads();  // every wavefront is done with the last tile
-    float* red = (float*)lds;
+    float* red = (float*)xs;  // 32 x 64 floats, inside the input tile
 #pragma unroll
-    for (int e = 0; e < 8; e++) red[(t / D8) * COB + 8 * (t % D8) + e] = bsum[e];
+    for (int e = 0; e < 8; e++) red[(t >> 3) * 64 + 8 * (t & 7) + e] = bsum[e];
     __syncthreads();
-    if (t < COB) {
+    if (t < 64) {
       float b = 0.f;
-      for (int k = 0; k < 256 / D8; k++) b += red[k * COB + t];
-      a.bpart[(long)range * Cout + co0 + t] = b;
+      for (int k = 0; k < 32; k++) b += red[k * 64 + t];
+      bpart[(long)range * Cout + co0 + t] = b;
     }
-  }
-}
-
-template <int MAX>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-    wgrad_tr(const WgradMany<MAX> m) {
-  __shared__ __attribute__((aligned(16))) bf16 lds[kWgradLds];
-  const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
-  const WgradArgs a = m.l[k];
-  const int b = blockIdx.x - m.first[k], range = b % a.ranges, block = b / a.ranges;
-  if (a.Cin % 32 == 0) {
-    if (a.Cout % 32 == 0) wgrad_block<8, 32, 32>(a, range, block, lds);
-    else wgrad_block<8, 32, 16>(a, range, block, lds);
-  } else {
-    if (a.Cout % 32 == 0) wgrad_block<8, 16, 32>(a, range, block, lds);
-    else wgrad_block<8, 16, 16>(a, range, block, lds);
   }
 }
 
@@ -835,6 +1112,23 @@ __device__ __forceinline__ float sum8(int m, F&& v) {
   return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
+// Pass 2 of the bias: 4 partial rows x 64 channels per block, each thread adding
+// every 4th block partial (sum8), then the 4 row sums in row order.
+__device__ __forceinline__ void bias_sum(const float* __restrict__ part, float* __restrict__ db,
+                                         int nb, int C, int block) {
+  __shared__ float red[256];
+  const int cl = (int)threadIdx.x & 63, r = (int)threadIdx.x >> 6;
+  const int c = block * 64 + cl;
+  float s = 0.f;
+  if (c < C) {
+    const int m = nb > r ? (nb - r + 3) / 4 : 0;  // partials r, r + 4, ...
+    s = sum8(m, [&](int k) { return part[(long)(r + 4 * k) * C + c]; });
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (r == 0 && c < C) db[c] = ((red[cl] + red[64 + cl]) + red[128 + cl]) + red[192 + cl];
+}
+
 struct ReduceArgs {
   const float* part;
   const float* bpart;
@@ -842,6 +1136,7 @@ struct ReduceArgs {
   float* db;
   long n;
   int nb, ranges;
+  int bblocks, sums;  // bias_sum of bblocks partials, in `sums` workgroups
 };
 template <int MAX>
 struct ReduceMany {
@@ -855,56 +1150,27 @@ template <int MAX>
 __global__ void __launch_bounds__(256) wgrad_reduce(const ReduceMany<MAX> m) {
   const int k = MAX > 1 ? entry_of(m.first, m.n, blockIdx.x) : 0;
   const ReduceArgs& a = m.l[k];
-  const long i = (blockIdx.x - m.first[k]) * 256L + threadIdx.x;
+  const int b = blockIdx.x - m.first[k];
+  if (b < a.sums) {
+    bias_sum(a.bpart, a.db, a.bblocks, a.nb, b);
+    return;
+  }
+  const long i = (b - a.sums) * 256L + threadIdx.x;
   if (i < a.n) a.dW[i] = sum8(a.ranges, [&](int r) { return a.part[r * a.n + i]; });
-  else if (i < a.n + a.nb)
+  else if (!a.sums && i < a.n + a.nb)
     a.db[i - a.n] = sum8(a.ranges, [&](int r) { return a.bpart[(long)r * a.nb + (i - a.n)]; });
 }
 
-// Bias gradient db[c] = sum_p dz[p][c] in two deterministic passes.  Pass 1:
-// block b sums the pixels [b chunk, (b + 1) chunk) of every channel, threads
-// laid out channel-fastest so that a pixel's channels are one coalesced row
-// (channel groups of up to 256; 256 / group pixel rows in parallel, summed in
-// a fixed order).  Pass 2 adds the block partials in block order.
 __global__ void __launch_bounds__(256) bias_grad_part(const bf16* __restrict__ dz,
                                                       float* __restrict__ part, long P, int C,
                                                       long chunk) {
   __shared__ float red[256];
-  const long p0 = (long)blockIdx.x * chunk;
-  const long p1 = p0 + chunk < P ? p0 + chunk : P;
-  for (int cb = 0; cb < C; cb += 256) {
-    const int cw = C - cb < 256 ? C - cb : 256;
-    const int rows = 256 / cw;
-    const int c = (int)threadIdx.x % cw, r = (int)threadIdx.x / cw;
-    float s = 0.f;
-    if (r < rows)
-      for (long p = p0 + r; p < p1; p += rows) s += bf2f(dz[p * C + cb + c]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if ((int)threadIdx.x < cw) {
-      float t = 0.f;
-      for (int k = 0; k < rows; k++) t += red[k * cw + threadIdx.x];
-      part[(long)blockIdx.x * C + cb + threadIdx.x] = t;
-    }
-    __syncthreads();
-  }
+  bias_part(dz, part, P, C, chunk, blockIdx.x, red);
 }
 
-// Pass 2: 4 partial rows x 64 channels per block, each thread adding every
-// 4th block partial (sum8), then the 4 row sums in row order.
 __global__ void __launch_bounds__(256) bias_grad_sum(const float* __restrict__ part,
                                                      float* __restrict__ db, int nb, int C) {
-  __shared__ float red[256];
-  const int cl = (int)threadIdx.x & 63, r = (int)threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + cl;
-  float s = 0.f;
-  if (c < C) {
-    const int m = nb > r ? (nb - r + 3) / 4 : 0;  // partials r, r + 4, ...
-    s = sum8(m, [&](int k) { return part[(long)(r + 4 * k) * C + c]; });
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  if (r == 0 && c < C) db[c] = ((red[cl] + red[64 + cl]) + red[128 + cl]) + red[192 + cl];
+  bias_sum(part, db, nb, C, blockIdx.x);
 }
 
 __global__ void combine_kernel(bf16* __restrict__ out, int ost, int ooff, const bf16* __restrict__ a,
@@ -1245,36 +1511,55 @@ int launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
   return a.Cin == 32 ? launch_conv<32>(a, s) : launch_conv<16>(a, s);
 }
 
-int wgrad_blocks(const WgradArgs& a) {
-  return (a.Cin / (a.Cin % 32 == 0 ? 32 : 16)) * (a.Cout / (a.Cout % 32 == 0 ? 32 : 16));
+// Workgroups of a layer per range: blocks of 64 x 64 channels (many layers in one
+// launch: 64 x 32) in the tile orders, of 32 x 32, or 16 where the count asks for it, in
+// kLinear, where `split` workgroups share out the taps of a block.
+int wgrad_blocks(const WgradArgs& a, bool many) {
+  if (a.order != kLinear) return (a.Cin / 64) * (a.Cout / (many ? 32 : 64));
+  return (a.Cin / (a.Cin % 32 == 0 ? 32 : 16)) * (a.Cout / (a.Cout % 32 == 0 ? 32 : 16)) * a.split;
 }
 
-// 8 x 16-pixel tiles of a layer, -1 if they do not fit an int.
-int wgrad_tiles(const WgradArgs& a) {
-  const long t = (long)a.N * ((a.W + 15) / 16) * ((a.H + 7) / 8);
-  return t > 2147483647L ? -1 : (int)t;
+// Blocks and pixels per block of the two-pass bias sum, whose partials may take cap
+// rows of cout values.
+long bias_blocks(long P, int cout, long cap, long* chunk) {
+  *chunk = 256 / (cout < 256 ? cout : 256) * 64;  // 64 pixels per thread row
+  long nb = (P + *chunk - 1) / *chunk;
+  if (nb > cap) {
+    *chunk = (P + cap - 1) / cap;
+    nb = (P + *chunk - 1) / *chunk;
+  }
+  return nb;
 }
 
-// At most `ranges` ranges of whole tiles.
-void wgrad_set_ranges(WgradArgs& a, long ranges) {
-  ranges = std::max<long>(1, std::min<long>(ranges, a.ntiles));
-  a.tiles_per_range = (int)((a.ntiles + ranges - 1) / ranges);
-  a.ranges = (int)((a.ntiles + a.tiles_per_range - 1) / a.tiles_per_range);
+// Order and ranges of a layer split over at most nsplit ranges of pixels: tiles for
+// channels in multiples of 64 and whole tiles across, of 4 rows where the image is
+// lower than 8.  Returns whether the bias is summed with the weights (the ranges
+// then leave room after their partials for one row of cout values each).
+bool wgrad_plan(WgradArgs& a, int nsplit, bool bias) {
+  const long P = (long)a.N * a.H * a.W;
+  a.split = 1;
+  if (a.Cin % 64 || a.Cout % 64 || a.W % 16) {
+    a.order = kLinear;
+    a.ntiles = (int)P;
+    a.per = (int)(((P + nsplit - 1) / nsplit + 15) / 16 * 16);
+    a.ranges = (int)((P + a.per - 1) / a.per);
+    return false;
+  }
+  a.order = a.H >= 8 ? kTile8 : kTile4;
+  const int tr = a.H >= 8 ? 8 : 4;
+  a.ntiles = (int)((long)a.N * (a.W / 16) * ((a.H + tr - 1) / tr));
+  const bool fused = bias && nsplit >= 2 && nsplit - 1 <= 9 * a.Cin;
+  const long nr = fused ? nsplit - 1 : nsplit;
+  a.per = (int)((a.ntiles + nr - 1) / nr);
+  a.ranges = (a.ntiles + a.per - 1) / a.per;
+  return fused;
 }
 
-// Blocks of 32 x 32 channels (16 where the count asks for it): the partials of a
-// workgroup are 37 KB, and four times as many workgroups share a tile range as with
-// 64 x 64, so fewer ranges fill the chip and fewer partials are written and summed.
-// Two workgroups per CU, three from 32 blocks on, where the reduction has the
-// threads for more ranges (16 x 32 x 64, 256 -> 128: 42.9 us with two, 40.4 with
-// three; 16 x 64 x 128, 64 -> 64: 30.4 and 38.0).  With the reduction, against 64 x
-// 64 blocks (and one 32-pixel step at a time from global memory for the 32-channel
-// layers): 8 x 128 x 64, 128 -> 128 44 -> 42 us; 8 x 256 x 128, 64 -> 64 53 -> 45; 8 x
-// 64 x 128, 32 -> 32 41 -> 21; 16 x 128 x 256, 32 -> 32 166 -> 45.
-long wgrad_want(int blocks) { return std::max(1, (blocks >= 32 ? 768 : 512) / blocks); }
-
-// Partials of layers with ntiles, ranges and part set (db: bias gradients or null),
-// then their sums: two launches.
+// Partials of planned layers, one launch per kind of order, then their sums in one.
+// Base 32, 4 levels on 8 x 64 x 128: 44 + 60 us and 22 us of sums for the 18 layers,
+// against 522 one layer at a time (two to four launches each; before kLinear read
+// strips of pixels from LDS, one tap per workgroup, 585).
+// db: bias gradients, of the layers with bpart.
 template <int MAX>
 int launch_wgrad(const WgradArgs* l, float* const* dW, float* const* db, int n, hipStream_t s) {
   WgradMany<MAX> m;
@@ -1284,14 +1569,28 @@ int launch_wgrad(const WgradArgs* l, float* const* dW, float* const* db, int n, 
   for (int k = 0; k < n; k++) {
     const WgradArgs& a = m.l[k] = l[k];
     const long nw = 9L * a.Cout * a.Cin;
-    const int nb = a.bpart ? a.Cout : 0;
-    m.first[k + 1] = m.first[k] + a.ranges * wgrad_blocks(a);
-    r.first[k + 1] = r.first[k] + (int)((nw + nb + 255) / 256);
-    r.l[k] = {a.part, a.bpart, dW[k], db[k], nw, nb, a.ranges};
+    const int nb = a.bpart ? a.Cout : 0, sums = a.bblocks ? (a.Cout + 63) / 64 : 0;
+    r.first[k + 1] = r.first[k] + sums + (int)((nw + (sums ? 0 : nb) + 255) / 256);
+    r.l[k] = {a.part, a.bpart, dW[k], db[k], nw, nb, a.ranges, a.bblocks, sums};
   }
-  wgrad_tr<MAX><<<m.first[n], 256, 0, s>>>(m);
-  const int rc = launch_check("conv3x3_wgrad");
-  if (rc) return rc;
+  for (const int order : {kTile8, kTile4, kLinear}) {
+    for (int k = 0; k < n; k++)
+      m.first[k + 1] = m.first[k] + (l[k].order == order
+                                         ? l[k].bblocks + l[k].ranges * wgrad_blocks(l[k], MAX > 1) : 0);
+    if (!m.first[n]) continue;
+    if (order == kLinear) wgrad_linear<MAX><<<m.first[n], 256, 0, s>>>(m);
+    else if constexpr (MAX == 1) {
+      const WgradArgs& a = l[0];
+      const dim3 g((unsigned)a.ranges, (unsigned)wgrad_blocks(a, false));
+      if (order == kTile8)
+        wgrad_tr<8><<<g, 256, 0, s>>>(a.x, a.dz, a.part, a.bpart, a.N, a.H, a.W, a.Cin, a.Cout, a.per, a.ntiles);
+      else
+        wgrad_tr<4><<<g, 256, 0, s>>>(a.x, a.dz, a.part, a.bpart, a.N, a.H, a.W, a.Cin, a.Cout, a.per, a.ntiles);
+    } else if (order == kTile8) wgrad_tiles<MAX, kTile8><<<m.first[n], 256, 0, s>>>(m);
+    else wgrad_tiles<MAX, kTile4><<<m.first[n], 256, 0, s>>>(m);
+    const int rc = launch_check("conv3x3_wgrad");
+    if (rc) return rc;
+  }
   wgrad_reduce<MAX><<<r.first[n], 256, 0, s>>>(r);
   return launch_check("wgrad_reduce");
 }
@@ -1421,21 +1720,16 @@ int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int
   a.Cin = a.c1 = cin;
   a.Cout = cout;
   const long nw = 9L * cout * cin;
-  bool bias = false;  // summed with the weights
-  if (aligned16(x) && aligned16(dz)) {
-    if ((a.ntiles = wgrad_tiles(a)) < 0)
-      return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3_wgrad: too many tiles");
-    // room after the weight partials for one row of bias partials per range
-    long nr = std::min<long>(std::min<long>(a.ntiles, wgrad_want(wgrad_blocks(a))), nsplit);
-    if (db && nsplit >= 2) {
-      while (nr > 1 && (nsplit - nr) * 9L * cin < nr) nr--;
-      bias = (nsplit - nr) * 9L * cin >= nr;
-    }
-    wgrad_set_ranges(a, nr);
+  if (aligned16(x) && aligned16(dz) && P < 2147483647L - 256) {
+    const bool fused = wgrad_plan(a, nsplit, db != nullptr);
+    // a third of the taps per workgroup, which then stages one strip of three, until
+    // the chip is full several times over: 8 x 64 x 128, 32 -> 32 39.5 -> 30.9 us; 8 x 16
+    // x 8, 256 -> 256 35.7 -> 27.0; 16 x 128 x 256, 32 -> 32 112 -> 82 (with the sums)
+    if (a.order == kLinear && (long)a.ranges * wgrad_blocks(a, false) < 2048) a.split = 3;
     a.part = partial;
-    a.bpart = bias ? partial + a.ranges * nw : nullptr;
+    a.bpart = fused ? partial + a.ranges * nw : nullptr;
     const int rc = launch_wgrad<1>(&a, &dW, &db, 1, s);
-    if (rc || !db || bias) return rc;
+    if (rc || !db || fused) return rc;
   } else {
     long chunk = (P + nsplit - 1) / nsplit;
     chunk = (chunk + 15) / 16 * 16;
@@ -1448,22 +1742,14 @@ int coffee_unet_conv3x3_wgrad(const void* x, const void* dz, float* partial, int
     r.n = 1;
     r.first[0] = 0;
     r.first[1] = (int)((nw + 255) / 256);
-    r.l[0] = {partial, nullptr, dW, nullptr, nw, 0, used};
+    r.l[0] = {partial, nullptr, dW, nullptr, nw, 0, used, 0, 0};
     wgrad_reduce<1><<<r.first[1], 256, 0, s>>>(r);
     rc = launch_check("wgrad_reduce");
     if (rc || !db) return rc;
   }
-  // the weight partials have been reduced: their buffer holds the bias
-  // partials, one row of cout per block (at most nsplit x 9 x cin rows); a
-  // block covers 64 pixels per thread row
-  const long rows = 256 / (cout < 256 ? cout : 256);
-  const long cap = (long)nsplit * 9 * cin;
-  long bchunk = rows * 64;
-  long nbb = (P + bchunk - 1) / bchunk;
-  if (nbb > cap) {
-    bchunk = (P + cap - 1) / cap;
-    nbb = (P + bchunk - 1) / bchunk;
-  }
+  // the weight partials have been reduced: their buffer holds the bias partials
+  long bchunk;
+  const long nbb = bias_blocks(P, cout, (long)nsplit * 9 * cin, &bchunk);
   bias_grad_part<<<(unsigned)nbb, 256, 0, s>>>((const bf16*)dz, partial, P, cout, bchunk);
   int rc = launch_check("bias_grad_part");
   if (rc) return rc;
@@ -1477,14 +1763,16 @@ int coffee_unet_wgrad_many(const coffee_unet_wgrad* l, int count, float* partial
     return fail(nullptr, COFFEE_ERR_INVALID, "wgrad_many: bad arguments");
   std::vector<WgradArgs> a(count);
   std::vector<float*> dW(count), db(count);
-  long work = 0;
+  long used = 0;
   for (int k = 0; k < count; k++) {
     const coffee_unet_wgrad& q = l[k];
     if (!q.x || !q.dz || !q.dw || !q.db || q.n < 1 || q.h < 1 || q.wd < 1 || q.cin < 16 ||
         q.cout < 16 || q.cin % 16 || q.cout % 16 || q.cin1 < 16 || q.cin1 % 16 || q.cin1 > q.cin ||
-        (q.cin1 < q.cin && !q.x2) || (q.up && (q.h % 2 || q.wd % 2)) || !aligned16(q.x) ||
-        !aligned16(q.x2) || !aligned16(q.dz) || 9L * q.cout * q.cin > 2147483647L / 2)
+        (q.cin1 < q.cin && !q.x2) || (q.up && (q.h % 2 || q.wd % 2)) || q.nsplit < 1 ||
+        !aligned16(q.x) || !aligned16(q.x2) || !aligned16(q.dz))
       return fail(nullptr, COFFEE_ERR_INVALID, "wgrad_many: bad arguments of layer " + std::to_string(k));
+    const long P = (long)q.n * q.h * q.wd, nw = 9L * q.cout * q.cin;
+    if (P >= 2147483647L - 256) return fail(nullptr, COFFEE_ERR_SIZE, "wgrad_many: too many pixels");
     WgradArgs& w = a[k];
     w = WgradArgs{};
     w.x = (const bf16*)q.x;
@@ -1497,24 +1785,17 @@ int coffee_unet_wgrad_many(const coffee_unet_wgrad* l, int count, float* partial
     w.Cout = q.cout;
     w.c1 = q.cin1;
     w.up = q.up;
-    if ((w.ntiles = wgrad_tiles(w)) < 0)
-      return fail(nullptr, COFFEE_ERR_SIZE, "wgrad_many: too many tiles");
-    work += (long)w.ntiles * wgrad_blocks(w);
-    dW[k] = q.dw;
-    db[k] = q.db;
-  }
-  // One tile count for every workgroup of every layer, so that three per CU end
-  // together: base 32, 4 levels on 8 x 64 x 128: 59 us and 16 us of sums for the 18
-  // layers, against 346 one layer at a time (two launches each).
-  const long per = std::max<long>(1, (work + 767) / 768);
-  long used = 0;
-  for (int k = 0; k < count; k++) {
-    WgradArgs& w = a[k];
-    const long nw = 9L * w.Cout * w.Cin;
-    wgrad_set_ranges(w, (w.ntiles + per - 1) / per);
+    const bool fused = wgrad_plan(w, q.nsplit, true);
+    if (!fused) {
+      long chunk;
+      w.bblocks = (int)bias_blocks(P, q.cout, (long)q.nsplit * 9 * q.cin, &chunk);
+      w.bchunk = (int)chunk;
+    }
     w.part = partial + used;
     w.bpart = w.part + w.ranges * nw;
-    used += w.ranges * (nw + w.Cout);
+    used += w.ranges * nw + (long)(fused ? w.ranges : w.bblocks) * q.cout;
+    dW[k] = q.dw;
+    db[k] = q.db;
   }
   if (need) *need = used;
   if (!partial) return COFFEE_OK;

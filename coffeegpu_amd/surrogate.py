@@ -251,6 +251,11 @@ class UNet:
         self._tape = (tape, n, True)
         return out32[: n * hh * ww * P["cop"]]
 
+    @staticmethod
+    def _nsplit(npix: int) -> int:
+        """Pixel ranges of a weight gradient (part of its FP32 sum)."""
+        return max(1, min(256, npix // 512))
+
     def _backward_fused(self, dout):
         """One launch per convolution for the activation gradients, which leave
         each of them as the dz of the convolution before, then two for all
@@ -294,7 +299,7 @@ class UNet:
         layers = b"".join(
             _WGRAD.pack(_a(x), _a(x2), _a(dzs[k]), _a(self.params[name]["gw"]),
                         _a(self.params[name]["gb"]), n, hh, ww, self.params[name]["cip"], c1,
-                        self.params[name]["cop"], up, 0)
+                        self.params[name]["cop"], up, self._nsplit(n * hh * ww))
             for k, (name, x, x2, c1, up, _, hh, ww) in enumerate(tape))
         need = ctypes.c_long()
         _lib.check(self._lib.coffee_unet_wgrad_many(layers, len(tape), None, 0, ctypes.byref(need), s))
@@ -369,7 +374,7 @@ class UNet:
             pos[0] -= 1
             P = self.params[name]
             npix = n * hh * ww
-            nsplit = max(1, min(256, npix // 512))
+            nsplit = self._nsplit(npix)
             part = self._buf(("part",), nsplit * 9 * P["cop"] * P["cip"], torch.float32)
             _lib.check(self._lib.coffee_unet_conv3x3_wgrad(
                 _p(xin), _p(dz), _p(part), nsplit, _p(P["gw"]), _p(P["gb"]), n, hh, ww, P["cip"],

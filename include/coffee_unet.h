@@ -64,13 +64,14 @@ int coffee_unet_conv3x3_fusable(int n, int h, int wd, int cin, int cout, int pai
 int coffee_unet_conv3x3_wgrad(const void *x, const void *dz, float *partial, int nsplit, float *dW,
                               float *db, int n, int h, int wd, int cin, int cout, void *stream);
 
-/* Weight and bias gradients of many layers in two launches; x, x2, cin1 and up are
- * the input as in coffee_unet_conv.  partial holds `floats` FP32 values; with
+/* Weight and bias gradients of many layers in two launches, each the same bits as
+ * from coffee_unet_conv3x3_wgrad with its nsplit; x, x2, cin1 and up are the input
+ * as in coffee_unet_conv.  partial holds `floats` FP32 values; with
  * partial NULL only *need (the number required) is set. */
 typedef struct {
   const void *x, *x2, *dz;
   float *dw, *db;
-  int n, h, wd, cin, cin1, cout, up, pad;
+  int n, h, wd, cin, cin1, cout, up, nsplit;
 } coffee_unet_wgrad;
 int coffee_unet_wgrad_many(const coffee_unet_wgrad *l, int count, float *partial, long floats,
                            long *need, void *stream);
