@@ -461,6 +461,14 @@ int batch_create(coffee_ctx* c, int nruns, const coffee_grid* grids, const coffe
   HIP_TRY(c, hipMalloc(&S->d_clocks, sizeof(SphClock) * 2 * nruns));
   int rc = S->upload(c);
   if (rc) return rc;
+  // Until a tile is set or tuned: taps through the caches while the fields fit the
+  // L2s, the tile and its halo in LDS above (us per step of tiles 0, 5 and 9: FP32
+  // 524 k cells 94, 93, 94; 1.05 M 158, 151, 150; 2.1 M 358, 297, 304; 4.2 M 866,
+  // 693, 718; FP64 33 k 45, 48, 42; 131 k 66, 55, 55; 524 k 177, 169, 150).
+  double cells = 0;
+  for (const SphRun<T>& R : S->h_runs) cells += (double)R.n0 * R.n1;
+  if (sizeof(T) == 4 && cells >= 800e3) S->tile = 5;
+  if (sizeof(T) == 8 && cells >= 100e3) S->tile = 9;
   return S->build_items(c);
 }
 

@@ -62,3 +62,28 @@ def test_axis_rows_and_clocks(n, tile, graph):
                 for q in range(7):
                     r.U[q][...] = U[q]
     b.close()
+
+
+# total cells on both sides of the lines (FP32 800 k, FP64 100 k), extents off every
+# tile shape, runs that stop together and runs that do not (either order of the
+# work list)
+@pytest.mark.parametrize("dtype,n", [(np.float32, (799, 500)), (np.float32, (801, 501)),
+                                     (np.float64, (333, 150)), (np.float64, (335, 151))])
+@pytest.mark.parametrize("stops", [(0, 0), (1, 3)])
+def test_default_tile_is_bitwise_the_first(dtype, n, stops):
+    sp, U0 = case_sph(dtype, n=n, omega=0.3, dw0=0.2, pml=2)
+    env = SimEnvironment(sp, dtype, "cuda:0")
+    outs = []
+    for tile in (None, 0, 11):
+        datas = [SimData(env) for _ in range(2)]
+        for d in datas:
+            d.set_state(U0)
+        b = SphBatch([env, env], datas, nsteps=list(stops))
+        if tile is not None:
+            b.set_tile(tile)
+        b.step(2)
+        outs.append([d.get_state() for d in datas])
+        b.close()
+    for o in outs[1:]:
+        for x, y in zip(o, outs[0]):
+            assert np.array_equal(x, y)
