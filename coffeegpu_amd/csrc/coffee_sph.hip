@@ -105,7 +105,7 @@ int stage_occupancy() {
 
 struct SphStateBase : SolverState {
   virtual int prepare(coffee_ctx* c, hipStream_t s) = 0;
-  virtual int step(coffee_ctx* c, hipStream_t s) = 0;
+  virtual int step(coffee_ctx* c, int k, hipStream_t s) = 0;  // step k of a call
 };
 
 template <typename T>
@@ -113,8 +113,7 @@ struct SphState : SphStateBase {
   std::vector<SphRun<T>> h_runs;
   SphRun<T>* d_runs = nullptr;
   std::vector<SphClock> h_clocks;  // as set up
-  SphClock* d_clocks = nullptr;    // two of each run, see SphClock
-  int parity = 0;                  // which of the two the next step reads
+  SphClock* d_clocks = nullptr;    // the tables of SphClock
   SphItem* d_items = nullptr;
   int nitems = 0;
   int tile = 0;
@@ -123,8 +122,8 @@ struct SphState : SphStateBase {
   int max_guards = 0;           // most guard and axis cells of a run
   std::vector<void*> owned;
   bool use_graph = false;
-  hipGraphExec_t graph_exec[2] = {};  // one step from either parity
-  hipGraph_t graph[2] = {};
+  hipGraphExec_t graph_exec[kClockTables] = {};  // one step, by the table it reads
+  hipGraph_t graph[kClockTables] = {};
 
   ~SphState() override {
     drop_graph();
@@ -137,7 +136,7 @@ struct SphState : SphStateBase {
   // A captured graph holds the work-list pointer and the launch geometry of
   // the tile it was captured with: any rebuild of the work list drops it.
   void drop_graph() {
-    for (int q = 0; q < 2; q++) {
+    for (int q = 0; q < kClockTables; q++) {
       if (graph_exec[q]) (void)hipGraphExecDestroy(graph_exec[q]);
       if (graph[q]) (void)hipGraphDestroy(graph[q]);
       graph_exec[q] = nullptr;
@@ -146,6 +145,20 @@ struct SphState : SphStateBase {
   }
 
   SphClock* clocks(int which) { return d_clocks + (size_t)which * h_clocks.size(); }
+
+  // Table that step k of a call reads.
+  static int table_of(int k) { return k == 0 ? kStart : k & 1; }
+
+  // Every run's clock as the work launched so far leaves it (waits for that work).
+  int read_clocks(coffee_ctx* c, std::vector<SphClock>& out) {
+    HIP_TRY(c, hipDeviceSynchronize());
+    const int n = (int)h_clocks.size();
+    std::vector<SphClock> h(2 * (size_t)n);
+    HIP_TRY(c, hipMemcpy(h.data(), d_clocks, sizeof(SphClock) * h.size(), hipMemcpyDeviceToHost));
+    out.resize(n);
+    for (int r = 0; r < n; r++) out[r] = newer_clock(h.data(), n, r);
+    return COFFEE_OK;
+  }
 
   // Order of the tiles: item k is worked on by XCD k mod 8 (workgroups are handed
   // out in turn, and a grid smaller than the list is a multiple of 8), and every
@@ -207,9 +220,9 @@ struct SphState : SphStateBase {
   }
 
   template <typename Tag>
-  int launch_step(coffee_ctx* c, hipStream_t s) {
+  int launch_step(coffee_ctx* c, int table, hipStream_t s) {
     const int nr = (int)h_runs.size();
-    const SphClock* ck = clocks(parity);
+    const SphClock* ck = clocks(table);
     int rc = COFFEE_OK;
     // the march kernels leave the axis rows to a launch of their own
     const dim3 ga((max_n0 + 255) / 256, nr);
@@ -239,7 +252,7 @@ struct SphState : SphStateBase {
       if (rc || (rc = axis(src ^ 1))) return rc;
     }
     rc = timed(c, "sph_ko", s, [&] {
-      launch_ko<T, Tag>(grid_blocks, s, d_runs, ck, d_items, nitems, 1, nr, clocks(parity ^ 1));
+      launch_ko<T, Tag>(grid_blocks, s, d_runs, ck, d_items, nitems, 1, nr, clocks(table == 1 ? 0 : 1));
     });
     return rc ? rc : axis(0);
   }
@@ -248,34 +261,28 @@ struct SphState : SphStateBase {
   int prepare(coffee_ctx* c, hipStream_t s) override {
     const int nr = (int)h_runs.size();
     const dim3 g((max_guards + 255) / 256, nr);
-    return timed(c, "sph_prepare", s, [&] { sph_prepare_kernel<T><<<g, 256, 0, s>>>(d_runs, clocks(parity), nr); });
+    return timed(c, "sph_prepare", s, [&] { sph_prepare_kernel<T><<<g, 256, 0, s>>>(d_runs, d_clocks, nr); });
   }
 
   int prepare_single(coffee_ctx* c, hipStream_t s) {
     return timed(c, "sph_prepare", s, [&] {
       sph_prepare_single_kernel<T><<<(max_guards + 255) / 256, 256, 0, s>>>(h_runs[0], d_runs,
-                                                                              h_clocks[0], clocks(parity));
+                                                                              h_clocks[0], clocks(kStart));
     });
   }
 
-  int launch_step_tile(coffee_ctx* c, hipStream_t s) {
-    return with_tile(tile, [&](auto tag) { return launch_step<decltype(tag)>(c, s); });
+  int step_direct(coffee_ctx* c, int table, hipStream_t s) {
+    return with_tile(tile, [&](auto tag) { return launch_step<decltype(tag)>(c, table, s); });
   }
 
-  int step_direct(coffee_ctx* c, hipStream_t s) {
-    const int rc = launch_step_tile(c, s);
-    if (!rc) parity ^= 1;
-    return rc;
-  }
-
-  int step(coffee_ctx* c, hipStream_t s) override {
-    if (!use_graph || c->timing || c->diagnostics) return step_direct(c, s);
-    const int q = parity;
+  int step(coffee_ctx* c, int k, hipStream_t s) override {
+    const int q = table_of(k);
+    if (!use_graph || c->timing || c->diagnostics) return step_direct(c, q, s);
     if (!graph_exec[q]) {
       hipStream_t cs;
       HIP_TRY(c, hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
       HIP_TRY(c, hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      int rc = launch_step_tile(c, cs);
+      int rc = step_direct(c, q, cs);
       hipGraph_t g = nullptr;
       hipError_t e = hipStreamEndCapture(cs, &g);
       (void)hipStreamDestroy(cs);
@@ -285,15 +292,15 @@ struct SphState : SphStateBase {
       HIP_TRY(c, hipGraphInstantiate(&graph_exec[q], g, nullptr, nullptr, 0));
     }
     HIP_TRY(c, hipGraphLaunch(graph_exec[q], s));
-    parity ^= 1;
     return COFFEE_OK;
   }
 
   int upload(coffee_ctx* c) {
     HIP_TRY(c, hipMemcpy(d_runs, h_runs.data(), sizeof(SphRun<T>) * h_runs.size(),
                          hipMemcpyHostToDevice));
-    HIP_TRY(c, hipMemcpy(d_clocks, h_clocks.data(), sizeof(SphClock) * h_clocks.size(),
-                         hipMemcpyHostToDevice));
+    for (int q = 0; q < kClockTables; q++)
+      HIP_TRY(c, hipMemcpy(clocks(q), h_clocks.data(), sizeof(SphClock) * h_clocks.size(),
+                           hipMemcpyHostToDevice));
     return COFFEE_OK;
   }
 };
@@ -458,7 +465,7 @@ int batch_create(coffee_ctx* c, int nruns, const coffee_grid* grids, const coffe
     S->max_guards = std::max(S->max_guards, 2 * R.g1 * R.dims0 + 2 * R.g0 * R.n1 + R.n0);
   }
   HIP_TRY(c, hipMalloc(&S->d_runs, sizeof(SphRun<T>) * nruns));
-  HIP_TRY(c, hipMalloc(&S->d_clocks, sizeof(SphClock) * 2 * nruns));
+  HIP_TRY(c, hipMalloc(&S->d_clocks, sizeof(SphClock) * kClockTables * nruns));
   int rc = S->upload(c);
   if (rc) return rc;
   // Until a tile is set or tuned: taps through the caches while the fields fit the
@@ -531,7 +538,7 @@ int sph_step_impl(coffee_ctx* c, const coffee_fields* f, double time, hipStream_
     return fail(c, COFFEE_ERR_INVALID, "diagnostics need J, divE, divB");
   S->h_clocks[0] = SphClock{time, 0, 0, 1};
   int rc = S->prepare_single(c, s);
-  return rc ? rc : S->step_direct(c, s);
+  return rc ? rc : S->step_direct(c, kStart, s);
 }
 
 int sph_step(coffee_ctx* c, const coffee_fields* f, double time, hipStream_t s) {
@@ -652,6 +659,11 @@ using namespace coffee;
 template <typename T>
 int autotune_impl(coffee_ctx* c, int trials, hipStream_t s, int* best, double* ms_out) {
   auto* S = static_cast<SphState<T>*>(c->state);
+  // the runs that are still active (the launches read the table of a call's start)
+  std::vector<SphClock> now;
+  int rc = S->read_clocks(c, now);
+  if (rc) return rc;
+  HIP_TRY(c, hipMemcpy(S->clocks(kStart), now.data(), sizeof(SphClock) * now.size(), hipMemcpyHostToDevice));
   hipEvent_t a, b;
   HIP_TRY(c, hipEventCreate(&a));
   HIP_TRY(c, hipEventCreate(&b));
@@ -663,7 +675,7 @@ int autotune_impl(coffee_ctx* c, int trials, hipStream_t s, int* best, double* m
     auto launch = [&] {
       with_tile(t, [&](auto tag) {
         launch_stage<T, decltype(tag), true, false, false>(S->grid_blocks, s, S->d_runs,
-                                                           S->clocks(S->parity), S->d_items, S->nitems, 0, T(0),
+                                                           S->clocks(kStart), S->d_items, S->nitems, 0, T(0),
                                                            (T)kBs[0], T(0));
         return 0;
       });
@@ -679,7 +691,7 @@ int autotune_impl(coffee_ctx* c, int trials, hipStream_t s, int* best, double* m
     return COFFEE_OK;
   };
   for (int t = 0; t < kNumTiles; t++) {
-    int rc = time_tile(t, &ms[t]);
+    rc = time_tile(t, &ms[t]);
     if (rc) return rc;
   }
   double fastest = *std::min_element(ms.begin(), ms.end());
@@ -689,7 +701,7 @@ int autotune_impl(coffee_ctx* c, int trials, hipStream_t s, int* best, double* m
   for (int round = 0; round < 2 && near.size() > 1; round++)
     for (int t : near) {
       double m = 0;
-      int rc = time_tile(t, &m);
+      rc = time_tile(t, &m);
       if (rc) return rc;
       ms[t] = std::min(ms[t], m);
     }
@@ -762,7 +774,7 @@ int coffee_sph_batch_step(coffee_batch* c, int nsteps, void* stream) {
   auto* S = static_cast<SphStateBase*>(c->state);
   if (nsteps < 1) return COFFEE_OK;
   int rc = S->prepare(c, (hipStream_t)stream);
-  for (int k = 0; k < nsteps && !rc; k++) rc = S->step(c, (hipStream_t)stream);
+  for (int k = 0; k < nsteps && !rc; k++) rc = S->step(c, k, (hipStream_t)stream);
   return rc;
 }
 
@@ -821,18 +833,11 @@ int coffee_sph_batch_residuals(coffee_batch* c, double* out, void* stream) {
 
 int coffee_sph_batch_status(coffee_batch* c, int* active, double* t, int* step) {
   if (!is_batch(c)) return fail(c, COFFEE_ERR_STATE, "not a spherical batch");
-  HIP_TRY(c, hipDeviceSynchronize());
-  const SphClock* d;
-  size_t n;
-  auto of = [&](auto* S) {
-    d = S->clocks(S->parity);
-    n = S->h_clocks.size();
-  };
-  if (c->scalar == 4) of(static_cast<SphState<float>*>(c->state));
-  else of(static_cast<SphState<double>*>(c->state));
-  std::vector<SphClock> h(n);
-  HIP_TRY(c, hipMemcpy(h.data(), d, sizeof(SphClock) * n, hipMemcpyDeviceToHost));
-  for (size_t r = 0; r < n; r++) {
+  std::vector<SphClock> h;
+  const int rc = c->scalar == 4 ? static_cast<SphState<float>*>(c->state)->read_clocks(c, h)
+                                : static_cast<SphState<double>*>(c->state)->read_clocks(c, h);
+  if (rc) return rc;
+  for (size_t r = 0; r < h.size(); r++) {
     if (active) active[r] = h[r].active;
     if (t) t[r] = h[r].t;
     if (step) step[r] = h[r].step;

@@ -57,13 +57,25 @@ struct SphRun {
 };
 
 // Time and step counter of a run: the part of its state that a step changes.
-// Apart from the descriptor, which the kernels read as constant memory, and
-// kept twice: steps alternate between the two, each step's Kreiss-Oliger launch
-// writing the other one (sph_advance), so that no launch reads what it writes.
+// Apart from the descriptor, which the kernels read as constant memory, and in
+// three tables, so that no launch reads what it writes: the first launch of a
+// call (sph_prepare_kernel) puts every run's clock into the table kStart, the first
+// step reads that one and its Kreiss-Oliger launch writes the next clock into
+// table 1 (sph_advance), the second step reads table 1 and writes 0, and so on.
+// Which of 0 and 1 holds the newer clock is seen from the step counters on the
+// device: launches are the same for every call of so many steps, so a call
+// recorded in a graph by the caller goes on from whatever ran before each replay.
 struct SphClock {
   double t;  // time of the step being taken
   int step, nsteps, active;
 };
+enum { kStart = 2, kClockTables = 3 };
+
+// The newer of a run's clocks in tables 0 and 1 (equal where the step counts are).
+__host__ __device__ inline const SphClock& newer_clock(const SphClock* tables, int nruns, int run) {
+  const SphClock &a = tables[run], &b = tables[nruns + run];
+  return b.step > a.step ? b : a;
+}
 
 struct SphItem {
   int run, i0, j0;
@@ -938,11 +950,12 @@ __device__ __forceinline__ void sph_prepare_run(const SphRun<T>& R) {
 
 template <typename T>
 __global__ void __launch_bounds__(256)
-    sph_prepare_kernel(const SphRun<T>* __restrict__ runs, const SphClock* __restrict__ clocks,
-                       int nruns) {
+    sph_prepare_kernel(const SphRun<T>* __restrict__ runs, SphClock* __restrict__ tables, int nruns) {
   const int run = blockIdx.y;
-  if (run >= nruns || !clocks[run].active) return;
-  sph_prepare_run(runs[run]);
+  if (run >= nruns) return;
+  const SphClock c = newer_clock(tables, nruns, run);
+  if (blockIdx.x == 0 && threadIdx.x == 0) tables[kStart * nruns + run] = c;
+  if (c.active) sph_prepare_run(runs[run]);
 }
 
 // The same for a single run whose descriptor comes with the launch (it holds
