@@ -1470,45 +1470,105 @@ bool conv_tiled(const ConvArgs& a) {
 // Outputs of 2 x 2 pixels: a wavefront has to hold both rows (tiles of 8 rows).
 bool conv_pairs(const ConvArgs& a) { return a.form == kUpBack || a.pool; }
 
+// Tile of conv3x3_tile: image rows, 16-channel blocks of the output, channels
+// staged at once.
+struct ConvTile {
+  int tr, nb, cp;
+};
+
+long conv_groups(const ConvArgs& a, int tr, int nb) {
+  return (long)a.N * ((a.W + 15) / 16) * ((a.H + tr - 1) / tr) * (a.Cout / (16 * nb));
+}
+
+// The largest (most MFMAs per LDS read, least halo) that still gives two
+// workgroups per CU, else one with more workgroups; 4 rows for images of no more
+// (8 x 1 x 16384, 32 -> 64 83 us with 8 rows and 64 channels, 62 with 4 and 32).
+ConvTile conv_tile(const ConvArgs& a) {
+  const int cp = conv_by_chunks(a) ? 32 : a.Cin;
+  const bool c32 = a.Cout % 32 == 0, pairs = conv_pairs(a);
+  if (cp == 256) return {4, 1, 256};  // all channels staged at once: 126 KiB of LDS
+  if (cp == 128) return {pairs ? 8 : 4, c32 ? 2 : 1, 128};  // 63 to 117 KiB
+  if (a.Cout % 64 == 0 && cp == 32 && (a.H > 4 || pairs)) {
+    if (a.H > 8 && conv_groups(a, 16, 4) >= 512) return {16, 4, 32};
+    if (conv_groups(a, 8, 4) >= 512) return {8, 4, 32};
+  }
+  if (c32 && (pairs || (a.H > 4 && conv_groups(a, 8, 2) >= 256))) return {8, 2, cp};
+  if (c32) return {4, 2, cp};
+  return {8, 1, cp};
+}
+
+// 64 or 128 pixels (mb = 1 or 2) x 16 nb channels per workgroup of the kernels that
+// sum by taps from global memory: conv3x3_k32 takes two 16-pixel row blocks per
+// wavefront when that still leaves two workgroups per CU.
+struct ConvTaps {
+  int nb, mb;
+  long groups;
+};
+ConvTaps conv_taps(const ConvArgs& a) {
+  const long P = (long)a.N * a.H * a.W;
+  const int nb = a.Cout % 64 == 0 ? 4 : a.Cout % 32 == 0 ? 2 : 1;
+  const long cb = a.Cout / (16 * nb);
+  const int mb = a.Cin % 32 == 0 && (P + 127) / 128 * cb >= 512 ? 2 : 1;
+  return {nb, mb, (P + 64 * mb - 1) / (64 * mb) * cb};
+}
+
+// Estimated microseconds of conv3x3_tile and of conv3x3_k32 (Cin = 16: conv3x3_mfma)
+// on a shape that both sum by taps, to the same bits.  Both are a start-up and a
+// time per round of resident workgroups, fitted to 430 shapes (N 1 to 65536, H and W
+// 1 to 16384, 16 to 256 channels; most within 10 %, the worst 40 % off).  What decides:
+// a tile works on whole 16 x 4 .. 16 x 16 pixels, whatever the image fills of them,
+// and with 128 or 256 channels one workgroup has the CU to itself and restages its
+// input for every 16 or 32 output channels; the others read every tap from the
+// caches, a long chain that a few workgroups wait out.  Of the tile and the other kernel:
+// 256 -> 256 8 x 16 x 8 9 and 42 us, 16 x 78 x 89 931 and 336, 65536 images of 1 x 1 27554
+// and 127; 128 -> 128 12 x 48 x 134 122 and 65; 64 -> 64 6 x 73 x 40 7.5 and 16.3.
+double conv_tile_us(const ConvArgs& a) {
+  const ConvTile t = conv_tile(a);
+  const double base = t.cp == 16 ? 0.3 : t.cp == 32 ? 0.6 : t.cp == 64 ? 0.5 : t.cp == 128 ? 3.3 : 6.0;
+  const double slope = t.cp == 16 ? 0.105 : t.cp == 32 ? 0.125 : 0.265;
+  const double slots = t.cp == 256 || (t.cp == 128 && t.tr * t.nb > 4) ? 256 : 512;
+  return 3.5 + (base + slope * t.tr * t.nb) * std::max(1.0, conv_groups(a, t.tr, t.nb) / slots);
+}
+
+double conv_taps_us(const ConvArgs& a) {
+  const ConvTaps t = conv_taps(a);
+  const double rounds = std::max(1.0, t.groups / 512.0);
+  if (a.Cin == 16) return 3 + t.nb + (0.5 + 0.75 * t.nb) * rounds;
+  if (t.mb == 1) return 4 + a.Cin * (0.07 + (t.nb == 4 ? 0.11 : 0.09) * rounds);
+  return 5 + a.Cin * (0.11 + (t.nb == 4 ? 0.145 : t.nb == 2 ? 0.105 : 0.08) * rounds);
+}
+
+// Whether the tile is the faster kernel for a convolution that conv_tiled takes (in
+// doubt, within 5 %, the other one: tiny images are faster than its estimate).
+bool conv_tile_pays(const ConvArgs& a) {
+  return conv_by_chunks(a) || 1.05 * conv_tile_us(a) <= conv_taps_us(a);
+}
+
 template <int TR, int NB, int CP>
 void launch_conv_tile(const ConvArgs& a, hipStream_t s) {
-  const dim3 g((unsigned)((long)a.N * ((a.W + 15) / 16) * ((a.H + TR - 1) / TR)),
-               (unsigned)(a.Cout / (16 * NB)));
+  const dim3 g((unsigned)(conv_groups(a, TR, NB) / (a.Cout / (16 * NB))), (unsigned)(a.Cout / (16 * NB)));
   if (a.flip) conv3x3_tile<TR, NB, CP, true><<<g, 256, 0, s>>>(a);
   else conv3x3_tile<TR, NB, CP, false><<<g, 256, 0, s>>>(a);
 }
 
-// Tile of a convolution: the largest (most MFMAs per LDS read, least halo) that
-// still gives two workgroups per CU, else one with more workgroups.
 template <int CP>
-int launch_conv(const ConvArgs& a, hipStream_t s) {
-  auto blocks = [&](int tr, int nb) {
-    return (long)a.N * ((a.W + 15) / 16) * ((a.H + tr - 1) / tr) * (a.Cout / (16 * nb));
-  };
-  const bool c32 = a.Cout % 32 == 0, pairs = conv_pairs(a);
-  if (a.Cout % 64 == 0 && CP == 32 && a.H > 8 && blocks(16, 4) >= 512) launch_conv_tile<16, 4, 32>(a, s);
-  else if (a.Cout % 64 == 0 && CP == 32 && blocks(8, 4) >= 512) launch_conv_tile<8, 4, 32>(a, s);
-  else if (c32 && (pairs || (a.H > 4 && blocks(8, 2) >= 256))) launch_conv_tile<8, 2, CP>(a, s);
-  else if (c32) launch_conv_tile<4, 2, CP>(a, s);
+void launch_conv(const ConvArgs& a, const ConvTile& t, hipStream_t s) {
+  if (t.nb == 2 && t.tr == 8) launch_conv_tile<8, 2, CP>(a, s);
+  else if (t.nb == 2) launch_conv_tile<4, 2, CP>(a, s);
+  else if (CP == 128 && t.tr == 4) launch_conv_tile<4, 1, 128>(a, s);
   else launch_conv_tile<8, 1, CP>(a, s);
-  return launch_check("conv3x3");
 }
 
 int launch_conv_tiled(const ConvArgs& a, hipStream_t s) {
-  if (conv_by_chunks(a)) return launch_conv<32>(a, s);
-  if (a.Cin == 256) {  // all channels staged at once: 129 KB of LDS
-    launch_conv_tile<4, 1, 256>(a, s);
-    return launch_check("conv3x3");
-  }
-  if (a.Cin == 128) {  // 101 (64, 121, 84) KB
-    if (conv_pairs(a) && a.Cout % 32 == 0) launch_conv_tile<8, 2, 128>(a, s);
-    else if (conv_pairs(a)) launch_conv_tile<8, 1, 128>(a, s);
-    else if (a.Cout % 32 == 0) launch_conv_tile<4, 2, 128>(a, s);
-    else launch_conv_tile<4, 1, 128>(a, s);
-    return launch_check("conv3x3");
-  }
-  if (a.Cin == 64) return launch_conv<64>(a, s);
-  return a.Cin == 32 ? launch_conv<32>(a, s) : launch_conv<16>(a, s);
+  const ConvTile t = conv_tile(a);
+  if (t.cp == 256) launch_conv_tile<4, 1, 256>(a, s);
+  else if (t.cp == 128) launch_conv<128>(a, t, s);
+  else if (t.cp == 64) launch_conv<64>(a, t, s);
+  else if (t.cp == 16) launch_conv<16>(a, t, s);
+  else if (t.nb == 4 && t.tr == 16) launch_conv_tile<16, 4, 32>(a, s);
+  else if (t.nb == 4) launch_conv_tile<8, 4, 32>(a, s);
+  else launch_conv<32>(a, t, s);
+  return launch_check("conv3x3");
 }
 
 // Workgroups of a layer per range: blocks of 64 x 64 channels (many layers in one
@@ -1624,22 +1684,18 @@ int coffee_unet_conv3x3(const void* in, const void* w, const float* bias, void* 
   const long P = (long)n * h * wd;
   const long bx = (P + 63) / 64;
   if (bx > 2147483647L) return fail(nullptr, COFFEE_ERR_SIZE, "conv3x3: too many pixels");
-  if (conv_tiled(a)) return launch_conv_tiled(a, s);
+  if (conv_tiled(a) && conv_tile_pays(a)) return launch_conv_tiled(a, s);
   if (cin % 32 == 0 && aligned16(in) && aligned16(w)) {
-    // K = 32 kernel; two 16-pixel row blocks per wavefront when that still
-    // leaves two workgroups per CU
-    const int nb = cout % 64 == 0 ? 4 : (cout % 32 == 0 ? 2 : 1);
-    const long b2 = (P + 127) / 128, cb = cout / (16 * nb);
-    const bool mb2 = b2 * cb >= 512;
-    const unsigned gx = (unsigned)(mb2 ? b2 : bx);
-    const dim3 g(gx, (unsigned)cb);
+    const ConvTaps t = conv_taps(a);
+    const long cb = cout / (16 * t.nb);
+    const dim3 g((unsigned)(t.groups / cb), (unsigned)cb);
 #define COFFEE_CONV32(NBV)                                              \
   do {                                                                  \
-    if (mb2) conv3x3_k32<NBV, 2><<<g, 256, 0, s>>>(a);                 \
+    if (t.mb == 2) conv3x3_k32<NBV, 2><<<g, 256, 0, s>>>(a);           \
     else conv3x3_k32<NBV, 1><<<g, 256, 0, s>>>(a);                     \
   } while (0)
-    if (nb == 4) COFFEE_CONV32(4);
-    else if (nb == 2) COFFEE_CONV32(2);
+    if (t.nb == 4) COFFEE_CONV32(4);
+    else if (t.nb == 2) COFFEE_CONV32(2);
     else COFFEE_CONV32(1);
 #undef COFFEE_CONV32
   } else if (cout % 64 == 0) {
