@@ -117,6 +117,7 @@ SIGNATURES = {
     "coffee_unet_conv3x3_wgrad": (ctypes.c_int, [_V, _V, _V, _I, _V, _V, _I, _I, _I, _I, _I, _V]),
     "coffee_unet_conv3x3_fused": (ctypes.c_int, [_V, _V]),
     "coffee_unet_conv3x3_fusable": (ctypes.c_int, [_I, _I, _I, _I, _I, _I]),
+    "coffee_unet_conv3x3_excess": (ctypes.c_double, [_I, _I, _I, _I, _I, _I]),
     "coffee_unet_wgrad_many": (ctypes.c_int, [_V, _I, _V, _L, ctypes.POINTER(_L), _V]),
     "coffee_unet_mse_pinned": (ctypes.c_int, [_V, _I, _V, _I, _L, _V, _V,
                                               ctypes.POINTER(ctypes.c_double), _V]),

@@ -1512,6 +1512,18 @@ ConvTaps conv_taps(const ConvArgs& a) {
   return {nb, mb, (P + 64 * mb - 1) / (64 * mb) * cb};
 }
 
+// Arguments that are sizes alone (pairs: outputs of 2 x 2 pixels).
+ConvArgs conv_sizes(int n, int h, int w, int cin, int cout, bool pairs) {
+  ConvArgs a{};
+  a.N = n;
+  a.H = h;
+  a.W = w;
+  a.Cin = cin;
+  a.Cout = cout;
+  a.form = pairs ? kUpBack : kOut;
+  return a;
+}
+
 // Estimated microseconds of conv3x3_tile and of conv3x3_k32 (Cin = 16: conv3x3_mfma)
 // on a shape that both sum by taps, to the same bits.  Both are a start-up and a
 // time per round of resident workgroups, fitted to 430 shapes (N 1 to 65536, H and W
@@ -1710,14 +1722,15 @@ int coffee_unet_conv3x3(const void* in, const void* w, const float* bias, void* 
 
 int coffee_unet_conv3x3_fusable(int n, int h, int wd, int cin, int cout, int pairs) {
   if (n < 1 || h < 1 || wd < 1 || cin < 16 || cout < 16 || cin % 16 || cout % 16) return 0;
-  ConvArgs a{};
-  a.N = n;
-  a.H = h;
-  a.W = wd;
-  a.Cin = cin;
-  a.Cout = cout;
+  const ConvArgs a = conv_sizes(n, h, wd, cin, cout, false);
   // all of 256 channels leave no room for tiles of 8 rows
   return conv_tiled(a) && (!pairs || conv_by_chunks(a) || cin != 256);
+}
+
+double coffee_unet_conv3x3_excess(int n, int h, int wd, int cin, int cout, int pairs) {
+  if (!coffee_unet_conv3x3_fusable(n, h, wd, cin, cout, pairs)) return 0.0;
+  const ConvArgs a = conv_sizes(n, h, wd, cin, cout, pairs != 0);
+  return conv_by_chunks(a) ? 0.0 : std::max(0.0, conv_tile_us(a) - conv_taps_us(a));
 }
 
 int coffee_unet_conv3x3_fused(const coffee_unet_conv* c, void* stream) {

@@ -58,6 +58,11 @@ int coffee_unet_conv3x3_fused(const coffee_unet_conv *c, void *stream);
  * pool or form 3), else 0. */
 int coffee_unet_conv3x3_fusable(int n, int h, int wd, int cin, int cout, int pairs);
 
+/* Estimated microseconds that coffee_unet_conv3x3_fused takes longer on such a
+ * convolution than the kernel that coffee_unet_conv3x3 would choose for it (0 where
+ * that is the same one): large for many images of a few pixels. */
+double coffee_unet_conv3x3_excess(int n, int h, int wd, int cin, int cout, int pairs);
+
 /* Weight gradient: dW[tap][co][ci] = sum_p dz[p][co] * x[p + (dy,dx)][ci],
  * split over `nsplit` pixel ranges into `partial` (nsplit*9*cout*cin FP32),
  * then reduced into dW (FP32); db[co] = sum_p dz[p][co] (FP32, may be NULL). */

@@ -64,3 +64,37 @@ def test_conv_takes_the_faster_kernel(shape, ci, co):
     assert torch.equal(y, z)
     # 1.4: the estimate that decides is up to a third off, and short calls vary
     assert picked <= 1.4 * other, (picked, other)
+
+
+# (levels, base, images, rows, columns), and whether the forward and the backward
+# pass pay in their fused form: none, the second one, both
+@pytest.mark.parametrize("levels,base,n,h,w,pays", [
+    (4, 32, 4096, 8, 8, (False, False)), (4, 32, 512, 8, 8, (False, True)), (3, 32, 4096, 4, 4, (False, False)),
+    (3, 32, 2048, 4, 4, (False, True)), (4, 32, 3, 40, 72, (True, True))])
+def test_network_on_small_images_takes_the_faster_passes(levels, base, n, h, w, pays):
+    from coffeegpu_amd.surrogate import UNet, pad16
+
+    net = UNet(levels, base, 7, 6, seed=1)
+    g = torch.Generator(device=DEV).manual_seed(h)
+    x = rand(g, n * h * w * pad16(7)).bfloat16().view(torch.int16)
+    t = rand(g, n * h * w * 6)
+
+    def grads(out):
+        loss, d = net.loss_and_grad(out, t, n, h, w)
+        dx = net.backward(d)[: n * h * w * 16].clone()
+        return [dx] + [P[k].clone() for P in net.params.values() for k in ("gw", "gb")]
+
+    assert net._fused(x, n, h, w)
+    want = [net._forward_by_parts(x, n, h, w).clone()]
+    want += grads(want[0])
+    other = [net._forward_fused(x, n, h, w).clone()]
+    other += grads(other[0])
+    got = [net.forward(x, n, h, w).clone()]
+    assert net._tape[2] == pays[1]
+    got += grads(got[0])
+    for a, b, c in zip(got, want, other):
+        assert torch.equal(a, b) and torch.equal(a, c)
+    picked = microseconds(lambda: net.forward(x, n, h, w))
+    assert net._pays(n, h, w) == pays
+    # 1.5: the fused pass of 512 x 8 x 8 takes 1.8 times as long as the one by parts
+    assert picked <= 1.5 * microseconds(lambda: net._forward_by_parts(x, n, h, w))
