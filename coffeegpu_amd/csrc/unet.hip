@@ -35,6 +35,7 @@ namespace {
 
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // at any float's address
 typedef uint16_t bf16;
 typedef short s8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
@@ -465,7 +466,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CP > 6
   auto load_bias = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < NB; b++)
-      bias[b] = a.bias ? *(const f4*)(a.bias + co0 + 16 * b + 4 * lk) : f4{0.f, 0.f, 0.f, 0.f};
+      bias[b] = a.bias ? (f4)*(const f4u*)(a.bias + co0 + 16 * b + 4 * lk) : f4{0.f, 0.f, 0.f, 0.f};
   };
   if constexpr (NB < 4) load_bias();  // where the registers are free, not after the MFMAs
   store_chunk();
@@ -1464,7 +1465,7 @@ bool conv_tiled(const ConvArgs& a) {
   return (conv_by_chunks(a) || a.Cin == 16 || a.Cin == 32 || a.Cin == 64 || a.Cin == 128 ||
           a.Cin == 256) &&
          (long)a.N * a.H * a.W < 2147483647L / 4 && aligned16(a.in) && aligned16(a.w) &&
-         aligned16(a.out) && aligned16(a.out32) && aligned16(a.bias);
+         aligned16(a.out) && aligned16(a.out32);
 }
 
 // Outputs of 2 x 2 pixels: a wavefront has to hold both rows (tiles of 8 rows).

@@ -98,3 +98,22 @@ def test_network_on_small_images_takes_the_faster_passes(levels, base, n, h, w, 
     assert net._pays(n, h, w) == pays
     # 1.5: the fused pass of 512 x 8 x 8 takes 1.8 times as long as the one by parts
     assert picked <= 1.5 * microseconds(lambda: net._forward_by_parts(x, n, h, w))
+
+
+# both orders of products: 32-channel chunks, and taps
+@pytest.mark.parametrize("ci,co,w", [(64, 64, 128), (128, 128, 128), (32, 32, 128), (64, 64, 40), (16, 16, 24)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_bias_at_any_float(ci, co, w, off):
+    n, h = 4, 37
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = rand(g, n * h * w * ci).bfloat16()
+    wt = (rand(g, 9 * co * ci) * (9 * ci) ** -0.5).bfloat16()
+    b = rand(g, co + 4)
+    L, s = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    outs = []
+    for bias in (b[off:off + co].clone(), b[off:off + co]):
+        y = torch.zeros(n * h * w * co, device=DEV, dtype=torch.bfloat16)
+        z = torch.zeros(n * h * w * co, device=DEV)
+        _lib.check(L.coffee_unet_conv3x3(ptr(x), ptr(wt), ptr(bias), ptr(y), ptr(z), n, h, w, ci, co, 0, 1, s))
+        outs.append((y, z))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
