@@ -308,7 +308,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvArgs& a, const f4 (&acc)
         for (int e = 0; e < 4; e++) d[e] = (short)f2bf(0.25f * bf2f((bf16)o[m][e]));
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-          const long w = ((long)(img * 2 * a.H + 2 * y + q / 2) * (2 * a.W) + 2 * x + q % 2) * a.Cout + c;
+          const long w = ((2L * (img * a.H + y) + q / 2) * (2L * a.W) + 2 * x + q % 2) * a.Cout + c;
           s4 r = d;
           if (a.skip) {
             const s4 sk = *(const s4*)(a.skip + w);
@@ -367,8 +367,10 @@ __device__ __forceinline__ int csw(int k) {
 // the taps within a chunk, for images of whole 16-pixel rows and whole 64-channel
 // blocks (CP = 32, any Cin % 32 == 0); the taps, and the 32-channel chunks within
 // a tap, otherwise, as conv3x3_k32 (CP = Cin = 32, 64, 128 or 256 here); Cin = 16
-// takes the taps with v_mfma_f32_16x16x16_bf16, as conv3x3_mfma.  So every shape has one
-// result, whatever tile or kernel computes it.
+// takes the taps with v_mfma_f32_16x16x16_bf16, as conv3x3_mfma.  So every shape of
+// less than 2^31 pixels has one result, whatever tile or kernel computes it, as long
+// as in, w, out and out32 are 16-byte aligned (conv_tiled): others go to the kernels
+// that sum by taps, 32 channels at a time or, with in or w off, 16.
 //
 // With few output channels the LDS read rate counts: one 16-byte-per-lane read
 // takes 8 cycles of the CU's LDS, in which its SIMDs finish two MFMAs.  Where the
@@ -1459,12 +1461,12 @@ bool conv_by_chunks(const ConvArgs& a) {
   return a.Cin % 32 == 0 && a.Cout % 64 == 0 && a.W % 16 == 0;
 }
 
-// Whether conv3x3_tile takes the convolution: 16-byte aligned operands, pixel
-// indices in 32 bits, and a channel count it has the shape's order for.
+// Whether conv3x3_tile takes the convolution: 16-byte aligned arrays, pixel
+// indices of its input in 32 bits, and a channel count it has the shape's order for.
 bool conv_tiled(const ConvArgs& a) {
   return (conv_by_chunks(a) || a.Cin == 16 || a.Cin == 32 || a.Cin == 64 || a.Cin == 128 ||
           a.Cin == 256) &&
-         (long)a.N * a.H * a.W < 2147483647L / 4 && aligned16(a.in) && aligned16(a.w) &&
+         (long)a.N * a.H * a.W <= 2147483647L && aligned16(a.in) && aligned16(a.w) &&
          aligned16(a.out) && aligned16(a.out32);
 }
 

@@ -117,3 +117,29 @@ def test_bias_at_any_float(ci, co, w, off):
         _lib.check(L.coffee_unet_conv3x3(ptr(x), ptr(wt), ptr(bias), ptr(y), ptr(z), n, h, w, ci, co, 0, 1, s))
         outs.append((y, z))
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+def test_conv_of_half_a_billion_pixels_keeps_its_order():
+    """2^29 pixels and more of a shape summed by 32-channel chunks: the first and last
+    images as a call on these alone computes them."""
+    n, h, w, ci, co = 65537, 64, 128, 64, 64
+    need = n * h * w * (ci + co) * 2
+    if torch.cuda.mem_get_info()[0] < need + (8 << 30):
+        pytest.skip("needs 137 GB of GPU memory")
+    g = torch.Generator(device=DEV).manual_seed(11)
+    some = rand(g, 16, h * w * ci).bfloat16()
+    x = torch.empty(n, h * w * ci, device=DEV, dtype=torch.bfloat16)
+    for k in range(0, n, 16):
+        x[k:k + 16] = some[: min(16, n - k)]
+    wt = (rand(g, 9 * co * ci) * (9 * ci) ** -0.5).bfloat16()
+    b = rand(g, co)
+    y = torch.empty(n, h * w * co, device=DEV, dtype=torch.bfloat16)
+    z = torch.empty(16, h * w * co, device=DEV, dtype=torch.bfloat16)
+    L, s = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for a, out, m in ((x, y, n), (some, z, 16)):
+        _lib.check(L.coffee_unet_conv3x3(ptr(a), ptr(wt), ptr(b), ptr(out), None, m, h, w, ci, co, 0, 1, s))
+    assert torch.equal(y[:16], z) and torch.equal(y[-1], z[(n - 1) % 16])
+    mid = n // 32 * 16
+    assert torch.equal(y[mid:mid + 16], z)
+    del x, y
+    torch.cuda.empty_cache()
