@@ -143,3 +143,54 @@ def test_conv_of_half_a_billion_pixels_keeps_its_order():
     assert torch.equal(y[mid:mid + 16], z)
     del x, y
     torch.cuda.empty_cache()
+
+
+# channels and pixels for which the one-layer call takes the kernel with a tap per
+# workgroup (whole and partial blocks of 64 channels, ranges of one and many steps, a
+# remainder of pixels), and two for which it does not; the many-layer call never does
+@pytest.mark.parametrize("shape,ci,co,nsplit", [
+    ((16, 91, 79), 64, 64, 224), ((10, 99, 44), 256, 64, 85), ((1, 256, 255), 96, 48, 127), ((3, 33, 33), 96, 48, 1),
+    ((8, 67, 93), 96, 64, 97), ((65, 9, 9), 128, 128, 10), ((1, 256, 255), 16, 16, 127), ((2, 24, 148), 256, 256, 13)])
+def test_one_layer_weight_gradient_equals_the_many_layer_call(shape, ci, co, nsplit):
+    from coffeegpu_amd.surrogate import _WGRAD
+
+    n, h, w = shape
+    g = torch.Generator(device=DEV).manual_seed(13)
+    x = rand(g, n * h * w * ci).bfloat16()
+    dz = rand(g, n * h * w * co).bfloat16()
+    L, s = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    part = torch.empty(nsplit * 9 * ci * co, device=DEV)
+    gw, gb, mw, mb = (torch.full((m,), float("nan"), device=DEV) for m in (9 * ci * co, co) * 2)
+    _lib.check(L.coffee_unet_conv3x3_wgrad(ptr(x), ptr(dz), ptr(part), nsplit, ptr(gw), ptr(gb), n, h, w, ci, co, s))
+    layer = _WGRAD.pack(x.data_ptr(), 0, dz.data_ptr(), mw.data_ptr(), mb.data_ptr(), n, h, w, ci, ci, co, 0, nsplit)
+    need = ctypes.c_long()
+    _lib.check(L.coffee_unet_wgrad_many(layer, 1, None, 0, ctypes.byref(need), s))
+    work = torch.empty(need.value, device=DEV)
+    _lib.check(L.coffee_unet_wgrad_many(layer, 1, ptr(work), need.value, None, s))
+    assert torch.equal(gw, mw) and torch.equal(gb, mb)
+
+
+def test_weight_gradient_of_two_billion_pixels_keeps_its_order():
+    """Past 2^31 pixels, where only some images within one range are not zero: the same
+    sums, bit for bit, as over these images alone."""
+    n, h, w, c, at = 262145, 64, 128, 16, 100000
+    if torch.cuda.mem_get_info()[0] < n * h * w * c * 4 + (8 << 30):
+        pytest.skip("needs 138 GB of GPU memory")
+    per = -(-n * h * w // 256)
+    first = at * h * w
+    assert per % 32 == 0 and (first % per) % 32 == 0 and first % per + 4 * h * w <= per
+    g = torch.Generator(device=DEV).manual_seed(15)
+    x = torch.zeros(n, h * w * c, device=DEV, dtype=torch.bfloat16)
+    dz = torch.zeros(n, h * w * c, device=DEV, dtype=torch.bfloat16)
+    sx, sz = rand(g, 4, h * w * c).bfloat16(), rand(g, 4, h * w * c).bfloat16()
+    x[at:at + 4], dz[at:at + 4] = sx, sz
+    part = torch.empty(256 * 9 * c * c, device=DEV)
+    L, s = _lib.load(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    out = []
+    for a, b, m, nsplit in ((x, dz, n, 256), (sx, sz, 4, 1)):
+        gw = torch.empty(9 * c * c, device=DEV)
+        _lib.check(L.coffee_unet_conv3x3_wgrad(ptr(a), ptr(b), ptr(part), nsplit, ptr(gw), None, m, h, w, c, c, s))
+        out.append(gw)
+    assert torch.equal(*out)
+    del x, dz
+    torch.cuda.empty_cache()
