@@ -209,17 +209,22 @@ void tile_shape(int variant, int& tx, int& ty) {
 // - thread-per-cell kernels where a step is launches and latency: their one
 //   round of loads ends sooner than the planes a tile marches.  The line is
 //   where the two cross (us per step): FP32 64^3 68 against 69, 80^3 139
-//   against 117; FP64 48^3 91 against 94, 64^3 123 against 100; with a star,
-//   whose cells slow few workgroups, FP32 72 x 66 x 70 122 against 136, 77 x 89 x
-//   94 200 against 179, FP64 77 x 89 x 94 391 against 421, 72 x 130 x 90 523
-//   against 506.
+//   against 117; with a star, whose cells slow few workgroups, FP32 72 x 66 x 70
+//   122 against 136, 77 x 89 x 94 200 against 179, FP64 77 x 89 x 94 391 against 421,
+//   72 x 130 x 90 523 against 506.  FP64 without a star counts the cells of the 64 x
+//   4 tiles, filled or not (48^3 91 against 94, 64^3 123 against 100; 8 x 8 x 2000
+//   338 against 216, 4 x 158 x 158 513 against 384): there the launches last as long
+//   as their idle lanes, in the other three the line by cells fits boxes from 4 to 300
+//   cells wide better.
 // - then, where the balance of many small workgroups counts for more than the
 //   planes that start a chunk, tiles of 64 x 4 (FP64 star: 64 x 8) and chunks of
 //   a few planes: FP32 up to 2 M cells (96 x 111 x 105 180 -> 171 us against the
 //   cost model's choice, 72 x 130 x 90 183 -> 157; 128^3 247 against 266), with a
 //   star up to 10 M (96 x 111 x 105 362 -> 245, 130 x 180 x 140 839 -> 733, 192^3
 //   1475 -> 1387; 256^3 3067 against 3291); FP64 with a star always (128^3 964
-//   -> 938, 192^3 2974 -> 2714, 256^3 6451 -> 6316).
+//   -> 938, 192^3 2974 -> 2714, 256^3 6451 -> 6316).  Slabs whose plane alone has 500
+//   of these tiles march it whole (FP32 254 x 844 x 7 302 -> 260, 212 x 708 x 10 301
+//   -> 233, 73 x 1468 x 14 299 -> 254).
 // - above, the tile and z chunk of the lowest chunk_cost.  A plane of a 128 x
 //   8 tile takes 1.6 times as long as one of a 64 x 8 tile (21.2 against 12.1
 //   us at 128^3, less 10 % since it fetches half as many x halos per cell,
@@ -236,11 +241,13 @@ template <typename T>
 FlatSchedule auto_schedule(const FlatK<T>& k, bool star) {
   constexpr bool f32 = sizeof(T) == 4;
   const double n = (double)k.n[0] * k.n[1] * k.n[2];
-  const double small = f32 ? (star ? 450e3 : 300e3) : (star ? 800e3 : 130e3);
-  if (n <= small) return {false, 64, 8, 1};
-  if (f32 && n <= (star ? 10e6 : 2e6)) return {true, 64, 4, n <= 2.5e6 ? 3 : 4};
-  if (!f32 && star) return {true, 64, 8, n <= 2e6 ? 4 : 6};
   auto tiles = [&](int tx, int ty) { return ((k.n[0] + tx - 1) / tx) * ((k.n[1] + ty - 1) / ty); };
+  const int t64 = tiles(64, 4);
+  const bool small = f32 || star ? n <= (f32 ? (star ? 450e3 : 300e3) : 800e3)
+                                 : 256.0 * t64 * k.n[2] <= 150e3;
+  if (small) return {false, 64, 8, 1};
+  if (f32 && n <= (star ? 10e6 : 2e6)) return {true, 64, 4, !star && t64 >= 500 ? k.n[2] : n <= 2.5e6 ? 3 : 4};
+  if (!f32 && star) return {true, 64, 8, n <= 2e6 ? 4 : 6};
   double c64 = 0, c128 = 0;
   FlatSchedule s{true, 64, 8, auto_zchunk(tiles(64, 8), k.n[2], kFlatStart, star, &c64)};
   if (!f32) return s;
