@@ -229,12 +229,11 @@ int gr_step_impl(coffee_ctx* c, const coffee_fields* f, hipStream_t s) {
   tm.ntx = (k.n[0] + 63) / 64;
   tm.nty = (k.n[1] + TY - 1) / TY;
   // whole rounds of one workgroup per CU (the registers, and in FP64 the LDS,
-  // allow no second one): 384^3 FP32 12.0 -> 10.0 ms, 192^3 1617 -> 1358 us,
-  // FP64 128^3 986 -> 841 us against the earlier two workgroups per CU for
-  // whole columns.  The start-up of a chunk measured about 8 planes in FP32, 4
-  // in FP64 (its planes take twice as long).
-  tm.zc = c->zchunk > 0 ? c->zchunk
-                        : auto_zchunk(tm.ntx * tm.nty, k.n[2], sizeof(T) == 4 ? 8.0 : 4.0, false);
+  // allow no second one): 384^3 FP32 12.0 -> 10.1 ms, 192^3 1617 -> 1343 us, FP64
+  // 128^3 986 -> 841 us against the earlier two workgroups per CU for whole columns.
+  // The start-up of a chunk counts as 4 planes (with 8 in FP32 73 x 1468 x 14 took 553
+  // us instead of 469, 176^3 1201 instead of 1125; no box was faster).
+  tm.zc = c->zchunk > 0 ? c->zchunk : auto_zchunk(tm.ntx * tm.nty, k.n[2], 4.0, false);
   if (tm.zc > k.n[2]) tm.zc = k.n[2];
   tm.nzc = (k.n[2] + tm.zc - 1) / tm.zc;
   const int tblocks = tm.ntx * tm.nty * tm.nzc;

@@ -35,7 +35,8 @@ def microseconds(step):
 # (variant, zchunk) set by hand; the picked schedule took 1.16 to 1.58 times as long
 @pytest.mark.parametrize("gr,n,dtype,by_hand", [
     (False, (8, 8, 2000), np.float64, (3, 0)), (False, (4, 158, 158), np.float64, (3, 0)),
-    (False, (254, 844, 7), np.float32, (2, 7)), (False, (212, 708, 10), np.float32, (2, 10))])
+    (False, (254, 844, 7), np.float32, (2, 7)), (False, (212, 708, 10), np.float32, (2, 10)),
+    (True, (73, 1468, 14), np.float32, (0, 7)), (True, (194, 644, 12), np.float32, (0, 6))])
 def test_picked_schedule_is_no_slower(gr, n, dtype, by_hand):
     d = 1.0 / max(n)
     sp = SimParams(dt=0.1 * d, N=list(n), guard=[3, 3, 3], lower=[3.0, 3.0, 3.0] if gr else [0.0] * 3,
