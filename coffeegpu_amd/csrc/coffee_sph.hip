@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -195,7 +196,14 @@ struct SphState : SphStateBase {
     drop_graph();
     const Tile t = kTiles[tile];
     std::vector<SphItem> items;
-    for (int r = 0; r < (int)h_runs.size(); r++)
+    // the runs that go on longest first: what is still active is then always the head
+    // of the list, which the workgroups share out evenly (where every eighth of 100 runs
+    // of 16 x 512 went on, in their own order it was every eighth tile of few workgroups)
+    std::vector<int> order(h_runs.size());
+    for (int r = 0; r < (int)order.size(); r++) order[r] = r;
+    auto last = [&](int r) { return h_clocks[r].nsteps > 0 ? h_clocks[r].nsteps : INT_MAX; };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return last(a) > last(b); });
+    for (const int r : order)
       for (int j0 = 0; j0 < h_runs[r].n1; j0 += t.ty)
         for (int i0 = 0; i0 < h_runs[r].n0; i0 += t.tx) items.push_back({r, i0, j0});
     by_xcd(items);
