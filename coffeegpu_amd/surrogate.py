@@ -302,9 +302,9 @@ class UNet:
         tape, n, _ = self._tape
         npix = lambda k: n * tape[k][6] * tape[k][7]  # noqa: E731
         if dout.data_ptr() % 16:
-            dout = self._buf(("dout16",), dout.numel(), torch.int16).copy_(dout.view(torch.int16))
+            flat = dout.view(torch.int16).reshape(-1)
+            dout = self._buf(("dout16",), flat.numel(), torch.int16)[: flat.numel()].copy_(flat)
         dzs = {len(tape) - 1: dout}
-        pos = {t[0]: k for k, t in enumerate(tape)}
         dskip = {}
 
         def dz_of(k):
