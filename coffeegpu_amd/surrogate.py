@@ -302,8 +302,11 @@ class UNet:
         tape, n, _ = self._tape
         npix = lambda k: n * tape[k][6] * tape[k][7]  # noqa: E731
         if dout.data_ptr() % 16:
-            flat = dout.view(torch.int16).reshape(-1)
-            dout = self._buf(("dout16",), flat.numel(), torch.int16)[: flat.numel()].copy_(flat)
+            # a copy on the network's stream, which need not be torch's current one
+            c, moved = pad16(self.cout), dout
+            dout = self._buf(("dout16",), npix(0) * c, torch.int16)
+            _lib.check(self._lib.coffee_unet_combine(_p(dout), c, 0, _p(moved), c, 0, None, 0, 0, None,
+                                                     0, 0, c, npix(0), s))
         dzs = {len(tape) - 1: dout}
         dskip = {}
 

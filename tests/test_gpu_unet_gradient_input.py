@@ -43,3 +43,36 @@ def test_misaligned_gradients_of_several_sizes(shaped):
         got = grads(net, x, m if shaped else m.view(torch.int16).view(-1), n, h, w)
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+def test_misaligned_gradient_is_read_on_the_networks_stream():
+    side = torch.cuda.Stream()
+    net = UNet(2, 16, 7, 6, seed=3, stream=side)
+    n, h, w = 2, 16, 32
+    x, d = batch(net, n, h, w, seed=5)
+    flat = d.view(torch.int16).view(-1)
+    torch.cuda.synchronize()
+    want = grads_on(side, net, x, flat, n, h, w)
+    late = off_by_two(torch.zeros_like(flat))
+    a = torch.randn((4096, 4096), device=DEV)
+    net.forward(x, n, h, w)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(8):  # some milliseconds before the gradient is there
+            a = a @ a * 1e-3
+        late.copy_(flat)
+    net.backward(late)
+    side.synchronize()
+    for got, ref in zip([net.dx[: n * h * w * 16]] + parameters(net), want):
+        assert torch.equal(got, ref)
+
+
+def parameters(net):
+    return [P[k] for P in net.params.values() for k in ("gw", "gb")]
+
+
+def grads_on(stream, net, x, d, n, h, w):
+    net.forward(x, n, h, w)
+    dx = net.backward(d)
+    stream.synchronize()
+    return [dx[: n * h * w * 16].clone()] + [t.clone() for t in parameters(net)]
