@@ -295,8 +295,8 @@ class UNet:
 
     def _backward_fused(self, dout):
         """One launch per convolution for the activation gradients, which leave
-        each of them as the dz of the convolution before, then two for all
-        parameter gradients."""
+        each of them as the dz of the convolution before, then all parameter
+        gradients."""
         torch = _torch()
         s = self._s()
         tape, n, _ = self._tape
@@ -336,16 +336,34 @@ class UNet:
                     kw["csplit"] = c1
                     kw["out2"] = dskip[l] = self._buf(("dskip", l), npix(k) * (P["cip"] - c1), torch.int16)
             self._conv_fused(s, dzs[k], None, None, 0, P, n, hh, ww, out, form=form, mask=mask, **kw)
-        layers = b"".join(
+        self._parameter_gradients([
             _WGRAD.pack(_a(x), _a(x2), _a(dzs[k]), _a(self.params[name]["gw"]),
                         _a(self.params[name]["gb"]), n, hh, ww, self.params[name]["cip"], c1,
                         self.params[name]["cop"], up, self._nsplit(n * hh * ww))
-            for k, (name, x, x2, c1, up, _, hh, ww) in enumerate(tape))
-        need = ctypes.c_long()
-        _lib.check(self._lib.coffee_unet_wgrad_many(layers, len(tape), None, 0, ctypes.byref(need), s))
-        part = self._buf(("part",), need.value, torch.float32)
-        _lib.check(self._lib.coffee_unet_wgrad_many(layers, len(tape), _p(part), part.numel(), None, s))
+            for k, (name, x, x2, c1, up, _, hh, ww) in enumerate(tape)])
         return self.dx
+
+    def _parameter_gradients(self, layers):
+        """All layers together: their partial sums take the most memory of a training
+        step's workspaces (base 32, 4 levels: 101 MB on 8 x 64 x 128, 613 MB on 16 x 128 x 256).
+        Where that cannot be had, one layer after the other (9 and 75 MB), in 2 launches
+        each instead of 3 to 4 for all; the same bits."""
+        torch, s = _torch(), self._s()
+        many = self._lib.coffee_unet_wgrad_many
+
+        def need(l):
+            floats = ctypes.c_long()
+            _lib.check(many(b"".join(l), len(l), None, 0, ctypes.byref(floats), s))
+            return floats.value
+
+        groups = [layers]
+        try:
+            part = self._buf(("part",), need(layers), torch.float32)
+        except torch.OutOfMemoryError:
+            groups = [[l] for l in layers]
+            part = self._buf(("part",), max(map(need, groups)), torch.float32)
+        for g in groups:
+            _lib.check(many(b"".join(g), len(g), _p(part), part.numel(), None, s))
 
     def _forward_by_parts(self, x, n, h, w):
         torch = _torch()

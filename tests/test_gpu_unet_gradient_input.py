@@ -76,3 +76,28 @@ def grads_on(stream, net, x, d, n, h, w):
     dx = net.backward(d)
     stream.synchronize()
     return [dx[: n * h * w * 16].clone()] + [t.clone() for t in parameters(net)]
+
+
+def test_parameter_gradients_without_memory_for_all_layers(monkeypatch):
+    net = UNet(3, 32, 7, 6, seed=3)
+    n, h, w = 2, 16, 48
+    x, d = batch(net, n, h, w, seed=5)
+    flat = d.view(torch.int16).view(-1)
+    want = grads(net, x, flat, n, h, w)
+    whole = net._bufs.pop(("part",)).numel()
+    buf, asked = net._buf, []
+
+    def short(key, numel, dtype):
+        if key == ("part",):
+            asked.append(numel)
+            if numel > whole // 2:
+                raise torch.OutOfMemoryError("no memory for the partial sums of all layers")
+        return buf(key, numel, dtype)
+
+    monkeypatch.setattr(net, "_buf", short)
+    for t in parameters(net):
+        t.fill_(float("nan"))
+    got = grads(net, x, flat, n, h, w)
+    assert asked[0] == whole and 0 < asked[1] <= whole // 2
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
