@@ -306,9 +306,9 @@ struct SphState : SphStateBase {
   int upload(coffee_ctx* c) {
     HIP_TRY(c, hipMemcpy(d_runs, h_runs.data(), sizeof(SphRun<T>) * h_runs.size(),
                          hipMemcpyHostToDevice));
-    for (int q = 0; q < kClockTables; q++)
-      HIP_TRY(c, hipMemcpy(clocks(q), h_clocks.data(), sizeof(SphClock) * h_clocks.size(),
-                           hipMemcpyHostToDevice));
+    std::vector<SphClock> all;  // in every table
+    for (int q = 0; q < kClockTables; q++) all.insert(all.end(), h_clocks.begin(), h_clocks.end());
+    HIP_TRY(c, hipMemcpy(d_clocks, all.data(), sizeof(SphClock) * all.size(), hipMemcpyHostToDevice));
     return COFFEE_OK;
   }
 };
@@ -407,22 +407,18 @@ int make_run(coffee_ctx* c, SphState<T>* S, const coffee_grid& g, const coffee_p
   // axis rows within half a cell of theta = 0 and pi (.cu:690-748)
   R.axis0 = std::fabs(R.y0) < R.dy / T(2);
   R.axis1 = std::fabs(R.y0 + R.dy * T(R.n1) - T(M_PI)) < R.dy / T(2);
-  T *dr = nullptr, *ds = nullptr, *dc = nullptr, *dr3 = nullptr, *dir2 = nullptr;
+  T *dr = nullptr, *ds = nullptr, *dr3 = nullptr, *dir2 = nullptr;
   if ((rc = alloc_owned(c, S, r.size(), &dr))) return rc;
-  if ((rc = alloc_owned(c, S, sth.size(), &ds))) return rc;
-  if ((rc = alloc_owned(c, S, sth.size(), &dc))) return rc;
+  if ((rc = alloc_owned(c, S, 2 * sth.size(), &ds))) return rc;  // and cos(theta): sph_cos_tables
   if ((rc = alloc_owned(c, S, r3.size(), &dr3))) return rc;
   if ((rc = alloc_owned(c, S, ir2.size(), &dir2))) return rc;
   HIP_TRY(c, hipMemcpy(dr, r.data(), r.size() * sizeof(T), hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(ds, sth.data(), sth.size() * sizeof(T), hipMemcpyHostToDevice));
-  sph_cos_table<T><<<(g.dims[1] + 255) / 256, 256>>>(dc, R.y0, R.dy, R.g1, g.dims[1]);
-  HIP_TRY(c, hipGetLastError());
-  HIP_TRY(c, hipStreamSynchronize(nullptr));
   HIP_TRY(c, hipMemcpy(dr3, r3.data(), r3.size() * sizeof(T), hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(dir2, ir2.data(), ir2.size() * sizeof(T), hipMemcpyHostToDevice));
   R.r = dr;
   R.sth = ds;
-  R.cth = dc;
+  R.cth = ds + sth.size();
   R.r3 = dr3;
   R.ir2 = dir2;
   R.inv_tau = (T)(1.0 / p.tau);
@@ -476,6 +472,9 @@ int batch_create(coffee_ctx* c, int nruns, const coffee_grid* grids, const coffe
   HIP_TRY(c, hipMalloc(&S->d_clocks, sizeof(SphClock) * kClockTables * nruns));
   int rc = S->upload(c);
   if (rc) return rc;
+  sph_cos_tables<T><<<dim3(4, nruns), 256>>>(S->d_runs);
+  HIP_TRY(c, hipGetLastError());
+  HIP_TRY(c, hipStreamSynchronize(nullptr));
   // Until a tile is set or tuned: taps through the caches while the fields fit the
   // L2s, the tile and its halo in LDS above (us per step of tiles 0, 5 and 9: FP32
   // 524 k cells 94, 93, 94; 1.05 M 158, 151, 150; 2.1 M 358, 297, 304; 4.2 M 866,

@@ -833,11 +833,14 @@ __global__ void __launch_bounds__(TX) __attribute__((amdgpu_waves_per_eu(TX >= 5
   sph_advance(runs, clocks, next, nruns);
 }
 
-// cos(theta_j) as the cells would evaluate it (the host's may round differently).
+// cos(theta_j) of every run as the cells would evaluate it (the host's may round
+// differently): one launch when the runs are set up.
 template <typename T>
-__global__ void __launch_bounds__(256) sph_cos_table(T* __restrict__ cth, T y0, T dy, int g1, int n) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n) cth[j] = cos(y0 + dy * T(j - g1));
+__global__ void __launch_bounds__(256) sph_cos_tables(const SphRun<T>* __restrict__ runs) {
+  const SphRun<T>& R = runs[blockIdx.y];
+  T* const cth = const_cast<T*>(R.cth);
+  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < R.dims1; j += gridDim.x * blockDim.x)
+    cth[j] = cos(R.y0 + R.dy * T(j - R.g1));
 }
 
 // theta-axis boundary (kernel_boundary_axis_sph, .cu:690-748) on buffer `buf`
