@@ -94,8 +94,9 @@ class UNet:
         self._bufs: Dict[tuple, object] = {}
         self._fusable: Dict[tuple, bool] = {}  # by (n, h, w), as _pay
         self._pay: Dict[tuple, Tuple[bool, bool]] = {}
-        # partial sums of the loss: written by the device, summed here
-        self._work = _torch().empty(1024, dtype=_torch().float64, pin_memory=True)
+        # free pinned arrays for the partial sums of the loss (written by the device,
+        # summed by the host): one for each thread that is in loss_and_grad
+        self._works: List[object] = []
 
     # ---- parameters ------------------------------------------------------
     def _alloc_param(self, w: np.ndarray, b: np.ndarray, ci: int, co: int, relu: bool) -> dict:
@@ -493,9 +494,16 @@ class UNet:
         cop = pad16(self.cout)
         dout = self._buf(("dout",), n * h * w * cop, torch.int16)
         loss = ctypes.c_double()
-        _lib.check(self._lib.coffee_unet_mse_pinned(_p(out32), cop, _p(target), self.cout,
-                                                    n * h * w, _p(dout), _p(self._work),
-                                                    ctypes.byref(loss), self._s()))
+        try:
+            work = self._works.pop()
+        except IndexError:
+            work = torch.empty(1024, dtype=torch.float64, pin_memory=True)
+        try:
+            _lib.check(self._lib.coffee_unet_mse_pinned(_p(out32), cop, _p(target), self.cout,
+                                                        n * h * w, _p(dout), _p(work),
+                                                        ctypes.byref(loss), self._s()))
+        finally:
+            self._works.append(work)
         return loss.value, dout
 
     def adam_step(self, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999,
