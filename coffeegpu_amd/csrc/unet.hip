@@ -2082,7 +2082,7 @@ int coffee_unet_adam_many(const coffee_unet_tensor* l, int count, float lr, floa
                           float eps, int t, void* stream) {
   if (!l || count < 1 || t < 1) return fail(nullptr, COFFEE_ERR_INVALID, "adam_many: bad arguments");
   for (int k = 0; k < count; k++)
-    if (!l[k].p || !l[k].g || !l[k].m || !l[k].v || l[k].n < 1 || l[k].n > 1 << 30 ||
+    if (!l[k].p || !l[k].g || !l[k].m || !l[k].v || l[k].n < 1 ||
         (l[k].wb && (!l[k].wbt || l[k].cout < 1 || l[k].cin < 1 || 9L * l[k].cout * l[k].cin != l[k].n)))
       return fail(nullptr, COFFEE_ERR_INVALID, "adam_many: bad arguments of tensor " + std::to_string(k));
   AdamMany a;
@@ -2092,20 +2092,28 @@ int coffee_unet_adam_many(const coffee_unet_tensor* l, int count, float lr, floa
   a.eps = eps;
   a.c1 = 1.f - powf(beta1, (float)t);
   a.c2 = 1.f - powf(beta2, (float)t);
-  for (int k0 = 0; k0 < count; k0 += kAdamTensors) {
-    a.n = std::min(count - k0, kAdamTensors);
-    a.first[0] = 0;
-    for (int k = 0; k < a.n; k++) {
-      const coffee_unet_tensor& q = l[k0 + k];
-      a.l[k] = {q.p, q.g, q.m, q.v, (bf16*)q.wb, (bf16*)q.wbt, (int)q.n, q.cout, q.cin};
-      a.first[k + 1] = a.first[k] + (q.wb ? 9 * ((q.cout + 31) / 32) * ((q.cin + 31) / 32)
-                                          : (int)((q.n + 1023) / 1024));
-    }
+  auto launch = [&]() -> int {
+    if (!a.n) return COFFEE_OK;
     adam_many_kernel<<<a.first[a.n], 256, 0, (hipStream_t)stream>>>(a);
-    const int rc = launch_check("adam_many");
+    a.n = 0;
+    return launch_check("adam_many");
+  };
+  a.n = a.first[0] = 0;
+  for (int k = 0; k < count; k++) {
+    const coffee_unet_tensor& q = l[k];
+    int rc = COFFEE_OK;
+    if (q.n > 1L << 30) {  // beyond the 32-bit indices of the kernel for many
+      rc = coffee_unet_adam(q.p, q.g, q.m, q.v, q.n, lr, beta1, beta2, eps, t, q.wb, q.wbt, q.cout, q.cin,
+                            stream);
+    } else {
+      a.l[a.n] = {q.p, q.g, q.m, q.v, (bf16*)q.wb, (bf16*)q.wbt, (int)q.n, q.cout, q.cin};
+      a.first[a.n + 1] = a.first[a.n] + (q.wb ? 9 * ((q.cout + 31) / 32) * ((q.cin + 31) / 32)
+                                              : (int)((q.n + 1023) / 1024));
+      if (++a.n == kAdamTensors) rc = launch();
+    }
     if (rc) return rc;
   }
-  return COFFEE_OK;
+  return launch();
 }
 
 int coffee_unet_weights_bf16(const float* w32, void* wb, void* wbt, int cout, int cin, void* stream) {
