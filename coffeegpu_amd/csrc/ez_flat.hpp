@@ -277,7 +277,9 @@ __device__ __forceinline__ void star_boundary(const FlatK<T>& k, const StarPhase
         w0 = wpert_d(t, th, k.tp_start, k.tp_end, k.dw0, k.nT, k.rpert1, k.rpert2);
         w1 = wpert_d(t, th, k.tp_start1, k.tp_end1, k.dw1, k.nT1, k.rpert11, k.rpert21);
       } else {
-        T ph = atan2(y, x);
+        // in FP64: the compiler evaluates the FP32 function's division in one of two
+        // ways, by kernel, and the schedules then differ in the last bit
+        T ph = (T)atan2((double)y, (double)x);
         w0 = wpert3d_d(t, th, ph, k.tp_start, k.tp_end, k.dw0, k.nT, k.rpert1, k.rpert2, k.ph1,
                        k.ph2, k.dph);
         w1 = wpert3d_d(t, th, ph, k.tp_start1, k.tp_end1, k.dw1, k.nT1, k.rpert11, k.rpert21,
