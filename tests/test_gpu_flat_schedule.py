@@ -48,3 +48,12 @@ def test_picked_schedule_is_bitwise_the_same(n, problem, dtype):
     assert np.isfinite(outs[0]).all()
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
+
+
+# FP32 boxes that get 128 x 8 tiles (by the cost estimate 86 planes against 108 of 64 x
+# 8, 50 against 62), and with a star on both sides of the line at 10 M cells, above
+# which it gets them too (84 against 107)
+@pytest.mark.parametrize("n,problem", [((254, 259, 131), 0), ((382, 350, 21), 0), ((250, 245, 163), 1),
+                                       ((253, 245, 167), 1)])
+def test_picked_schedule_of_large_boxes(n, problem):
+    test_picked_schedule_is_bitwise_the_same(n, problem, np.float32)
