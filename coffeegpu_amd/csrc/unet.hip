@@ -1,9 +1,10 @@
 // U-Net building blocks for gfx950 (include/coffee_unet.h): BF16 activations
 // and weights, FP32 accumulation on the matrix cores.
 //
-// The 3x3 convolution is an implicit GEMM.  With Cin % 32 == 0 or Cin == 16 it
-// runs on v_mfma_f32_16x16x32_bf16 with the input tile and the weights staged
-// in LDS (conv3x3_tile below); otherwise, or with operands that are not 16-byte
+// The 3x3 convolution is an implicit GEMM.  With Cin % 32 == 0 it runs on
+// v_mfma_f32_16x16x32_bf16, the input tile and the weights staged in LDS
+// (conv3x3_tile; Cin = 16 too) or, where the images fill the tiles badly, the input
+// from the caches (conv3x3_k32); otherwise, or with operands that are not 16-byte
 // aligned, on v_mfma_f32_16x16x16_bf16 from global memory: the M dimension is
 // 16 pixels per wavefront (4 wavefronts = 64 pixels per workgroup), N is 16*NB
 // output channels, K runs over the 9 taps times the input channels in steps of

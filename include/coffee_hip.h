@@ -199,23 +199,22 @@ int coffee_set_diagnostics(coffee_ctx *ctx, int enable);
 
 /* Kernel schedule of the solver (no reference counterpart: the reference
  * has one thread-per-cell launch geometry, field_solver_EZ.cu:10-12).
- * variant 0 = chosen from the grid's size (flat solver: one thread per cell
- * on small grids, else LDS-tiled z-marching kernels with the tile and z chunk
- * of the lowest estimated time; with a zchunk, the default tile, FP32 128 x 8,
- * FP64 64 x 8), 1 = one thread per cell, 2/3/4 =
- * tiled 64 wide with 4/8/16 rows per tile (16 in FP32, 8 in FP64), 5/6 = tiled
- * 128/256 wide (FP32 128 x 8 and 256 x 4; FP64 128 x 4 for both), 7 = 128 x 4;
- * variant 0 in FP32 runs Kreiss-Oliger with 32-bit field offsets when every
- * array is below 4 GiB, variant 5 is the same tile with 64-bit addressing;
- * the GR solver runs its tiled schedule, every metric point computed on the
- * fly, for every variant but 0 on small grids without a zchunk and 1 (point
- * sweep + stage sweep) and 2 (the halo points' metric in stages 2-5 read from
- * a table filled once); in FP32 its middle stages load the x-y halo three
- * planes ahead except in variant 3 (one plane ahead); variants 1 and 2
- * allocate 12 grid-sized scratch arrays on first use, small grids with the
- * context, and GR arrays of 4 GiB or more always take the point schedule;
- * zchunk = z planes per
- * workgroup of the tiled kernels, 0 = automatic.
+ * Flat solver: variant 0 = chosen from the grid's size (one thread per cell on
+ * small grids, else LDS-tiled z-marching kernels with the tile and z chunk of the
+ * lowest estimated time; with a zchunk, the default tile, FP32 128 x 8, FP64
+ * 64 x 8), 1 = one thread per cell, 2/3/4 = tiled 64 wide with 4/8/16 rows per
+ * tile (16 in FP32, 8 in FP64), 5/6 = tiled 128/256 wide (FP32 128 x 8 and 256 x
+ * 4; FP64 128 x 4 for both), 7 = 128 x 4.  Where variant 0 takes the 128 x 8 tile
+ * and every array is below 4 GiB, Kreiss-Oliger addresses the fields by 32-bit
+ * offsets; variant 5 is that tile with 64-bit addressing.
+ * GR solver: 1 = point sweep + stage sweep, 2 = tiled, the halo points' metric of
+ * stages 2-5 read from a table filled once, 0 without a zchunk on small grids as
+ * 1, all others tiled with every metric point computed on the fly; in FP32 the
+ * middle stages then load the x-y halo three planes ahead, in variant 3 one plane
+ * ahead.  The schedules of 1 and 2 allocate 12 grid-sized scratch arrays on first
+ * use (small grids with the context); arrays of 4 GiB or more always take the
+ * point schedule.
+ * zchunk = z planes per workgroup of the tiled kernels, 0 = automatic.
  * Schedules change speed only: results are bitwise identical. */
 int coffee_set_schedule(coffee_ctx *ctx, int variant, int zchunk);
 
