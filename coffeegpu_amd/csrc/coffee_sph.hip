@@ -171,25 +171,18 @@ struct SphState : SphStateBase {
   void by_xcd(std::vector<SphItem>& items) const {
     bool together = true;
     for (const SphClock& k : h_clocks) together = together && k.nsteps == h_clocks[0].nsteps;
-    std::vector<SphItem> q[8];
-    int extra = 0;  // XCDs that have taken one tile more, over the runs so far
+    std::vector<SphItem> out(items.size());
+    size_t at[8] = {};  // items of each XCD so far
+    int extra = 0;      // XCDs that have taken one tile more, over the runs so far
     for (size_t k = 0; k < items.size();) {
       size_t e = together ? items.size() : k;
       while (e < items.size() && items[e].run == items[k].run) e++;
       const int m = (int)(e - k);
-      for (int x = 0; x < 8; x++) {
-        const int take = m / 8 + (((x - extra) & 7) < m % 8);
-        q[x].insert(q[x].end(), items.begin() + k, items.begin() + k + take);
-        k += take;
-      }
+      for (int x = 0; x < 8; x++)
+        for (int t = m / 8 + (((x - extra) & 7) < m % 8); t > 0; t--) out[8 * at[x]++ + x] = items[k++];
       extra += m % 8;
     }
-    size_t at[8] = {};
-    for (size_t k = 0; k < items.size(); k++) {
-      int x = (int)(k & 7);
-      while (at[x] == q[x].size()) x = (x + 1) & 7;
-      items[k] = q[x][at[x]++];
-    }
+    items.swap(out);
   }
 
   int build_items(coffee_ctx* c) {
