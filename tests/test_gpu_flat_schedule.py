@@ -57,3 +57,15 @@ def test_picked_schedule_is_bitwise_the_same(n, problem, dtype):
                                        ((253, 245, 167), 1)])
 def test_picked_schedule_of_large_boxes(n, problem):
     test_picked_schedule_is_bitwise_the_same(n, problem, np.float32)
+
+
+# FP64 at the line by cells of tiles (148480 and 151040 of them, 49 of 64 columns and
+# all filled), narrow boxes, FP32 at its line and slabs whose plane has 498 and 500
+# tiles of 64 x 4
+@pytest.mark.parametrize("n,problem,dtype", [
+    ((49, 38, 58), 0, np.float64), ((49, 40, 59), 0, np.float64), ((64, 40, 58), 0, np.float64),
+    ((64, 40, 59), 0, np.float64), ((8, 9, 500), 0, np.float64), ((4, 33, 200), 0, np.float64),
+    ((66, 66, 68), 0, np.float32), ((65, 996, 8), 0, np.float32), ((65, 1000, 8), 0, np.float32),
+    ((65, 1000, 8), 1, np.float32), ((254, 844, 7), 0, np.float32)])
+def test_picked_schedule_of_narrow_boxes_and_slabs(n, problem, dtype):
+    test_picked_schedule_is_bitwise_the_same(n, problem, dtype)
