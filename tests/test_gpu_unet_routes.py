@@ -26,18 +26,20 @@ def rand(g, *shape):
     return torch.randn(shape, device=DEV, generator=g)
 
 
-def microseconds(f):
-    """Of one call of f among others: the least of six runs of 20."""
-    best = 1e30
-    f()
-    for _ in range(6):
-        torch.cuda.synchronize()
-        t = time.perf_counter()
-        for _ in range(20):
+def microseconds(*calls):
+    """Of one call of each among others of its own: the least of eight runs of 20, the
+    calls in turn."""
+    best = [1e30] * len(calls)
+    for _ in range(8):
+        for k, f in enumerate(calls):
             f()
-        torch.cuda.synchronize()
-        best = min(best, time.perf_counter() - t)
-    return best / 20 * 1e6
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(20):
+                f()
+            torch.cuda.synchronize()
+            best[k] = min(best[k], (time.perf_counter() - t) / 20 * 1e6)
+    return best
 
 
 # (images, rows, columns), channels in and out: many images of a few pixels, single rows and
@@ -60,7 +62,7 @@ def test_conv_takes_the_faster_kernel(shape, ci, co):
     def call(out):
         _lib.check(L.coffee_unet_conv3x3(ptr(x), ptr(wt), ptr(b), ptr(out), None, n, h, w, ci, co, 0, 1, s))
 
-    picked, other = microseconds(lambda: call(y)), microseconds(lambda: call(z))
+    picked, other = microseconds(lambda: call(y), lambda: call(z))
     assert torch.equal(y, z)
     # 1.4: the estimate that decides is up to a third off, and short calls vary
     assert picked <= 1.4 * other, (picked, other)
@@ -94,10 +96,10 @@ def test_network_on_small_images_takes_the_faster_passes(levels, base, n, h, w, 
     got += grads(got[0])
     for a, b, c in zip(got, want, other):
         assert torch.equal(a, b) and torch.equal(a, c)
-    picked = microseconds(lambda: net.forward(x, n, h, w))
     assert net._pays(n, h, w) == pays
+    picked, parts = microseconds(lambda: net.forward(x, n, h, w), lambda: net._forward_by_parts(x, n, h, w))
     # 1.5: the fused pass of 512 x 8 x 8 takes 1.8 times as long as the one by parts
-    assert picked <= 1.5 * microseconds(lambda: net._forward_by_parts(x, n, h, w))
+    assert picked <= 1.5 * parts, (picked, parts)
 
 
 # both orders of products: 32-channel chunks, and taps
