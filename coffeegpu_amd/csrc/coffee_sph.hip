@@ -278,7 +278,12 @@ struct SphState : SphStateBase {
 
   int step(coffee_ctx* c, int k, hipStream_t s) override {
     const int q = table_of(k);
-    if (!use_graph || c->timing || c->diagnostics) return step_direct(c, q, s);
+    // a graph launched on a stream that the caller is recording would run now, and
+    // not in the replays
+    hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+    if (use_graph && hipStreamIsCapturing(s, &recording) != hipSuccess) (void)hipGetLastError();
+    if (!use_graph || c->timing || c->diagnostics || recording != hipStreamCaptureStatusNone)
+      return step_direct(c, q, s);
     if (!graph_exec[q]) {
       hipStream_t cs;
       HIP_TRY(c, hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));

@@ -66,3 +66,27 @@ def test_replays_go_on_from_the_state_before_them(dtype, tile):
     assert ref.status()[0] == [1, 0, 0] and ref.status()[2] == [22, 9, 14]
     b.close()
     ref.close()
+
+
+@pytest.mark.parametrize("warm", [0, 1, 4])
+def test_recording_a_batch_that_replays_its_own_graphs(warm):
+    b, datas = make(np.float64, 0)
+    ref, rdatas = make(np.float64, 0)
+    b.use_graph(True)
+    if warm:
+        b.step(warm)
+        ref.step(warm)
+    g = record(b, 3)
+    torch.cuda.synchronize()
+    assert b.status() == ref.status()
+    for _ in range(3):
+        g.replay()
+        ref.step(3)
+        b.step(1)
+        ref.step(1)
+        torch.cuda.synchronize()
+        assert b.status() == ref.status()
+        for d, r in zip(datas, rdatas):
+            assert np.array_equal(d.get_state(), r.get_state())
+    b.close()
+    ref.close()
