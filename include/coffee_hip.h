@@ -254,7 +254,9 @@ int coffee_sph_batch_set_tile(coffee_batch *b, int tile_index);
  * go to the lower index); ms_per_tile may be NULL. */
 int coffee_sph_batch_autotune(coffee_batch *b, int trials, void *stream, int *best_tile,
                               double *ms_per_tile);
-/* Capture one step's launch sequence into a HIP graph and replay it. */
+/* Capture one step's launch sequence into a HIP graph and replay it for the second
+ * and later steps of a call (not while `stream` is being recorded by the caller: then
+ * the launches themselves are recorded). */
 int coffee_sph_batch_use_graph(coffee_batch *b, int enable);
 /* Residual monitor of every run (the quantities of coffee_residuals for the
  * spherical solver), out[5*run .. 5*run+4].  Synchronous on `stream`. */
